@@ -7,30 +7,25 @@
 // against q' = (q . R_k) / sqrt(D); the live token is folded in at the merge;
 // the history value sum is inverse-rotated by R_v when given.
 //
-// Launches, with grids fixed by host shapes:
-//   prepare  (rows x heads)          q' in log2 units, live score, group sums
-//                                    of q', q' as 16-bit integers split into
-//                                    four nibble planes for v_dot8_u32_u4
-//                                    (with one split per (row, head) the
-//                                    decode workgroup does this itself and
-//                                    the call is one launch);
-//   decode   (rows x heads x splits) one workgroup = 4 waves streaming the
-//                                    pages of one split, two 16-token units
-//                                    per wave iteration; lane = token x
-//                                    32-channel quarter (decode_kernel), or
-//                                    token x 48-channel half for D = 96
-//                                    (decode96_dma_kernel); QK on
-//                                    integer dot8 units, PV in FP32 registers,
-//                                    online softmax per wave, LDS merge of the
-//                                    waves; the split that finishes last for
-//                                    its (row, head) does the log-sum-exp
-//                                    merge of the splits and the live token,
-//                                    the V inverse rotation and the BF16
-//                                    output.
-// The BF16 baseline keeps a separate merge launch.
+// A call is one launch of (items x heads) workgroups, the grid fixed by host
+// shapes and the items planned on the device from the request lengths
+// (rq_plan.h).  One workgroup = 4 waves: it prepares its query (q' in log2
+// units, live score, group sums of q', q' as 16-bit integers split into four
+// nibble planes for v_dot8_u32_u4) and streams the pages of one split, two
+// 16-token units per wave iteration; lane = token x 32-channel quarter
+// (decode_kernel), or token x 48-channel half for D = 96
+// (decode96_dma_kernel); QK on integer dot8 units, PV in FP32 registers,
+// online softmax per wave, LDS merge of the waves; the split that finishes
+// last for its (row, head) does the log-sum-exp merge of the splits and the
+// live token, the V inverse rotation and the BF16 output.
+// Every split prepares the query again: the 32 KB of R_k come from L2 and the
+// arithmetic overlaps the first page loads, where a prepare launch before the
+// decode launch took 5 us and its gap in every split call.
+// The BF16 baseline keeps separate prepare and merge launches.
 #include "rq_chain.h"
 #include "rq_device.h"
 #include "rq_kernels.h"
+#include "rq_plan.h"
 
 namespace rq {
 
@@ -292,15 +287,13 @@ __device__ __forceinline__ void prepare_record(const AttentionParams& p, int hea
     lds_barrier();
 }
 
-// Separate prepare pass (used when a (row, head) is split over several
-// workgroups, and by the BF16 baseline): one 128-thread workgroup per (row, head).
+// Separate prepare pass (used by the BF16 baseline): one 128-thread workgroup per (row, head).
 template <int D>
 __global__ __launch_bounds__(128) void prepare_kernel(AttentionParams p) {
     __shared__ int request_counts[2];
     const int64_t row = blockIdx.x;
     const int head = blockIdx.y;
     const int64_t rh = row * p.heads + head;
-    if (threadIdx.x == 0) p.arrivals[rh] = 0;
     PrepareInputs<D, 128> in;
     prepare_load<D, 128>(p, row, head, in);
     const int request = find_request_parallel(p.query_start_loc, p.requests, row, request_counts);
@@ -562,29 +555,42 @@ __device__ __forceinline__ void write_partial(const SplitResult& r, float* parti
     }
 }
 
-// One split covers the whole history of this (row, head): merge the waves
-// (`merge_waves()` returns this split's SplitResult), fold in the live token,
-// inverse-rotate V and write the BF16 output without a round trip through the
-// partials.  R_v row c and the live value are loaded before the wave merge so
-// their latency overlaps it.
-template <int D, typename MergeWaves>
+// What the output of (row, head) takes beside the history sum: half `part` of
+// R_v row c for thread 128 part + c, and the live value.  Loaded before the
+// wave merge (and, for a split, before its arrival) so that their latency
+// overlaps it.
+template <int D>
+struct OutputInputs {
+    uint4 rv[D / 16];
+    float v_live;
+};
+
+template <int D>
+__device__ __forceinline__ OutputInputs<D> output_load(const AttentionParams& p, int64_t row, int head) {
+    OutputInputs<D> in;
+    const int tid = threadIdx.x;
+    const int c = tid & 127, part = tid >> 7;
+    if (p.value_rotation != nullptr && c < D && tid < 256) {
+        const uint4* r = reinterpret_cast<const uint4*>(p.value_rotation + ((int64_t)head * D + c) * D + part * (D / 2));
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) in.rv[i] = r[i];
+    }
+    in.v_live = tid < D ? bf16_f32(p.value[row * p.value_stride + head * D + tid]) : 0.f;
+    return in;
+}
+
+// One split covers the whole history of this (row, head), merged over the
+// waves in `r`: fold in the live token, inverse-rotate V and write the BF16
+// output without a round trip through the partials.
+template <int D>
 __device__ __forceinline__ void finish_single(const AttentionParams& p, int64_t row, int head, float live,
-                                              MergeWaves merge_waves) {
+                                              const OutputInputs<D>& in, const SplitResult& r) {
     __shared__ float hist[128];
     __shared__ float halves[2][128];
     const int tid = threadIdx.x;
     const int c = tid & 127, part = tid >> 7;
     const bool in_halves = tid < 256;  // two threads per channel, half of k each
     const bool rotate = p.value_rotation != nullptr;
-    uint4 rv[D / 16];
-    if (rotate && c < D && in_halves) {
-        const uint4* r = reinterpret_cast<const uint4*>(p.value_rotation + ((int64_t)head * D + c) * D + part * (D / 2));
-#pragma unroll
-        for (int i = 0; i < D / 16; ++i) rv[i] = r[i];
-    }
-    const float v_live = tid < D ? bf16_f32(p.value[row * p.value_stride + head * D + tid]) : 0.f;
-
-    const SplitResult r = merge_waves();
     const float mx = fmaxf(r.m, live);
     const float w_hist = r.m == -INFINITY ? 0.f : exp2f(r.m - mx);
     const float w_live = exp2f(live - mx);
@@ -598,7 +604,7 @@ __device__ __forceinline__ void finish_single(const AttentionParams& p, int64_t 
 #pragma unroll
             for (int i = 0; i < D / 16; ++i) {
                 const float* hk = hist + part * (D / 2) + 8 * i;
-                const uint32_t w[4] = {rv[i].x, rv[i].y, rv[i].z, rv[i].w};
+                const uint32_t w[4] = {in.rv[i].x, in.rv[i].y, in.rv[i].z, in.rv[i].w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     a[j] = fmaf(hk[2 * j], f16_f32((uint16_t)(w[j] & 0xffffu)), a[j]);
@@ -614,7 +620,7 @@ __device__ __forceinline__ void finish_single(const AttentionParams& p, int64_t 
     __syncthreads();
     if (tid < D)
         p.output[row * p.output_stride + head * D + tid] =
-            (uint16_t)bf16_rn(fmaf(w_live * inv, v_live, halves[0][tid] + halves[1][tid]));
+            (uint16_t)bf16_rn(fmaf(w_live * inv, in.v_live, halves[0][tid] + halves[1][tid]));
 }
 
 // Page range of one split (in 16-token units) for the request of `row`.
@@ -671,6 +677,65 @@ __device__ __forceinline__ SplitRange fused_range(const AttentionParams& p, int6
     if (own) return guessed;
     const int request = find_request_parallel(p.query_start_loc, p.requests, row, lds_counts);
     return split_range_of(p, request, request < 0 ? 0 : lens[request], split);
+}
+
+// What a decode workgroup does: its row, its split's units and where the
+// split's partial goes.  Every field is wave-uniform.
+struct DecodeItem {
+    int64_t row;
+    SplitRange range;
+    int splits;
+    float* partials;     // of the (row, head)'s split 0
+    float* partial;      // of this split
+    uint64_t* arrivals;  // of the (row, head)
+    bool priority;       // every workgroup with work is resident at once
+};
+
+// Item `item` of `head`: from the plan over the request lengths, or, with
+// more requests than the plan covers, part item % p.splits of row
+// item / p.splits.
+template <int D, int PT>
+__device__ __forceinline__ DecodeItem decode_item(const AttentionParams& p, int item, int head, int* lds_counts) {
+    constexpr int UnitsPerPage = PT / kUnitTokens;
+    DecodeItem d;
+    int offset, total;
+    if (p.requests <= kPlanRequests) {
+        const int requests = (int)p.requests;
+        const int rows = (int)p.rows;
+        const PlanItem plan =
+            plan_item(requests, item, p.plan_target, p.plan_min_pages, INT_MAX, kMaxSplits, [&](int b) {
+                const int at = b < requests ? b : requests - 1;
+                const int lo = min(max(p.query_start_loc[at], 0), rows), hi = min(p.query_start_loc[at + 1], rows);
+                const int history = max(p.seq_lens[at] - 1, 0);
+                const int64_t pages = min((int64_t)(history / PT + (history % PT != 0)), p.max_pages);
+                return PlanEntry{b < requests ? max(hi - lo, 0) : 0, (int)pages, lo,
+                                 (int)min((int64_t)history, pages * PT)};
+            });
+        d.row = __builtin_amdgcn_readfirstlane(plan.first + plan.index);
+        d.splits = plan.splits;
+        d.range.request = plan.request;
+        d.range.history = plan.tokens;
+        d.range.unit_begin = (int64_t)__builtin_amdgcn_readfirstlane(split_begin(plan.length, plan.split, plan.splits)) * UnitsPerPage;
+        d.range.unit_end =
+            (int64_t)__builtin_amdgcn_readfirstlane(split_begin(plan.length, plan.split + 1, plan.splits)) * UnitsPerPage;
+        offset = plan.offset;
+        total = plan.total;
+    } else {
+        d.row = item / p.splits;
+        d.splits = p.splits;
+        d.range = fused_range(p, d.row, item % p.splits, lds_counts);
+        d.range.request = __builtin_amdgcn_readfirstlane(d.range.request);
+        d.range.history = uniform64(d.range.history);
+        d.range.unit_begin = uniform64(d.range.unit_begin);
+        d.range.unit_end = uniform64(d.range.unit_end);
+        offset = item - item % p.splits;
+        total = p.items;
+    }
+    d.arrivals = p.arrivals + (d.row * p.heads + head);
+    d.partials = p.partials + ((int64_t)head * p.items + offset) * (D + 2);
+    d.partial = p.partials + ((int64_t)head * p.items + item) * (D + 2);
+    d.priority = (int64_t)total * p.heads <= p.resident;
+    return d;
 }
 
 // Wave max of one value per token, broadcast to every lane (quad lanes agree).
@@ -760,9 +825,9 @@ constexpr int kMergeThreads = 256;
 constexpr int kMergeLdsFloats = kMaxSplits + 4 + 128 + kWaves * 128;
 
 template <int D>
-__device__ __forceinline__ void merge_output(const AttentionParams& p, int64_t row, int head, float* lds) {
+__device__ __forceinline__ void merge_output(const AttentionParams& p, int64_t row, int head, const float* partials,
+                                             int splits, float live, const OutputInputs<D>& in, float* lds) {
     const int tid = threadIdx.x;
-    const int64_t rh = row * p.heads + head;
     float* weights = lds;                    // [kMaxSplits]
     float* totals = lds + kMaxSplits;        // [2]: live weight, 1 / denominator
     float* hist = totals + 4;                // [128]
@@ -770,11 +835,10 @@ __device__ __forceinline__ void merge_output(const AttentionParams& p, int64_t r
     // Partials [split][D + 2] of this (row, head), read with coherent loads.
     constexpr uint32_t kSplitBytes = (D + 2) * 4;
     const __amdgpu_buffer_rsrc_t parts =
-        handoff_resource(p.partials + rh * p.splits * (int64_t)(D + 2), (uint32_t)(p.splits * kSplitBytes));
+        handoff_resource(partials, (uint32_t)(splits * kSplitBytes));
     if (tid < 64) {
         // One lane per split (splits <= 64): (m, l) of split tid.
-        const float live = p.prep[rh * kPrepFloats + 1];
-        const bool has = tid < p.splits;
+        const bool has = tid < splits;
         const float2 ml = has ? handoff_load2(parts, tid * kSplitBytes) : make_float2(-INFINITY, 0.f);
         float m = fmaxf(ml.x, live);
 #pragma unroll
@@ -800,7 +864,7 @@ __device__ __forceinline__ void merge_output(const AttentionParams& p, int64_t r
         float2 h = make_float2(0.f, 0.f);
         if (2 * pair < D) {
 #pragma unroll 8
-            for (int s = group; s < p.splits; s += groups) {
+            for (int s = group; s < splits; s += groups) {
                 const float2 v = handoff_load2(parts, s * kSplitBytes + 8 + 8 * pair);
                 h.x = fmaf(weights[s], v.x, h.x);
                 h.y = fmaf(weights[s], v.y, h.y);
@@ -818,20 +882,16 @@ __device__ __forceinline__ void merge_output(const AttentionParams& p, int64_t r
     }
     __syncthreads();
     // out[c] = sum_k hist[k] R_v[c][k]: half `part` of the k range per thread
-    // (the first 256 threads), R_v row c read straight from global memory (L2)
-    // as 16-byte vectors.
+    // (the first 256 threads).
     const bool in_halves = tid < 256;
     float o = 0.f;
     if (c < D && in_halves) {
         if (p.value_rotation != nullptr) {
-            const uint4* r = reinterpret_cast<const uint4*>(p.value_rotation + ((int64_t)head * D + c) * D +
-                                                            part * (D / 2));
             float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < D / 16; ++i) {
-                const uint4 v = r[i];
                 const float* hk = hist + part * (D / 2) + 8 * i;
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+                const uint32_t w[4] = {in.rv[i].x, in.rv[i].y, in.rv[i].z, in.rv[i].w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     a[j] = fmaf(hk[2 * j], f16_f32((uint16_t)(w[j] & 0xffffu)), a[j]);
@@ -847,9 +907,8 @@ __device__ __forceinline__ void merge_output(const AttentionParams& p, int64_t r
     if (in_halves) halves[part * 128 + c] = o;
     __syncthreads();
     if (tid < D) {
-        const float v = bf16_f32(p.value[row * p.value_stride + head * D + tid]);
         p.output[row * p.output_stride + head * D + tid] =
-            (uint16_t)bf16_rn(fmaf(totals[0], v, halves[tid] + halves[128 + tid]));
+            (uint16_t)bf16_rn(fmaf(totals[0], in.v_live, halves[tid] + halves[128 + tid]));
     }
 }
 
@@ -859,19 +918,30 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(AttentionParams p)
     __shared__ float lds[kMergeLdsFloats];
     const int64_t row = blockIdx.x;
     if (p.row_request[row] < 0) return;
-    merge_output<D>(p, row, blockIdx.y, lds);
+    const int64_t rh = row * p.heads + blockIdx.y;
+    merge_output<D>(p, row, blockIdx.y, p.partials + rh * p.splits * (int64_t)(D + 2), p.splits,
+                    p.prep[rh * kPrepFloats + 1], output_load<D>(p, row, blockIdx.y), lds);
 }
 
-// The split that finishes last for its (row, head) merges: every split
-// publishes its partial, then counts itself in `arrivals` (zeroed by prepare);
-// the one that sees splits - 1 earlier arrivals reads them all.  Nothing
-// waits, so no workgroup depends on another being scheduled.
-template <int D>
-__device__ __forceinline__ void finish_split(const AttentionParams& p, int64_t row, int head) {
+// The end of a decode workgroup: `merge_waves()` returns its split's
+// SplitResult.  The split that finishes last for its (row, head) merges:
+// every split publishes its partial, then counts itself in the pair's
+// arrival word; the one that sees splits - 1 earlier arrivals reads them
+// all.  Nothing waits, so no workgroup depends on another being scheduled.
+template <int D, typename MergeWaves>
+__device__ __forceinline__ void finish_item(const AttentionParams& p, const DecodeItem& item, int head, float live,
+                                            MergeWaves merge_waves) {
     __shared__ float lds[kMergeLdsFloats];
     __shared__ int last;
-    if (!arrive_last(&p.arrivals[row * p.heads + head], p.splits, &last)) return;
-    merge_output<D>(p, row, head, lds);
+    const OutputInputs<D> in = output_load<D>(p, item.row, head);
+    const SplitResult r = merge_waves();
+    if (item.splits == 1) {
+        finish_single<D>(p, item.row, head, live, in, r);
+        return;
+    }
+    write_partial<D>(r, item.partial);
+    if (!arrive_last_tagged(item.arrivals, item.splits, &last)) return;
+    merge_output<D>(p, item.row, head, item.partials, item.splits, live, in, lds);
 }
 
 #ifndef RQ_DECODE_MIN_WAVES
@@ -891,10 +961,7 @@ void decode_kernel(AttentionParams p) {
     const int qd = lane & 3;
     const bool lane_active = qd < Quarters;
     const int lq = lane_active ? qd : 0;
-    const int split = blockIdx.x % p.splits;
-    const int64_t rh = blockIdx.x / p.splits;
-    const int head = (int)(rh % p.heads);
-    const int64_t row = rh / p.heads;
+    const int head = (int)(blockIdx.x % (unsigned)p.heads);
     // Nibble planes of q' per quarter: [quarter][anchor words 0..3 | loop words 0..3][plane]
     __shared__ __attribute__((aligned(16))) uint32_t planes_lds[4][8][4];
     __shared__ __attribute__((aligned(16))) float prep_lds[kPrepFloats];
@@ -902,26 +969,16 @@ void decode_kernel(AttentionParams p) {
     __shared__ __attribute__((aligned(16))) float scratch_lds[kWaves * 16 * 128];
     __shared__ int request_counts[kWaves];
 
-    // With one split per (row, head) this workgroup prepares its own query;
-    // otherwise prepare_kernel has written the record.  The request lookup
-    // comes first either way, so the first units' page loads are in flight
-    // while the query record is computed (the loop's first iteration uses them).
-    SplitRange range;
+    // The plan comes first, so the first units' page loads are in flight
+    // while the query record is computed (the loop's first iteration uses
+    // them).  Its fields are in scalar registers, so the block table below is
+    // read with scalar loads.
+    const DecodeItem item = decode_item<D, PT>(p, (int)(blockIdx.x / (unsigned)p.heads), head, request_counts);
+    if (item.range.request < 0) return;
+    const SplitRange& range = item.range;
     PrepareInputs<D, kDecodeThreads> in;
-    if (p.fused_prepare) {
-        prepare_load<D, kDecodeThreads>(p, row, head, in);
-        range = fused_range(p, row, split, request_counts);
-    } else {
-        range = split_range(p, p.row_request[row], split);
-    }
-    if (range.request < 0) return;
-    // The range is the same in every lane; kept in scalar registers so the
-    // block table below is read with scalar loads.
-    range.request = __builtin_amdgcn_readfirstlane(range.request);
-    range.history = uniform64(range.history);
-    range.unit_begin = uniform64(range.unit_begin);
-    range.unit_end = uniform64(range.unit_end);
-    float* partial = p.partials + (rh * p.splits + split) * (int64_t)(D + 2);
+    const uint64_t arrivals_seen = peek_arrivals(item.arrivals);
+    prepare_load<D, kDecodeThreads>(p, item.row, head, in);
 
     // Per-lane byte offsets inside a page (first 16-token half); the second
     // half of a 32-token page adds a wave-uniform step per region.
@@ -1002,13 +1059,8 @@ void decode_kernel(AttentionParams p) {
     // Table entries of the next iteration, read while this one computes.
     blocks = pair_blocks(first + 2 * kWaves);
 
-    if (p.fused_prepare) {
-        prepare_record<D, kDecodeThreads>(p, head, in, prep_lds);
-    } else {
-        const float* src = p.prep + rh * (int64_t)kPrepFloats;
-        for (int i = threadIdx.x; i < kPrepFloats; i += kDecodeThreads) prep_lds[i] = src[i];
-        __syncthreads();
-    }
+    prepare_record<D, kDecodeThreads>(p, head, in, prep_lds);
+    if (item.splits > 1 && threadIdx.x == 0) tag_arrivals(item.arrivals, p.call_tag, arrivals_seen);
     const float* prep = prep_lds;
     if (threadIdx.x < 128) {
         // thread -> (quarter, record, word, plane); prep stores [plane][word] per order
@@ -1116,7 +1168,7 @@ void decode_kernel(AttentionParams p) {
     // (the first iteration's were loaded before the query preparation).
     const int iterations =
         first < range.unit_end ? (int)((range.unit_end - first + 2 * kWaves - 1) / (2 * kWaves)) : 0;
-    const StreamPriority priority(iterations, p.stream_priority != 0);
+    const StreamPriority priority(iterations, item.priority);
     int step = 0;
     for (int64_t u = first; u < range.unit_end; u += 2 * kWaves, ++step) {
         priority.set(step);
@@ -1134,13 +1186,8 @@ void decode_kernel(AttentionParams p) {
         acc[i] += cst0;
         acc[16 + i] += cst1;
     }
-    if (p.splits == 1) {
-        finish_single<D>(p, row, head, prep_lds[1],
-                         [&] { return merge_waves<D>(acc, m, l, lane, wave, lane_active, scratch_lds); });
-    } else {
-        write_partial<D>(merge_waves<D>(acc, m, l, lane, wave, lane_active, scratch_lds), partial);
-        finish_split<D>(p, row, head);
-    }
+    finish_item<D>(p, item, head, prep_lds[1],
+                   [&] { return merge_waves<D>(acc, m, l, lane, wave, lane_active, scratch_lds); });
 }
 
 // ------------------------------------------------------------------ D = 96 packed decode
@@ -1408,10 +1455,7 @@ void decode96_dma_kernel(AttentionParams p) {
     const bool upper = slot >= 16;       // slot on the iteration's second unit
     const int tok = PT == 32 ? slot : (slot & 15);  // token row inside the slot's page
     const int page_of_slot = PT == 32 ? 0 : (upper ? 1 : 0);
-    const int split = blockIdx.x % p.splits;
-    const int64_t rh = blockIdx.x / p.splits;
-    const int head = (int)(rh % p.heads);
-    const int64_t row = rh / p.heads;
+    const int head = (int)(blockIdx.x % (unsigned)p.heads);
     __shared__ __attribute__((aligned(16))) float prep_lds[kPrepFloats];
     __shared__ __attribute__((aligned(16))) uint32_t half_planes[2][2][6][4];
     __shared__ int request_counts[kWaves];
@@ -1428,20 +1472,12 @@ void decode96_dma_kernel(AttentionParams p) {
                                                                                            : kScratchBytes];
     float* scratch_lds = reinterpret_cast<float*>(ring2);
 
-    SplitRange range;
+    const DecodeItem item = decode_item<D, PT>(p, (int)(blockIdx.x / (unsigned)p.heads), head, request_counts);
+    if (item.range.request < 0) return;
+    const SplitRange& range = item.range;
     PrepareInputs<D, kDecodeThreads> in;
-    if (p.fused_prepare) {
-        prepare_load<D, kDecodeThreads>(p, row, head, in);
-        range = fused_range(p, row, split, request_counts);
-    } else {
-        range = split_range(p, p.row_request[row], split);
-    }
-    if (range.request < 0) return;
-    range.request = __builtin_amdgcn_readfirstlane(range.request);
-    range.history = uniform64(range.history);
-    range.unit_begin = uniform64(range.unit_begin);
-    range.unit_end = uniform64(range.unit_end);
-    float* partial = p.partials + (rh * p.splits + split) * (int64_t)(D + 2);
+    const uint64_t arrivals_seen = peek_arrivals(item.arrivals);
+    prepare_load<D, kDecodeThreads>(p, item.row, head, in);
 
     const ConstantInt32* table =
         (const ConstantInt32*)(p.block_table + (int64_t)range.request * p.block_table_stride);
@@ -1516,10 +1552,6 @@ void decode96_dma_kernel(AttentionParams p) {
     // share vmcnt with the DMA loads).
     static_assert(kDma96Stages == 3, "the loop below rotates three stages");
     PagePair pages0 = pages_of(0), pages1 = pages_of(1), pages2;
-    if (!p.fused_prepare) {
-        const float* src = p.prep + rh * (int64_t)kPrepFloats;
-        for (int i = threadIdx.x; i < kPrepFloats; i += kDecodeThreads) prep_lds[i] = src[i];
-    }
     // The prologue's own loads (R_k, q) may still be in flight: they are
     // older than the page loads, so the query preparation waits for them
     // only, and every wait of the loop below, which counts the page loads
@@ -1529,8 +1561,8 @@ void decode96_dma_kernel(AttentionParams p) {
     issue(pages0, Stage0{});
     issue(pages1, Stage1{});
 
-    if (p.fused_prepare) prepare_record<D, kDecodeThreads>(p, head, in, prep_lds);
-    else lds_barrier();
+    prepare_record<D, kDecodeThreads>(p, head, in, prep_lds);
+    if (item.splits > 1 && threadIdx.x == 0) tag_arrivals(item.arrivals, p.call_tag, arrivals_seen);
     const float* prep = prep_lds;
     const float delta = prep[0];
     const float q_mean_anchor = h == 0 ? prep[2] : 0.f;  // added once per token
@@ -1593,7 +1625,7 @@ void decode96_dma_kernel(AttentionParams p) {
 
     // Iteration g consumes stage g % 3 after issuing stage (g + 2) % 3
     // (iteration g - 1's stage, whose reads are complete).
-    const StreamPriority priority(iterations, p.stream_priority != 0);
+    const StreamPriority priority(iterations, item.priority);
     auto iteration = [&](int g, auto stage_constant) __attribute__((always_inline)) {
         constexpr int stage = decltype(stage_constant)::value;
         constexpr int ahead = (stage + 2) % 3;
@@ -1715,13 +1747,8 @@ void decode96_dma_kernel(AttentionParams p) {
     for (int b = 0; b < 3; ++b)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[16 * b + i] += cst[b];
-    if (p.splits == 1) {
-        finish_single<D>(p, row, head, prep_lds[1],
-                         [&] { return merge_waves_half(acc, m, l, lane, wave, scratch_lds); });
-    } else {
-        write_partial<D>(merge_waves_half(acc, m, l, lane, wave, scratch_lds), partial);
-        finish_split<D>(p, row, head);
-    }
+    finish_item<D>(p, item, head, prep_lds[1],
+                   [&] { return merge_waves_half(acc, m, l, lane, wave, scratch_lds); });
 }
 
 // ------------------------------------------------------------------ adjacent mode, loops > 0
@@ -1747,10 +1774,7 @@ void decode_chain_kernel(AttentionParams p) {
     const int qd = lane & 3;
     const bool lane_active = qd < Quarters;
     const int lq = lane_active ? qd : 0;
-    const int split = blockIdx.x % p.splits;
-    const int64_t rh = blockIdx.x / p.splits;
-    const int head = (int)(rh % p.heads);
-    const int64_t row = rh / p.heads;
+    const int head = (int)(blockIdx.x % (unsigned)p.heads);
     __shared__ __attribute__((aligned(16))) float prep_lds[kPrepFloats];
     // bf16(mu_r) of records 0 .. L - 1 (the K plane's chain), FP32.
     __shared__ __attribute__((aligned(16))) float mean_lds[kMaxRecords][128];
@@ -1759,20 +1783,12 @@ void decode_chain_kernel(AttentionParams p) {
     __shared__ __attribute__((aligned(16))) uint32_t qpair_lds[2][64];
     __shared__ int request_counts[kWaves];
 
-    SplitRange range;
+    const DecodeItem item = decode_item<D, PT>(p, (int)(blockIdx.x / (unsigned)p.heads), head, request_counts);
+    if (item.range.request < 0) return;
+    const SplitRange& range = item.range;
     PrepareInputs<D, kDecodeThreads> in;
-    if (p.fused_prepare) {
-        prepare_load<D, kDecodeThreads>(p, row, head, in);
-        range = fused_range(p, row, split, request_counts);
-    } else {
-        range = split_range(p, p.row_request[row], split);
-    }
-    if (range.request < 0) return;
-    range.request = __builtin_amdgcn_readfirstlane(range.request);
-    range.history = uniform64(range.history);
-    range.unit_begin = uniform64(range.unit_begin);
-    range.unit_end = uniform64(range.unit_end);
-    float* partial = p.partials + (rh * p.splits + split) * (int64_t)(D + 2);
+    const uint64_t arrivals_seen = peek_arrivals(item.arrivals);
+    prepare_load<D, kDecodeThreads>(p, item.row, head, in);
 
     for (int i = threadIdx.x; i < (Links - 1) * 128; i += kDecodeThreads) {
         const int r = i / 128, c = i % 128;
@@ -1780,13 +1796,8 @@ void decode_chain_kernel(AttentionParams p) {
                              ? bf16_f32(bf16_rn(p.key_mean_all[((int64_t)r * p.heads + head) * D + c]))
                              : 0.f;
     }
-    if (p.fused_prepare) {
-        prepare_record<D, kDecodeThreads>(p, head, in, prep_lds);
-    } else {
-        const float* src = p.prep + rh * (int64_t)kPrepFloats;
-        for (int i = threadIdx.x; i < kPrepFloats; i += kDecodeThreads) prep_lds[i] = src[i];
-        __syncthreads();
-    }
+    prepare_record<D, kDecodeThreads>(p, head, in, prep_lds);
+    if (item.splits > 1 && threadIdx.x == 0) tag_arrivals(item.arrivals, p.call_tag, arrivals_seen);
     // q' (FP32, log2 units, scale folded in) as a high and a low BF16 pair
     // per two channels (16 bits of mantissa: relative error 2^-17), so the
     // score is two v_dot2_f32_bf16 per channel pair.  It stays in LDS and is
@@ -1921,13 +1932,8 @@ void decode_chain_kernel(AttentionParams p) {
         pages = next;
     }
 
-    if (p.splits == 1) {
-        finish_single<D>(p, row, head, prep_lds[1],
-                         [&] { return merge_waves<D>(acc, m, l, lane, wave, lane_active, scratch_lds); });
-    } else {
-        write_partial<D>(merge_waves<D>(acc, m, l, lane, wave, lane_active, scratch_lds), partial);
-        finish_split<D>(p, row, head);
-    }
+    finish_item<D>(p, item, head, prep_lds[1],
+                   [&] { return merge_waves<D>(acc, m, l, lane, wave, lane_active, scratch_lds); });
 }
 
 // ------------------------------------------------------------------ BF16 baseline decode
@@ -2021,29 +2027,30 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_bf16_kernel(AttentionPa
 
 // ------------------------------------------------------------------ launch
 
-// The launch parameters with stream_priority set: whether `blocks`
-// workgroups of `kernel` fit the device at once.
-inline AttentionParams with_priority(const AttentionParams& params, int per_cu, int64_t blocks) {
+// The launch parameters with `resident` set: the workgroups of the kernel
+// that the device holds at once.
+inline AttentionParams with_resident(const AttentionParams& params, int per_cu) {
     AttentionParams p = params;
-    p.stream_priority = blocks <= (int64_t)per_cu * p.compute_units ? 1 : 0;
+    p.resident = (int64_t)per_cu * p.compute_units;
     return p;
 }
 
+inline dim3 item_grid(const AttentionParams& p) { return dim3((unsigned)((int64_t)p.items * p.heads)); }
+
 template <int D, int PT, int BA, int GA, int BL, int GL, bool HasL>
 void launch_decode(const AttentionParams& p, hipStream_t stream) {
-    const unsigned blocks = (unsigned)(p.rows * p.heads * p.splits);
     if constexpr (D == 96) {
         // Per-lane page offsets are 32-bit buffer offsets into one plane.
         if (p.plane_stride > 0 && p.plane_stride <= (int64_t)UINT32_MAX - 0x10000) {
             const auto kernel = decode96_dma_kernel<PT, BA, GA, BL, GL, HasL>;
             static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kDecodeThreads);
-            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kDecodeThreads), 0, stream, with_priority(p, per_cu, blocks));
+            hipLaunchKernelGGL(kernel, item_grid(p), dim3(kDecodeThreads), 0, stream, with_resident(p, per_cu));
             return;
         }
     }
     const auto kernel = decode_kernel<D, PT, BA, GA, BL, GL, HasL>;
     static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kDecodeThreads);
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kDecodeThreads), 0, stream, with_priority(p, per_cu, blocks));
+    hipLaunchKernelGGL(kernel, item_grid(p), dim3(kDecodeThreads), 0, stream, with_resident(p, per_cu));
 }
 
 template <int D, int PT, int BA, int GA>
@@ -2080,10 +2087,9 @@ bool dispatch_anchor(const AttentionParams& p, hipStream_t stream) {
 
 template <int D, int PT, int Links>
 void launch_chain_links(const AttentionParams& p, hipStream_t stream) {
-    const unsigned blocks = (unsigned)(p.rows * p.heads * p.splits);
     const auto kernel = decode_chain_kernel<D, PT, Links>;
     static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kDecodeThreads);
-    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kDecodeThreads), 0, stream, with_priority(p, per_cu, blocks));
+    hipLaunchKernelGGL(kernel, item_grid(p), dim3(kDecodeThreads), 0, stream, with_resident(p, per_cu));
 }
 
 template <int D, int PT>
@@ -2108,7 +2114,7 @@ hipError_t launch_all(const AttentionParams& p, hipStream_t stream, hipEvent_t b
                       bool bf16) {
     // The timed window holds every launch of the call.
     if (begin) (void)hipEventRecord(begin, stream);
-    if (bf16 || !p.fused_prepare)
+    if (bf16)
         hipLaunchKernelGGL((prepare_kernel<D>), dim3((unsigned)p.rows, (unsigned)p.heads), dim3(128), 0,
                            stream, p);
     if (bf16) {

@@ -9,15 +9,18 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
+#include <random>
 #include <string>
 #include <vector>
 
 #include "../../include/rq_hip.h"
 #include "rq_kernels.h"
+#include "rq_plan.h"
 
 namespace {
 
@@ -104,21 +107,25 @@ int compute_units() {
     return g_compute_units[device];
 }
 
-// Splits per (row, head): enough workgroups for `target` (by default
-// `per_cu` per compute unit: two for the streaming decode kernels, whose long
-// page streams per workgroup measured best at batch 32 x 8k, one at D = 96),
-// at least 16 pages per split, at most rq::kMaxSplits.  With 4 pages per
-// split a one-row call's 512 workgroups spent their time in the prologue and
-// the merge: 4-call step at batch 1, 16 heads, 2048 history 90.3 -> 74.1 us
-// with 16 pages (4096: 93.3 -> 83.9 us; 8192 and every batch-8 shape keep
-// their counts and times).
-int split_count(int64_t rows, int heads, int64_t max_pages, int per_cu = 2) {
+// Workgroups that a decode call is spread over: `per_cu` per compute unit,
+// or the caller's rq_set_split_target.
+int64_t split_target(int per_cu) {
     int64_t target;
     {
         std::lock_guard<std::mutex> lock(g_device_mutex);
         target = g_split_target;
     }
-    if (target <= 0) target = (int64_t)per_cu * compute_units();
+    return target > 0 ? target : (int64_t)per_cu * compute_units();
+}
+
+// Splits per (row, head) where every row takes the same count (the BF16
+// baseline, packed decode past rq::kPlanRequests requests) and the workspace
+// size of packed decode: enough workgroups for the target (two per compute
+// unit for the streaming decode kernels, whose long page streams per
+// workgroup measured best at batch 32 x 8k, one at D = 96), at least 16 pages
+// per split, at most rq::kMaxSplits.
+int split_count(int64_t rows, int heads, int64_t max_pages, int per_cu = 2) {
+    const int64_t target = split_target(per_cu);
     const int64_t pairs = std::max<int64_t>(1, rows * heads);
     int64_t splits = (target + pairs - 1) / pairs;
     const int64_t by_pages = std::max<int64_t>(1, (max_pages + 15) / 16);
@@ -128,8 +135,9 @@ int split_count(int64_t rows, int heads, int64_t max_pages, int per_cu = 2) {
 
 size_t align256(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 
+// Workspace of the BF16 baseline, and the size that a packed call requires.
 struct WorkspaceLayout {
-    size_t row_request, arrivals, prep, partials, total;
+    size_t row_request, prep, partials, total;
 };
 
 constexpr int64_t kMultiRowMinRows = 3;          // anchor-loop calls
@@ -190,11 +198,64 @@ MultiRowLayout multirow_layout(int64_t rows, int heads, int splits) {
     return w;
 }
 
+// A call's tag for its arrival words (rq_plan.h), never 0.
+uint64_t next_call_tag() {
+    static std::atomic<uint64_t> counter{[] {
+        std::random_device source;
+        return ((uint64_t)source() << 32) | source();
+    }()};
+    constexpr uint64_t kMask = (1ull << 56) - 1;
+    uint64_t tag;
+    do tag = counter.fetch_add(1, std::memory_order_relaxed) & kMask;
+    while (tag == 0);
+    return tag;
+}
+
+// The grid of a packed decode call, planned on the device (decode_item in
+// attention.hip): `items` workgroups per head and the `target` over which a
+// head's work is spread.  `splits` is split_count of the call, `bytes` the
+// workspace its layout with that many splits for every row takes; the
+// arrival words and one partial per item fit in it (they need no query
+// records).  The plan's items number at most rows + target, and at most
+// rows x ceil(max_pages / min_pages).
+struct DecodePlan {
+    int items, target, min_pages;
+    size_t partials;  // offset in the workspace, behind the arrival words
+};
+
+// Least tokens of one split: a workgroup spends about 10 us in its prologue,
+// merge and output whatever it streams.  Adjacent-mode chains take 512 (8
+// requests of 514..4096 tokens x 16 heads, loops 1 / 2 / 3: 41 / 54 / 62 us at
+// 256, 36 / 44 / 53 us at 512), the other loops 256 (one request of 2047
+// tokens: 14.1 us per residual call at 256 and at 64, 16.2 us at 512).
+constexpr int kPlanMinTokens = 256, kChainMinTokens = 512;
+
+DecodePlan decode_plan(int64_t rows, int heads, int head_dim, int64_t requests, int64_t max_pages, int splits,
+                       int per_cu, int min_tokens, int page_tokens, size_t bytes) {
+    DecodePlan plan;
+    const int min_pages = plan.min_pages = min_tokens / page_tokens;
+    plan.partials = align256(sizeof(uint64_t) * (size_t)rows * heads);
+    if (requests > rq::kPlanRequests) {
+        plan.items = (int)(rows * splits);
+        plan.target = 0;
+        return plan;
+    }
+    const int64_t target = split_target(per_cu);
+    int64_t per_head = (target + heads - 1) / heads;
+    const int64_t fit = (int64_t)((bytes - plan.partials) / (sizeof(float) * (head_dim + 2)) / (size_t)heads);
+    per_head = std::max<int64_t>(0, std::min<int64_t>(per_head, fit - rows));
+    // The device sums rows x pages in 31 bits.
+    if (max_pages > 0 && rows > INT32_MAX / max_pages) per_head = 0;
+    const int64_t by_pages = std::max<int64_t>(1, (max_pages + min_pages - 1) / min_pages);
+    plan.items = (int)(by_pages <= per_head / rows ? rows * by_pages : rows + per_head);
+    plan.target = (int)per_head;
+    return plan;
+}
+
 WorkspaceLayout workspace_layout(int64_t rows, int heads, int head_dim, int splits) {
     WorkspaceLayout w;
     w.row_request = 0;
-    w.arrivals = align256(sizeof(int32_t) * (size_t)rows);
-    w.prep = w.arrivals + align256(sizeof(int32_t) * (size_t)rows * heads);
+    w.prep = align256(sizeof(int32_t) * (size_t)rows) + align256(sizeof(int32_t) * (size_t)rows * heads);
     w.partials = w.prep + align256(sizeof(float) * (size_t)rows * heads * rq::kPrepFloats);
     w.total = w.partials + align256(sizeof(float) * (size_t)rows * heads * splits * (head_dim + 2));
     return w;
@@ -322,11 +383,11 @@ int rq_quantize(int records, const void* const* key_ptrs, const int64_t* key_str
 
 // One workspace serves both paths of a packed attention call (the per-row
 // decode kernels and the multi-row kernels), so its size is the larger one.
-static int chain_splits(int64_t rows, int heads, int64_t max_pages);
+constexpr int kChainPerCu = 8;
 
 static size_t attention_workspace_total(int64_t rows, int heads, int head_dim, int64_t max_pages,
                                         int page_tokens) {
-    const int splits = std::max(split_count(rows, heads, max_pages), chain_splits(rows, heads, max_pages));
+    const int splits = std::max(split_count(rows, heads, max_pages), split_count(rows, heads, max_pages, kChainPerCu));
     size_t total = workspace_layout(rows, heads, head_dim, splits).total;
     if ((head_dim == 96 || head_dim == 128) && (page_tokens == 16 || page_tokens == 32))
         total = std::max(total,
@@ -396,32 +457,23 @@ static int attention_common(const void* query, int64_t query_stride, const void*
     p->block_table_stride = block_table_stride;
     p->max_pages = max_pages;
     p->row_request = reinterpret_cast<int32_t*>(ws + layout.row_request);
-    p->arrivals = reinterpret_cast<int32_t*>(ws + layout.arrivals);
     p->prep = reinterpret_cast<float*>(ws + layout.prep);
     p->partials = reinterpret_cast<float*>(ws + layout.partials);
     p->splits = splits;
     return RQ_OK;
 }
 
-// Splits per (row, head) of a packed attention call.  At D = 96 a call takes
-// one workgroup per (row, head) once those fill the compute units: every loop
-// runs decode96_dma_kernel (one token half per lane, pages staged in LDS),
-// which prepares its query inside the decode launch (one launch per call; at
-// 55 heads x B8 x 4096 the residual call measured 82.1, 85.8, 92.4 and 92.3
-// us at 1, 2, 3 and 4 splits).
-static int packed_splits(int64_t rows, int heads, int head_dim, int64_t max_pages) {
-    return split_count(rows, heads, max_pages, head_dim == 96 ? 1 : 2);
-}
+// Workgroups per compute unit that a packed decode call's plan spreads its
+// work over.  At D = 96 one (decode96_dma_kernel; at 55 heads x B8 x 4096 the
+// residual call measured 82.1, 85.8, 92.4 and 92.3 us at 1, 2, 3 and 4 splits
+// per (row, head)).
+static int packed_per_cu(int head_dim) { return head_dim == 96 ? 1 : 2; }
 
-// Splits per (row, head) of an adjacent-mode call past loop 0
-// (decode_chain_kernel).  That kernel is bound by its VALU work, not by HBM,
-// and shorter page spans per workgroup let one workgroup's prologue and
-// finish overlap another's chain: at batch 32 x 8k x 16 heads, loops 1 / 2 /
-// 3 measured 364 / 512 / 660 us at two workgroups per compute unit and
-// 320 / 498 / 628 us at eight.
-static int chain_splits(int64_t rows, int heads, int64_t max_pages) {
-    return split_count(rows, heads, max_pages, 8);
-}
+// Of an adjacent-mode call past loop 0 (decode_chain_kernel): that kernel is
+// bound by its VALU work, not by HBM, and shorter page spans per workgroup
+// let one workgroup's prologue and finish overlap another's chain: at batch
+// 32 x 8k x 16 heads, loops 1 / 2 / 3 measured 364 / 512 / 660 us at two
+// workgroups per compute unit and 320 / 498 / 628 us at eight (kChainPerCu).
 
 static int attention_packed(const void* query, int64_t query_stride, const void* key, int64_t key_stride,
                             const void* value, int64_t value_stride, void* output, int64_t output_stride,
@@ -537,8 +589,9 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
     }
     rq::AttentionParams p;
     // Never more splits than rq_attention_workspace_bytes() provides for.
-    const int splits = adjacent && loop_index > 0 ? chain_splits(rows, heads, max_pages)
-                                                  : packed_splits(rows, heads, head_dim, max_pages);
+    const bool chain = adjacent && loop_index > 0;
+    const int per_cu = chain ? kChainPerCu : packed_per_cu(head_dim);
+    const int splits = split_count(rows, heads, max_pages, per_cu);
     const int anchor_record = adjacent ? 0 : anchor_index;
     status = attention_common(query, query_stride, key, key_stride, value, value_stride, output,
                               output_stride, rows, heads, head_dim, query_start_loc, seq_lens, requests,
@@ -561,10 +614,19 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
     p.residual = regions[loop_index];
     p.key_mean_loop = key_mean ? key_mean + (int64_t)loop_index * heads * head_dim : nullptr;
     p.key_mean_anchor = (key_mean && p.has_residual) ? key_mean + (int64_t)anchor * heads * head_dim : nullptr;
-    p.fused_prepare = p.splits == 1 ? 1 : 0;
+    const DecodePlan plan =
+        decode_plan(rows, heads, head_dim, requests, max_pages, splits, per_cu,
+                    chain ? kChainMinTokens : kPlanMinTokens, page_tokens,
+                    workspace_layout(rows, heads, head_dim, splits).total);
+    p.items = plan.items;
+    p.plan_target = plan.target;
+    p.plan_min_pages = plan.min_pages;
+    p.arrivals = static_cast<uint64_t*>(workspace);
+    p.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + plan.partials);
+    p.call_tag = next_call_tag();
     p.compute_units = compute_units();
     // Adjacent mode past loop 0 decodes the restore chain of records 0..loop.
-    p.chain_length = adjacent && loop_index > 0 ? loop_index + 1 : 0;
+    p.chain_length = chain ? loop_index + 1 : 0;
     for (int r = 0; r < p.chain_length; ++r) p.chain[r] = regions[r];
     p.key_mean_all = key_mean;
     hipEvent_t begin = nullptr, end = nullptr;
@@ -574,13 +636,12 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
 
 // ------------------------------------------------- attention without a workspace
 
-// Device scratch of rq_attention_noalloc: the attention workspace (request of
-// each row, split arrival counters, query records, split partials) for
-// callers that cannot allocate.  Each GPU holds its own copy for the life of
+// Device scratch of rq_attention_noalloc: the attention workspace (split
+// arrival words, split partials) for callers that cannot allocate.  Each GPU holds its own copy for the life of
 // the process; host code reaches it only through the address that
 // hipGetSymbolAddress returns on that device (ScratchState::address), never
-// through the name.  Every noalloc call on a GPU shares it; what must start
-// at zero (the arrival counters) is cleared by the call's own kernels.
+// through the name.  Every noalloc call on a GPU shares it; nothing in it
+// must start at zero (the arrival words carry the call's tag, rq_plan.h).
 // Calls made eagerly are ordered by the library: a call on another stream
 // than the previous one first makes its stream wait for an event recorded
 // after the previous call's kernels.  Calls captured into a graph are not

@@ -229,18 +229,6 @@ __device__ __forceinline__ int find_request_parallel(const int32_t* qsl, int64_t
     return total;
 }
 
-// Counts this workgroup's arrival at `counter` (after every thread's shared
-// stores) and returns true in every thread of the workgroup that arrives last
-// of `expected`.  Nothing waits for other workgroups.
-__device__ __forceinline__ bool arrive_last(int* counter, int expected, int* lds_flag) {
-    wait_vector_memory();
-    __syncthreads();
-    if (threadIdx.x == 0)
-        *lds_flag = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == expected - 1;
-    __syncthreads();
-    return *lds_flag != 0;
-}
-
 // ------------------------------------------------------------------ layout
 
 // Bytes of one token of record (bits, group) at head_dim D

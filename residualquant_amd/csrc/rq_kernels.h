@@ -173,14 +173,17 @@ struct AttentionParams {
     RecordRegion anchor;
     RecordRegion residual;
     int has_residual;
-    int32_t* row_request;  // workspace [rows]
-    int32_t* arrivals;     // workspace [rows, heads]: finished splits (zeroed by prepare)
-    float* prep;           // workspace [rows, heads, kPrepFloats]
-    float* partials;       // workspace [rows, heads, splits, D + 2]
-    int splits;
-    int fused_prepare;     // 1: each decode workgroup prepares its own query (requires splits == 1)
+    int32_t* row_request;  // BF16 baseline: workspace [rows]
+    float* prep;           // BF16 baseline: workspace [rows, heads, kPrepFloats]
+    uint64_t* arrivals;    // packed decode: workspace [rows, heads], tagged arrival counts (rq_plan.h)
+    uint64_t call_tag;     // of this call (56 bits)
+    float* partials;       // workspace: packed decode [heads, items, D + 2], BF16 [rows, heads, splits, D + 2]
+    int splits;            // BF16 baseline, and packed decode past kPlanRequests requests: splits of every row
+    int items;             // packed decode: workgroups per head
+    int plan_target;       // packed decode: workgroups per head that the plan spreads the work over
+    int plan_min_pages;    // and the least pages of one split
     int compute_units;     // of the launching device
-    int stream_priority;   // set by the launch: the grid fits the device at once, so its waves take StreamPriority
+    int64_t resident;      // set by the launch: workgroups the device holds at once
     // Adjacent mode, loop L > 0: records 0..L of the restore chain (chain_length = L + 1, else 0)
     // and the key means of every record [records, heads, D] (or null).
     RecordRegion chain[kMaxRecords];

@@ -1,0 +1,96 @@
+"""Decode calls whose work is planned on the device from the request lengths
+(csrc/rq_plan.h): requests of very different lengths, several rows of one
+request among single ones, requests without rows, more requests than one
+64-lane register set or than the plan covers, against the FP64 oracle with
+the attention bars."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import residualquant_amd as rq
+
+from .cases import OURO_G32, make_decode, oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+MAX_ABS, MEAN_ABS = 2e-2, 1e-3
+ADJACENT = ((4, 32), (2, 32), (2, 32), (2, 32))
+
+CASES = [
+    # lengths, rows per request, heads, dim, page tokens, mode, split target (0: default)
+    ([4097, 1, 257, 258, 33], None, 2, 128, 16, "anchor", 0),
+    ([2900, 513, 2, 1030], [1, 3, 0, 1], 2, 128, 32, "anchor", 0),
+    ([1700, 300, 16, 17], None, 3, 96, 16, "anchor", 64),
+    ([2600, 1, 600], None, 2, 128, 16, "adjacent", 0),
+    ([1400] + [3] * 64 + [700], None, 1, 128, 16, "anchor", 9),
+    ([600] + [2, 35] * 130, None, 1, 128, 16, "anchor", 600),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{len(c[0])}x{c[0][0]}-d{c[3]}-pt{c[4]}-{c[5]}-t{c[6]}")
+def test_planned_decode_matches_oracle(oracle, device, case):
+    print(f"[case] planned decode {str(case)[:120]}", flush=True)
+    lengths, rows, heads, dim, pt, mode, target = case
+    records = ADJACENT if mode == "adjacent" else OURO_G32
+    d = make_decode(lengths, heads, dim, records, seed=len(lengths) + dim, page_tokens=pt, mode=mode,
+                    anchor=0 if mode == "adjacent" else 3, rows_per_request=rows)
+    g = d.group
+    cache_np = g.oracle_cache(oracle)
+    cache = torch.from_numpy(cache_np).to(device)
+    kr, vr, km = g.device_args(device)
+    q, k, v = (t.to(device) for t in (d.query, d.key, d.value))
+    starts, lens, table = (t.to(device) for t in (d.query_start_loc, d.seq_lens, d.table))
+    # The arrival words of split rows lie in a workspace of any content.
+    size = rq.ops.attention_workspace_bytes(q.size(0), heads, dim, table.size(1), pt)
+    workspace = torch.full((size,), 0xFF, dtype=torch.uint8, device=device)
+    try:
+        rq.ops.set_split_target(target)
+        for loop in (0, 1, 3):
+            out = torch.full_like(q, float("nan"))
+            for _ in range(2):  # the second call finds the words as the first left them
+                rq.attention(q, k, v, cache, out, starts, lens, table, kr, vr, km, g.records, g.mode, g.anchor, loop,
+                             workspace=workspace)
+            expected = oracle_attention(oracle, d, cache_np, loop)
+            err = np.abs(out.float().cpu().numpy() - expected)
+            print(f"[case]   loop {loop}: max {err.max():.3g} mean {err.mean():.3g}", flush=True)
+            # Histories of a token or two leave outputs near 1 in magnitude,
+            # whose BF16 rounding alone averages up to 2^-9 of them (a quarter
+            # of an ulp, the ulp at most 2^-7 of the value).
+            bar = MEAN_ABS + np.abs(expected).mean() * 2.0 ** -9
+            assert err.max() <= MAX_ABS and err.mean() <= bar, (loop, err.max(), err.mean(), bar)
+    finally:
+        rq.ops.set_split_target(0)
+
+
+def test_planned_decode_replays(device):
+    """A captured call repeats its tag: every replay, with other lengths in
+    place of the captured ones, equals the eager call."""
+    d = make_decode([3000, 400, 50], 2, 128, OURO_G32, seed=5)
+    g = d.group
+    cache = torch.zeros(g.cache_shape, dtype=torch.uint8, device=device)
+    kr, vr, km = g.device_args(device)
+    rq.quantize([(a.to(device), b.to(device)) for a, b in g.pairs], cache, g.slots.to(device), kr, vr, km, g.records,
+                g.mode, g.anchor, g.coefficient)
+    q, k, v = (t.to(device) for t in (d.query, d.key, d.value))
+    starts, lens, table = (t.to(device) for t in (d.query_start_loc, d.seq_lens, d.table))
+    out, want = torch.empty_like(q), torch.empty_like(q)
+
+    def call(to):
+        rq.attention(q, k, v, cache, to, starts, lens, table, kr, vr, km, g.records, g.mode, g.anchor, 1)
+
+    call(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for lengths in ([3000, 400, 50], [257, 400, 50], [2800, 1, 33], [3000, 399, 2]):
+        lens.copy_(torch.tensor(lengths, dtype=torch.int32))
+        call(want)
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16)), lengths
