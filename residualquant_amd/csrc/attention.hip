@@ -22,6 +22,8 @@
 // arithmetic overlaps the first page loads, where a prepare launch before the
 // decode launch took 5 us and its gap in every split call.
 // The BF16 baseline keeps separate prepare and merge launches.
+#include <algorithm>
+
 #include "rq_chain.h"
 #include "rq_device.h"
 #include "rq_kernels.h"
@@ -699,18 +701,17 @@ __device__ __forceinline__ DecodeItem decode_item(const AttentionParams& p, int 
     constexpr int UnitsPerPage = PT / kUnitTokens;
     DecodeItem d;
     int offset, total;
-    if (p.requests <= kPlanRequests) {
+    if (p.requests > 0 && p.requests <= kPlanRequests) {
         const int requests = (int)p.requests;
         const int rows = (int)p.rows;
-        const PlanItem plan =
-            plan_item(requests, item, p.plan_target, p.plan_min_pages, INT_MAX, kMaxSplits, [&](int b) {
-                const int at = b < requests ? b : requests - 1;
-                const int lo = min(max(p.query_start_loc[at], 0), rows), hi = min(p.query_start_loc[at + 1], rows);
-                const int history = max(p.seq_lens[at] - 1, 0);
-                const int64_t pages = min((int64_t)(history / PT + (history % PT != 0)), p.max_pages);
-                return PlanEntry{b < requests ? max(hi - lo, 0) : 0, (int)pages, lo,
-                                 (int)min((int64_t)history, pages * PT)};
-            });
+        const int b = threadIdx.x & 63, at = b < requests ? b : requests - 1;
+        const int lo = min(max(p.query_start_loc[at], 0), rows), hi = min(p.query_start_loc[at + 1], rows);
+        const int history = max(p.seq_lens[at] - 1, 0);
+        const int64_t pages = min((int64_t)(history / PT + (history % PT != 0)), p.max_pages);
+        const int count = b < requests ? max(hi - lo, 0) : 0;
+        const PlanItem plan = plan_find(
+            requests, item, PlanSizes{p.plan_target, p.splits, p.plan_min_pages, INT_MAX, kMaxSplits, p.plan_round_pages, p.plan_round_target},
+            PlanEntry{count, (int)pages, lo, (int)min((int64_t)history, pages * PT), count});
         d.row = __builtin_amdgcn_readfirstlane(plan.first + plan.index);
         d.splits = plan.splits;
         d.range.request = plan.request;
@@ -2027,11 +2028,19 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_bf16_kernel(AttentionPa
 
 // ------------------------------------------------------------------ launch
 
-// The launch parameters with `resident` set: the workgroups of the kernel
-// that the device holds at once.
-inline AttentionParams with_resident(const AttentionParams& params, int per_cu) {
+// The launch parameters of a kernel of which the device holds `per_cu`
+// workgroups per compute unit at once: those and the grid.
+inline AttentionParams with_plan(const AttentionParams& params, int per_cu) {
     AttentionParams p = params;
     p.resident = (int64_t)per_cu * p.compute_units;
+    if (p.requests <= kPlanRequests) {
+        // No more than one item per plan_min_pages pages of every row.
+        const int64_t by_pages = std::max<int64_t>(1, (p.max_pages + p.plan_min_pages - 1) / p.plan_min_pages);
+        const int64_t ragged = by_pages <= p.plan_target / p.rows ? p.rows * by_pages : p.rows + p.plan_target;
+        p.items = (int)std::max(ragged, p.rows * p.splits);
+    } else {
+        p.items = (int)(p.rows * p.splits);
+    }
     return p;
 }
 
@@ -2044,13 +2053,15 @@ void launch_decode(const AttentionParams& p, hipStream_t stream) {
         if (p.plane_stride > 0 && p.plane_stride <= (int64_t)UINT32_MAX - 0x10000) {
             const auto kernel = decode96_dma_kernel<PT, BA, GA, BL, GL, HasL>;
             static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kDecodeThreads);
-            hipLaunchKernelGGL(kernel, item_grid(p), dim3(kDecodeThreads), 0, stream, with_resident(p, per_cu));
+            const AttentionParams planned = with_plan(p, per_cu);
+            hipLaunchKernelGGL(kernel, item_grid(planned), dim3(kDecodeThreads), 0, stream, planned);
             return;
         }
     }
     const auto kernel = decode_kernel<D, PT, BA, GA, BL, GL, HasL>;
     static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kDecodeThreads);
-    hipLaunchKernelGGL(kernel, item_grid(p), dim3(kDecodeThreads), 0, stream, with_resident(p, per_cu));
+    const AttentionParams planned = with_plan(p, per_cu);
+    hipLaunchKernelGGL(kernel, item_grid(planned), dim3(kDecodeThreads), 0, stream, planned);
 }
 
 template <int D, int PT, int BA, int GA>
@@ -2089,7 +2100,8 @@ template <int D, int PT, int Links>
 void launch_chain_links(const AttentionParams& p, hipStream_t stream) {
     const auto kernel = decode_chain_kernel<D, PT, Links>;
     static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kDecodeThreads);
-    hipLaunchKernelGGL(kernel, item_grid(p), dim3(kDecodeThreads), 0, stream, with_resident(p, per_cu));
+    const AttentionParams planned = with_plan(p, per_cu);
+    hipLaunchKernelGGL(kernel, item_grid(planned), dim3(kDecodeThreads), 0, stream, planned);
 }
 
 template <int D, int PT>

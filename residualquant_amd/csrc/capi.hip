@@ -186,16 +186,46 @@ int multirow_workspace_splits(int64_t rows, int heads, int64_t max_pages, int pa
     return multirow_splits(min_groups, max_pages, page_tokens);
 }
 
-struct MultiRowLayout {
-    size_t partials, row_shift, total;
-};
+// Workspace that a multi-row call requires: partials of `splits` splits of
+// every row (and 4 bytes per row and head that are not used).
+size_t multirow_bytes(int64_t rows, int heads, int splits) {
+    return align256(sizeof(float) * (size_t)rows * heads) +
+           align256(sizeof(float) * (size_t)rows * heads * splits * rq::kMultiRowEntry);
+}
 
-MultiRowLayout multirow_layout(int64_t rows, int heads, int splits) {
-    MultiRowLayout w;
-    w.partials = 0;
-    w.row_shift = align256(sizeof(float) * (size_t)rows * heads * splits * rq::kMultiRowEntry);
-    w.total = w.row_shift + align256(sizeof(float) * (size_t)rows * heads);
-    return w;
+// The plan of a multi-row call (multirow_plan in multirow.hip).  `splits`,
+// for every row alike, is what the call requires of its workspace
+// (multirow_bytes); the plan may use up to `bytes` of it.
+void plan_multirow(rq::MultiRowParams& m, int splits, size_t bytes) {
+    // Rows per stream tile: 16 when the call's requests average 16 rows or
+    // fewer, else 32.
+    m.tile_rows = m.rows <= 16 * m.requests ? 16 : 32;
+    m.splits = splits;
+    m.entries = m.rows * splits;
+    if (m.requests > rq::kPlanRequests) {
+        if ((int64_t)splits * ((m.rows + 15) / 16) > 65535) m.tile_rows = 32;  // the grid's z extent
+        return;
+    }
+    const int64_t tiles = std::max<int64_t>(1, (m.max_pages * m.page_tokens + 31) / 32);
+    const int64_t row_tiles = m.rows / m.tile_rows + m.requests;  // at most, over all requests
+    // A split's pages fit its LDS block table, so long histories take `forced` splits at least.
+    m.plan_max = (rq::kMultiRowMaxSplitPages - 1) * m.page_tokens / 32;
+    const int64_t forced = (tiles + m.plan_max - 1) / m.plan_max;
+    m.plan_min = 4;  // one tile per wave
+    m.plan_max_splits = (int)std::max<int64_t>(rq::kMultiRowMaxSplits, forced);
+    // Three quarters of the two stream workgroups that a compute unit holds, so
+    // that with every request's share rounded up to whole splits all are
+    // resident at once: 16 requests of 824..8192 tokens x 4 rows x 16 heads took
+    // 62.3 us per residual call at 3/4 against 79.5 us at 1 and 76.4 us at 1/2.
+    // Entries: at most rows x forced + target x tile_rows, and rows x max splits.
+    const int64_t fit = (int64_t)(bytes / (sizeof(float) * rq::kMultiRowEntry) / m.heads);
+    int64_t target = (3LL * compute_units() / 2 + m.heads - 1) / m.heads;
+    if (m.rows * m.plan_max_splits > fit)
+        target = std::max<int64_t>(0, std::min<int64_t>(target, (fit - m.rows * forced) / m.tile_rows));
+    if (row_tiles > INT32_MAX / tiles) target = 0;  // the device sums row tiles x history tiles in 31 bits
+    m.plan_target = (int)target;
+    m.entries = fit;
+    m.items = (int)std::max(row_tiles * forced + target, row_tiles * splits);
 }
 
 // A call's tag for its arrival words (rq_plan.h), never 0.
@@ -211,44 +241,36 @@ uint64_t next_call_tag() {
     return tag;
 }
 
-// The grid of a packed decode call, planned on the device (decode_item in
-// attention.hip): `items` workgroups per head and the `target` over which a
-// head's work is spread.  `splits` is split_count of the call, `bytes` the
-// workspace its layout with that many splits for every row takes; the
-// arrival words and one partial per item fit in it (they need no query
-// records).  The plan's items number at most rows + target, and at most
-// rows x ceil(max_pages / min_pages).
+// What the device-side plan of a packed decode call (decode_item in
+// attention.hip) may use.  `splits` is split_count of the call and `bytes`
+// the workspace that its layout with that many splits for every row takes;
+// the arrival words and one partial per item fit in it (they need no query
+// records).  The items number at most rows x splits where the lengths are
+// near equal, else at most rows + target.
 struct DecodePlan {
-    int items, target, min_pages;
+    int target, min_pages;
     size_t partials;  // offset in the workspace, behind the arrival words
 };
 
 // Least tokens of one split: a workgroup spends about 10 us in its prologue,
-// merge and output whatever it streams.  Adjacent-mode chains take 512 (8
-// requests of 514..4096 tokens x 16 heads, loops 1 / 2 / 3: 41 / 54 / 62 us at
-// 256, 36 / 44 / 53 us at 512), the other loops 256 (one request of 2047
-// tokens: 14.1 us per residual call at 256 and at 64, 16.2 us at 512).
-constexpr int kPlanMinTokens = 256, kChainMinTokens = 512;
+// merge and output whatever it streams (one request of 2047 tokens: 14.1 us
+// per residual call at 256 and at 64, 16.2 us at 512).  Adjacent-mode chains,
+// which spread over more workgroups than fit at once, take at least 512 where
+// fewer would not fit in one round (8 requests of 514..4096 tokens x 16 heads,
+// loops 1 / 2 / 3: 41 / 54 / 62 us at 256, 36 / 44 / 53 us at 512; one request
+// of 4096 tokens, loops 1 / 3: 28 / 37 us at 256, 30 / 42 us at 512).
+constexpr int kPlanMinTokens = 256, kChainRoundTokens = 512;
 
-DecodePlan decode_plan(int64_t rows, int heads, int head_dim, int64_t requests, int64_t max_pages, int splits,
-                       int per_cu, int min_tokens, int page_tokens, size_t bytes) {
+DecodePlan decode_plan(int64_t rows, int heads, int head_dim, int64_t max_pages, int per_cu,
+                       int page_tokens, size_t bytes) {
     DecodePlan plan;
-    const int min_pages = plan.min_pages = min_tokens / page_tokens;
+    plan.min_pages = kPlanMinTokens / page_tokens;
     plan.partials = align256(sizeof(uint64_t) * (size_t)rows * heads);
-    if (requests > rq::kPlanRequests) {
-        plan.items = (int)(rows * splits);
-        plan.target = 0;
-        return plan;
-    }
-    const int64_t target = split_target(per_cu);
-    int64_t per_head = (target + heads - 1) / heads;
     const int64_t fit = (int64_t)((bytes - plan.partials) / (sizeof(float) * (head_dim + 2)) / (size_t)heads);
-    per_head = std::max<int64_t>(0, std::min<int64_t>(per_head, fit - rows));
+    const int64_t target = (split_target(per_cu) + heads - 1) / heads;
+    plan.target = (int)std::max<int64_t>(0, std::min<int64_t>(target, fit - rows));
     // The device sums rows x pages in 31 bits.
-    if (max_pages > 0 && rows > INT32_MAX / max_pages) per_head = 0;
-    const int64_t by_pages = std::max<int64_t>(1, (max_pages + min_pages - 1) / min_pages);
-    plan.items = (int)(by_pages <= per_head / rows ? rows * by_pages : rows + per_head);
-    plan.target = (int)per_head;
+    if (max_pages > 0 && rows > INT32_MAX / max_pages) plan.target = 0;
     return plan;
 }
 
@@ -391,7 +413,7 @@ static size_t attention_workspace_total(int64_t rows, int heads, int head_dim, i
     size_t total = workspace_layout(rows, heads, head_dim, splits).total;
     if ((head_dim == 96 || head_dim == 128) && (page_tokens == 16 || page_tokens == 32))
         total = std::max(total,
-                         multirow_layout(rows, heads, multirow_workspace_splits(rows, heads, max_pages, page_tokens)).total);
+                         multirow_bytes(rows, heads, multirow_workspace_splits(rows, heads, max_pages, page_tokens)));
     return total;
 }
 
@@ -530,9 +552,10 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         const int64_t row_tiles = (rows + 31) / 32;
         const int64_t average_tiles = std::max<int64_t>(1, (rows / requests + 31) / 32);
         const int splits = multirow_splits(requests * heads * average_tiles, max_pages, page_tokens);
-        const MultiRowLayout layout = multirow_layout(rows, heads, splits);
-        if (workspace == nullptr || workspace_bytes < layout.total)
-            return workspace_too_small(layout.total, workspace_bytes, static_scratch);
+        const size_t required = multirow_bytes(rows, heads, splits);
+        const size_t full_bytes = attention_workspace_total(rows, heads, head_dim, max_pages, page_tokens);
+        if (workspace == nullptr || workspace_bytes < required)
+            return workspace_too_small(required, workspace_bytes, static_scratch);
         rq::RecordRegion regions[rq::kMaxRecords];
         fill_regions(head_dim, records, bits, groups, page_tokens, regions);
         rq::MultiRowParams m{};
@@ -572,13 +595,11 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         m.key_mean_loop = key_mean ? key_mean + (int64_t)loop_index * heads * head_dim : nullptr;
         m.key_mean_anchor = (key_mean && m.has_residual) ? key_mean + (int64_t)anchor * heads * head_dim : nullptr;
         m.causal = causal ? 1 : 0;
-        m.splits = splits;
-        m.row_tiles = (int)row_tiles;
         m.compute_units = compute_units();
-        uint8_t* ws = static_cast<uint8_t*>(workspace);
-        m.partials = reinterpret_cast<float*>(ws + layout.partials);
-        m.row_shift = reinterpret_cast<float*>(ws + layout.row_shift);
-        if ((int64_t)m.splits * m.row_tiles > 65535 || requests > (int64_t)INT32_MAX || rows > (int64_t)INT32_MAX)
+        m.partials = static_cast<float*>(workspace);
+        m.call_tag = next_call_tag();
+        plan_multirow(m, splits, std::min(workspace_bytes, full_bytes));
+        if ((int64_t)splits * row_tiles > 65535 || requests > (int64_t)INT32_MAX || rows > (int64_t)INT32_MAX)
             return fail(RQ_EINVAL, "Too many rows for one multi-row attention launch");
         hipEvent_t begin = nullptr, end = nullptr;
         if (timed) timing_events(stream, &begin, &end);
@@ -614,13 +635,23 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
     p.residual = regions[loop_index];
     p.key_mean_loop = key_mean ? key_mean + (int64_t)loop_index * heads * head_dim : nullptr;
     p.key_mean_anchor = (key_mean && p.has_residual) ? key_mean + (int64_t)anchor * heads * head_dim : nullptr;
-    const DecodePlan plan =
-        decode_plan(rows, heads, head_dim, requests, max_pages, splits, per_cu,
-                    chain ? kChainMinTokens : kPlanMinTokens, page_tokens,
-                    workspace_layout(rows, heads, head_dim, splits).total);
-    p.items = plan.items;
-    p.plan_target = plan.target;
+    const DecodePlan plan = decode_plan(rows, heads, head_dim, max_pages, per_cu, page_tokens,
+                                        workspace_layout(rows, heads, head_dim, splits).total);
     p.plan_min_pages = plan.min_pages;
+    p.plan_target = plan.target;
+    p.plan_round_pages = 0;
+    p.plan_round_target = 1;
+    if (chain) {
+        // One round: two workgroups per compute unit, three quarters of them
+        // by share (every request's last split is a part of one).
+        const int64_t round = 2LL * compute_units();
+        p.plan_round_pages = kChainRoundTokens / page_tokens;
+        p.plan_round_target = (int)std::max<int64_t>(1, round * 3 / 4 / heads);
+        p.splits = (int)std::min<int64_t>(
+            splits, std::max<int64_t>((round + rows * heads - 1) / (rows * heads),
+                                      (max_pages + p.plan_round_pages - 1) / p.plan_round_pages));
+        p.splits = std::max(p.splits, 1);
+    }
     p.arrivals = static_cast<uint64_t*>(workspace);
     p.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + plan.partials);
     p.call_tag = next_call_tag();

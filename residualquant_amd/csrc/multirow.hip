@@ -17,10 +17,10 @@
 // (the token order of each P.V step is permuted to match the accumulator
 // layout, and V^T is read with the same permutation).  Each of the four
 // waves takes every fourth tile with its own online softmax; the waves meet
-// once in LDS at the end and the workgroup writes one partial (m, l, O) per
-// row.  The query prologue (q . R_k) runs on MFMA as well.  A finish launch
-// per (request, head, 32-row tile) merges the splits, applies R_v^T (on
-// MFMA) and adds the live tokens.
+// once in LDS at the end.  The query prologue (q . R_k) runs on MFMA as well.
+// The workgroup whose split of a (request, head, row tile) ends last (the
+// others have written one partial (m, l, O) per row) merges the splits,
+// applies R_v^T (on MFMA), adds the live tokens and writes the output.
 //
 // Calls whose requests average 16 rows or fewer take 16-row tiles instead:
 // the same pages and dequantization, with the tile's products on
@@ -52,6 +52,7 @@
 #include "rq_chain.h"
 #include "rq_device.h"
 #include "rq_kernels.h"
+#include "rq_plan.h"
 
 namespace rq {
 
@@ -401,30 +402,426 @@ struct ChainDecoder {
     }
 };
 
+// ---------------------------------------------------------------- finish
+
+// Row strides of the finish kernel's tiles for head dim D: BF16/FP16 rows
+// (halves) and the rotated history [row][channel] (FP32).  Region A holds
+// the merged rows' FP16 parts for the rotation, then the causal tiles;
+// region B the rotated history.
+template <int D>
+struct FinishGeometry {
+    static constexpr int Parts = D / 16;
+    static constexpr int FS = D + 8;
+    static constexpr int OS = D + 4;
+    static constexpr int kRotationBytes = 2 * 32 * FS * 2;                  // high and low FP16 parts
+    static constexpr int kCausalBytes = 3 * 32 * FS * 2 + 32 * 33 * 4;     // q, k, v tiles and probabilities
+    static constexpr int kRegionABytes = kRotationBytes > kCausalBytes ? kRotationBytes : kCausalBytes;
+    static constexpr int kRegionBFloats = 32 * OS;
+    static_assert(kRegionABytes % 16 == 0 && kRegionABytes + 4 * kRegionBFloats <= Geometry<D>::kLdsBytes,
+                  "the finish fits in the tile LDS");
+};
+
+__device__ __forceinline__ float row8_max(float x) {
+    x = fmaxf(x, __shfl_xor(x, 1));
+    x = fmaxf(x, __shfl_xor(x, 2));
+    return fmaxf(x, __shfl_xor(x, 4));
+}
+
+__device__ __forceinline__ float row8_sum(float x) {
+    x += __shfl_xor(x, 1);
+    x += __shfl_xor(x, 2);
+    return x + __shfl_xor(x, 4);
+}
+
+// Whether rows of a BF16 tensor at `base` with row stride `stride`
+// (elements) start on 16-byte boundaries.  The boundary guarantees 8 bytes
+// for queries and keys and 2 bytes for values and outputs.
+__device__ __forceinline__ bool aligned_rows(const void* base, int64_t stride) {
+    return (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && (stride & 7) == 0;
+}
+
+// 16 consecutive BF16 values at `src` (a 32-byte aligned offset of an
+// aligned_rows tensor when `vec`) as two 16-byte words.
+__device__ __forceinline__ void load_halves16(const uint16_t* src, bool vec, uint4 (&w)[2]) {
+    if (vec) {
+        w[0] = reinterpret_cast<const uint4*>(src)[0];
+        w[1] = reinterpret_cast<const uint4*>(src)[1];
+    } else {
+        uint32_t x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = (uint32_t)src[2 * i] | ((uint32_t)src[2 * i + 1] << 16);
+        w[0] = make_uint4(x[0], x[1], x[2], x[3]);
+        w[1] = make_uint4(x[4], x[5], x[6], x[7]);
+    }
+}
+
+// Eight BF16 values of a 16-byte word as FP32.
+__device__ __forceinline__ void widen_bf16(uint4 w, float* x) {
+    const uint32_t v[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        x[2 * i] = bf16_f32(v[i] & 0xffffu);
+        x[2 * i + 1] = bf16_f32(v[i] >> 16);
+    }
+}
+
+// The finish of one (request, head) and its rows row0 .. row0 + TR - 1, by the
+// stream workgroup (256 threads) whose split of them ends last.  Thread t
+// takes row t / 8 of the tile and part p = t % 8 of it: the 16 channels
+// 16p..16p+15 of the merge, the query-key dots, the live values and the
+// output (parts p < D / 16), and the 4 tokens 4p..4p+3 of a live chunk's
+// scores.  The eight threads of a row are adjacent lanes of one wave.
+//   1. (finish_merge, only with several splits) merge the splits' partials
+//      (m, l, O) of each row (log2 units);
+//   2. rotate the tile's merged rows by R_v^T on the matrix cores (wave w
+//      computes output channels 32 w .. 32 w + 31);
+//   3. add the live tokens: in decode semantics the row's own token; in
+//      causal semantics the request's new tokens j <= row, 32 at a time with
+//      an online softmax over the rows' (m, l, O);
+//   4. write O / l in BF16.
+// A finish launch of its own read every partial back, one split or several,
+// and looked the plan up again: 2 requests of 4096 tokens x 8 rows took 26.5
+// us per residual call with it and 24.6 us without, 40 requests of 50..1500
+// tokens x 3 rows 54.0 and 43.8 us.
+
+// Loads that depend on the tile alone, issued before the split's arrival:
+// R_v as the B operand of the rotation MFMAs (wave w computes output channels
+// 32 w .. 32 w + 31, lane l takes row 32 w + l % 32 of R_v at features 16 m +
+// 8 (l / 32) .. + 7), the row's query and, in decode semantics, its own key
+// and value.
+template <int D>
+struct FinishInputs {
+    F16x8 rv[D / 16];
+    uint4 qw[2], kw[2], vw[2];
+};
+
+template <int D, int TR>
+__device__ __forceinline__ void finish_load(const MultiRowParams& p, int head, int first, int row0, int n,
+                                            FinishInputs<D>& in) {
+    const int tid = threadIdx.x;
+    const int r = tid >> 3, part = tid & 7;
+    const bool part_active = part < D / 16;
+    const int wave = tid >> 6, lane = tid & 63;
+    if (p.value_rotation != nullptr && wave < D / 32) {
+        const uint16_t* src = p.value_rotation + ((int64_t)head * D + 32 * wave + (lane & 31)) * D + 8 * (lane >> 5);
+#pragma unroll
+        for (int m = 0; m < D / 16; ++m) in.rv[m] = *reinterpret_cast<const F16x8*>(src + 16 * m);
+    }
+    const int64_t row = (int64_t)first + row0 + (r < TR && row0 + r < n ? r : 0);
+    // The part's 16 channels of a token row (part 0's for an inactive part,
+    // whose values are never used).
+    const int64_t channels = (int64_t)head * D + 16 * (part_active ? part : 0);
+    load_halves16(p.query + row * p.query_stride + channels, aligned_rows(p.query, p.query_stride), in.qw);
+    if (!part_active) in.qw[0] = in.qw[1] = make_uint4(0u, 0u, 0u, 0u);  // no share of the row's dots
+    if (!p.causal) {
+        load_halves16(p.key + row * p.key_stride + channels, aligned_rows(p.key, p.key_stride), in.kw);
+        load_halves16(p.value + row * p.value_stride + channels, aligned_rows(p.value, p.value_stride), in.vw);
+    }
+}
+
+// Merges the splits' partials of the thread's row and part online, four at a
+// time: every load of a batch is issued before any of its arithmetic (split
+// indices past the last are clamped and weighted zero, so no load sits behind
+// a branch).  Rows past the tile merge nothing.  `row_at` is the offset of the
+// row's split 0 in the tile's entries.
+__device__ __forceinline__ void finish_merge(__amdgpu_buffer_rsrc_t entries, uint32_t row_at, int splits, bool valid,
+                                             int part, float& m, float& l, float (&acc)[16]) {
+    m = -__builtin_inff();
+    l = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    for (int s0 = 0; s0 < splits; s0 += 4) {
+        float2 ml[4];
+        float4 ox[4][4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int s = s0 + b < splits ? s0 + b : splits - 1;
+            const uint32_t at = row_at + (uint32_t)(s * kMultiRowEntry * 4);
+            ml[b] = handoff_load2(entries, at);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ox[b][c] = handoff_load4(entries, at + 16 + 64 * part + 16 * c);
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const float ms = (valid && s0 + b < splits) ? ml[b].x : -__builtin_inff();
+            const float new_max = fmaxf(m, ms);
+            const float base = new_max == -__builtin_inff() ? 0.f : new_max;
+            const float keep = __builtin_amdgcn_exp2f(m - base), w = __builtin_amdgcn_exp2f(ms - base);
+            m = new_max;
+            l = fmaf(l, keep, ml[b].y * w);
+            const float x[16] = {ox[b][0].x, ox[b][0].y, ox[b][0].z, ox[b][0].w, ox[b][1].x, ox[b][1].y,
+                                 ox[b][1].z, ox[b][1].w, ox[b][2].x, ox[b][2].y, ox[b][2].z, ox[b][2].w,
+                                 ox[b][3].x, ox[b][3].y, ox[b][3].z, ox[b][3].w};
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] = fmaf(acc[i], keep, x[i] * w);
+        }
+    }
+}
+
+template <int D, int TR>
+__device__ __forceinline__ void finish_rows(const MultiRowParams& p, int head, int first, int row0, int n,
+                                            const FinishInputs<D>& in, float shift, float m, float l, float (&acc)[16],
+                                            uint8_t* lds) {
+    using G = FinishGeometry<D>;
+    constexpr int FS = G::FS;
+    constexpr int OS = G::OS;
+    uint8_t* region_a = lds;
+    float* hist_rot = reinterpret_cast<float*>(lds + G::kRegionABytes);
+    uint16_t* q_tile = reinterpret_cast<uint16_t*>(region_a);  // causal: the rows' queries
+    uint16_t* k_tile = q_tile + 32 * FS;                      // causal: 32 live keys
+    uint16_t* v_tile = k_tile + 32 * FS;                      // causal: their values
+    float* probs = reinterpret_cast<float*>(v_tile + 32 * FS);
+    const int tid = threadIdx.x;
+    const int r = tid >> 3, part = tid & 7;
+    const bool part_active = part < G::Parts;
+    const bool rotate = p.value_rotation != nullptr;
+    const int wave = tid >> 6, lane = tid & 63;
+    const bool rotation_wave = wave < D / 32;
+    const bool valid = r < TR && row0 + r < n;
+    const int64_t row = (int64_t)first + row0 + (valid ? r : 0);
+    const float scale = Geometry<D>::kScoreScale;  // log2(e) / sqrt(D)
+    const int64_t channels = (int64_t)head * D + 16 * (part_active ? part : 0);
+
+    // 2. hist . R_v^T for the tile's rows on the matrix cores: the merged
+    // rows divided by their sums (convex combinations of values, within the
+    // FP16 range) as FP16 high and low parts (~22 significant bits), times
+    // R_v (FP16), FP32 accumulation; the sums are multiplied back.
+    if (rotate) {
+        uint16_t* high = reinterpret_cast<uint16_t*>(region_a);  // [row][FS]
+        uint16_t* low = high + 32 * FS;
+        const float inverse = l > 0.f ? 1.0f / l : 0.f;
+        uint32_t hw[8], lw[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float x0 = acc[2 * i] * inverse, x1 = acc[2 * i + 1] * inverse;
+            const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
+            const _Float16 r0 = (_Float16)(x0 - (float)h0), r1 = (_Float16)(x1 - (float)h1);
+            hw[i] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+            lw[i] = (uint32_t)__builtin_bit_cast(uint16_t, r0) | ((uint32_t)__builtin_bit_cast(uint16_t, r1) << 16);
+        }
+        if (part_active) {
+            uint4* hd = reinterpret_cast<uint4*>(&high[r * FS + 16 * part]);
+            uint4* ld = reinterpret_cast<uint4*>(&low[r * FS + 16 * part]);
+            hd[0] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+            hd[1] = make_uint4(hw[4], hw[5], hw[6], hw[7]);
+            ld[0] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+            ld[1] = make_uint4(lw[4], lw[5], lw[6], lw[7]);
+        }
+        __syncthreads();
+        if (rotation_wave) {
+            // A operand: lane l takes merged row l % 32 at features 16 m + 8 (l / 32) .. + 7.
+            F32x16 rotated;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) rotated[e] = 0.f;
+            const int a_offset = (lane & 31) * FS + 8 * (lane >> 5);
+#pragma unroll
+            for (int mm = 0; mm < G::Parts; ++mm) {
+                rotated = mfma(*reinterpret_cast<const F16x8*>(&high[a_offset + 16 * mm]), in.rv[mm], rotated);
+                rotated = mfma(*reinterpret_cast<const F16x8*>(&low[a_offset + 16 * mm]), in.rv[mm], rotated);
+            }
+            // Register e of lane l: row 8 (e / 4) + 4 (l / 32) + e % 4, channel 32 w + l % 32.
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                hist_rot[(8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * OS + 32 * wave + (lane & 31)] = rotated[e];
+        }
+        __syncthreads();
+        if (part_active) {
+#pragma unroll
+            for (int c4 = 0; c4 < 4; ++c4) {
+                const float4 x = *reinterpret_cast<const float4*>(&hist_rot[r * OS + 16 * part + 4 * c4]);
+                acc[4 * c4] = x.x * l;
+                acc[4 * c4 + 1] = x.y * l;
+                acc[4 * c4 + 2] = x.z * l;
+                acc[4 * c4 + 3] = x.w * l;
+            }
+        }
+    }
+
+    // 3. Live tokens.
+    float q[16];
+    widen_bf16(in.qw[0], q);
+    widen_bf16(in.qw[1], q + 8);
+    if (!p.causal) {
+        // The row's own token.
+        float k[16], v[16];
+        widen_bf16(in.kw[0], k);
+        widen_bf16(in.kw[1], k + 8);
+        widen_bf16(in.vw[0], v);
+        widen_bf16(in.vw[1], v + 8);
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dot = fmaf(q[i], k[i], dot);
+        const float score = row8_sum(dot) * scale - shift;
+        const float total_max = fmaxf(m, score);
+        const float hist_weight = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - total_max);
+        const float live = __builtin_amdgcn_exp2f(score - total_max);
+        l = fmaf(l, hist_weight, live);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = fmaf(live, v[i], acc[i] * hist_weight);
+    } else {
+        // The request's new tokens 0 .. row0 + r, in chunks of 32 shared by the tile's rows.
+        const bool k_vec = aligned_rows(p.key, p.key_stride), v_vec = aligned_rows(p.value, p.value_stride);
+        __syncthreads();  // the rotation's reads of the region are done
+        if (part_active) {
+            uint4* dst = reinterpret_cast<uint4*>(&q_tile[r * FS + 16 * part]);
+            dst[0] = in.qw[0];
+            dst[1] = in.qw[1];
+        }
+        const int live_end = n < row0 + TR ? n : row0 + TR;
+        for (int c0 = 0; c0 < live_end; c0 += 32) {
+            __syncthreads();  // the previous chunk's reads are done
+            if (part_active) {
+                // Thread (r, part) stages the part's channels of live token c0 + r.
+                const int j = c0 + r;
+                uint4 kx[2] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)}, vx[2] = {kx[0], kx[1]};
+                if (j < n) {
+                    load_halves16(p.key + ((int64_t)first + j) * p.key_stride + channels, k_vec, kx);
+                    load_halves16(p.value + ((int64_t)first + j) * p.value_stride + channels, v_vec, vx);
+                }
+                uint4* kd = reinterpret_cast<uint4*>(&k_tile[r * FS + 16 * part]);
+                uint4* vd = reinterpret_cast<uint4*>(&v_tile[r * FS + 16 * part]);
+                kd[0] = kx[0];
+                kd[1] = kx[1];
+                vd[0] = vx[0];
+                vd[1] = vx[1];
+            }
+            __syncthreads();
+            // Scores of row r against tokens c0 + 4 part .. + 3.
+            float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+            for (int d = 0; d < D; d += 8) {
+                float qd[8];
+                widen_bf16(*reinterpret_cast<const uint4*>(&q_tile[r * FS + d]), qd);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float kd[8];
+                    widen_bf16(*reinterpret_cast<const uint4*>(&k_tile[(4 * part + i) * FS + d]), kd);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) s[i] = fmaf(qd[e], kd[e], s[i]);
+                }
+            }
+            float chunk_max = -__builtin_inff();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int j = c0 + 4 * part + i;
+                s[i] = (valid && j <= row0 + r && j < n) ? s[i] * scale - shift : -__builtin_inff();
+                chunk_max = fmaxf(chunk_max, s[i]);
+            }
+            const float new_max = fmaxf(m, row8_max(chunk_max));
+            const float base = new_max == -__builtin_inff() ? 0.f : new_max;
+            const float rescale = __builtin_amdgcn_exp2f(m - base);
+            m = new_max;
+            float chunk_sum = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float w = __builtin_amdgcn_exp2f(s[i] - base);
+                probs[r * 33 + 4 * part + i] = w;
+                chunk_sum += w;
+            }
+            l = fmaf(l, rescale, row8_sum(chunk_sum));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[i] *= rescale;
+            wave_sync();  // row r's probabilities come from lanes of this wave
+            if (part_active) {
+#pragma unroll 4
+                for (int jj = 0; jj < 32; ++jj) {
+                    const float w = probs[r * 33 + jj];
+                    float vd[16];
+                    widen_bf16(*reinterpret_cast<const uint4*>(&v_tile[jj * FS + 16 * part]), vd);
+                    widen_bf16(*reinterpret_cast<const uint4*>(&v_tile[jj * FS + 16 * part + 8]), vd + 8);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[i] = fmaf(w, vd[i], acc[i]);
+                }
+            }
+        }
+    }
+
+    // 4. Output.
+    if (valid && part_active) {
+        uint32_t w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = bf16_rn(acc[2 * i] / l) | (bf16_rn(acc[2 * i + 1] / l) << 16);
+        uint16_t* out = p.output + row * p.output_stride + channels;
+        if (aligned_rows(p.output, p.output_stride)) {
+            reinterpret_cast<uint4*>(out)[0] = make_uint4(w[0], w[1], w[2], w[3]);
+            reinterpret_cast<uint4*>(out)[1] = make_uint4(w[4], w[5], w[6], w[7]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                out[2 * i] = (uint16_t)(w[i] & 0xffffu);
+                out[2 * i + 1] = (uint16_t)(w[i] >> 16);
+            }
+        }
+    }
+}
+
+// One request's rows and history.
+struct RequestRows {
+    int first, rows, history;
+};
+
+__device__ __forceinline__ RequestRows request_rows(const MultiRowParams& p, int request) {
+    RequestRows r;
+    r.first = p.query_start_loc[request];
+    const int n = p.query_start_loc[request + 1] - r.first;
+    const int new_tokens = p.causal ? n : 1;
+    // Rows past the query tensor are not read or written.
+    r.rows = r.first < 0 || r.first >= p.rows ? 0 : (int)min((int64_t)max(n, 0), p.rows - r.first);
+    const int seq = p.seq_lens[request];
+    // Tokens past the page table are never read.
+    r.history = (int)min((int64_t)(seq > new_tokens ? seq - new_tokens : 0), p.max_pages * p.page_tokens);
+    return r;
+}
+
+// Item `key` of the call's plan, or, with more requests than the plan covers,
+// split `split` of the call's `splits` of row tile `tile` of `request`.
+// PlanItem: length in 32-token tiles, tokens the history.
+__device__ __forceinline__ PlanItem multirow_plan(const MultiRowParams& p, int key, int request, int tile, int split) {
+    if (p.items > 0) {
+        const int requests = (int)p.requests;
+        const int b = threadIdx.x & 63;
+        const RequestRows q = request_rows(p, b < requests ? b : requests - 1);
+        const int rows = b < requests ? q.rows : 0;
+        return plan_find(
+            requests, key, PlanSizes{p.plan_target, p.splits, p.plan_min, p.plan_max, p.plan_max_splits, 0, 1},
+            PlanEntry{(rows + p.tile_rows - 1) / p.tile_rows, (q.history + kTile - 1) / kTile, q.first, q.history,
+                      rows});
+    }
+    const RequestRows q = request_rows(p, request);
+    // About requests x the average request's row tiles x splits of the items have work.
+    const int64_t tiles = max(p.rows / (p.requests * p.tile_rows), (int64_t)1);
+    return PlanItem{request, tile, split, p.splits, (q.history + kTile - 1) / kTile, q.first, q.history, q.rows, 0,
+                    q.first * p.splits, (int)min(p.requests * tiles * p.splits, (int64_t)INT_MAX)};
+}
+
+// The head of a stream workgroup (stream_grid).
+__device__ __forceinline__ int stream_head(const MultiRowParams& p) {
+    return p.items > 0 ? (int)(blockIdx.x % (unsigned)p.heads) : (int)blockIdx.y;
+}
+
 template <int D, int PT, int TR, class Decoder>
 __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder& dec, uint8_t* lds,
                                                 int* split_blocks) {
     using G = Geometry<D, TR>;
     constexpr int KS = G::KS;
     constexpr int QRS = G::QRS;
-    const int request = blockIdx.x;
-    const int head = blockIdx.y;
-    const int split = (int)blockIdx.z % p.splits;
-    const int row0 = TR * ((int)blockIdx.z / p.splits);
-    const int first = p.query_start_loc[request];
-    int n = p.query_start_loc[request + 1] - first;
-    if (first < 0 || first >= p.rows) return;  // uniform over the workgroup, before any barrier
-    const int new_tokens = p.causal ? n : 1;
-    if (n > p.rows - first) n = (int)(p.rows - first);  // rows past the query tensor are not read or written
-    if (row0 >= n) return;
-    const int seq = p.seq_lens[request];
-    int history = seq > new_tokens ? seq - new_tokens : 0;
-    // Tokens past the page table are never read.
-    if ((int64_t)history > p.max_pages * PT) history = (int)(p.max_pages * PT);
-    const int tiles = (history + kTile - 1) / kTile;
-    const int per_split = (tiles + p.splits - 1) / p.splits;
-    const int tile_begin = split * per_split;
-    const int tile_end = tile_begin + per_split < tiles ? tile_begin + per_split : tiles;
+    const int head = stream_head(p);
+    const PlanItem item = multirow_plan(p, (int)(blockIdx.x / (unsigned)p.heads), blockIdx.x,
+                                               (int)blockIdx.z / p.splits, (int)blockIdx.z % p.splits);
+    const int request = __builtin_amdgcn_readfirstlane(item.request);
+    const int first = __builtin_amdgcn_readfirstlane(item.first), n = __builtin_amdgcn_readfirstlane(item.rows);
+    const int row0 = TR * __builtin_amdgcn_readfirstlane(item.index);
+    if (request < 0 || row0 >= n) return;  // uniform over the workgroup, before any barrier
+    const int split = item.split;
+    const int history = __builtin_amdgcn_readfirstlane(item.tokens);
+    const int tile_begin = __builtin_amdgcn_readfirstlane(split_begin(item.length, split, item.splits));
+    const int tile_end = __builtin_amdgcn_readfirstlane(split_begin(item.length, split + 1, item.splits));
+
+    // The row tile's arrival word lies in the two unused floats of its first
+    // row's entry of split 0.
+    float* tile_entries = p.partials + ((int64_t)head * p.entries + item.entry + row0 * item.splits) * kMultiRowEntry;
+    uint64_t* arrivals = reinterpret_cast<uint64_t*>(tile_entries + 2);
+    const uint64_t arrivals_seen = item.splits > 1 ? peek_arrivals(arrivals) : 0;
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // provably wave-uniform
@@ -502,6 +899,7 @@ __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder
         }
     }
     __syncthreads();
+    if (item.splits > 1 && tid == 0) tag_arrivals(arrivals, p.call_tag, arrivals_seen);
     if (p.key_rotation && wave < G::Quarters) {
         // q.R_k on the matrix cores: wave w takes columns 32 w .. 32 w + 31.
         // A: lane l reads scaled row l % 32 at k = 16 m + 8 (l / 32) .. + 7.
@@ -626,8 +1024,7 @@ __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder
         q_operand[m] = *reinterpret_cast<const F16x8*>(&q_p[tile_row * KS + (TR == 32 ? 16 : 32) * m + 8 * k_group]);
     const float q_mu_anchor = q_mu[tile_row];
     const float row_scale = q_scale[tile_row];
-    if (split == 0 && tid < TR && row0 + tid < n)
-        p.row_shift[(int64_t)(first + row0 + tid) * p.heads + head] = q_mu[32 + tid];
+    const float row_shift = q_mu[32 + (tid >> 3)];  // q'.mu_L of the finish thread's row
     __syncthreads();  // the scratch becomes the tiles
 
     // ---------------------------------------------------------------- history
@@ -707,7 +1104,7 @@ __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder
     // priority over each tile's MFMAs and softmax (residual call 129.3 ->
     // 122.5 us at 16 requests x 16 rows x 8k, A/B on one box).
     const int wave_tiles = first_tile < tile_end ? (tile_end - first_tile + kWaves - 1) / kWaves : 0;
-    const StreamPriority priority(wave_tiles, p.stream_priority != 0);
+    const StreamPriority priority(wave_tiles, (int64_t)item.total * p.heads <= p.resident);
     int step = 0;
     for (int tile = first_tile; tile < tile_end; tile += kWaves, ++step) {
         priority.set(step);
@@ -942,19 +1339,21 @@ __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder
         merge_ml[(wave * 32 + tile_row) * 2 + 1] = running_sum;
     }
     __syncthreads();
+    FinishInputs<D> in;
+    finish_load<D, TR>(p, head, first, row0, n, in);
     const int r = tid >> 3, chunk = tid & 7;  // row, 16-channel chunk
+    const bool chunk_active = chunk < G::Parts;
+    const bool valid = r < TR && row0 + r < n;
+    float total_max = -__builtin_inff(), l = 0.f, o[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) o[c] = 0.f;
     if (r < TR) {
-        float m_w[kWaves], total_max = -__builtin_inff();
+        float m_w[kWaves];
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
             m_w[w] = merge_ml[(w * 32 + r) * 2];
             total_max = fmaxf(total_max, m_w[w]);
         }
-        float l = 0.f;
-        float o[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c) o[c] = 0.f;
-        const bool chunk_active = chunk < G::Parts;
 #pragma unroll
         for (int w = 0; w < kWaves; ++w) {
             if (m_w[w] == -__builtin_inff()) continue;
@@ -964,17 +1363,30 @@ __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder
 #pragma unroll
             for (int c = 0; c < 16; ++c) o[c] = fmaf(src[c], weight, o[c]);
         }
-        if (row0 + r < n) {
-            float* entry = p.partials +
-                           (((int64_t)(first + row0 + r) * p.heads + head) * p.splits + split) * kMultiRowEntry;
-            if (chunk == 0) *reinterpret_cast<float4*>(entry) = make_float4(total_max, l, 0.f, 0.f);
-            if (chunk_active) {
-                float4* dst = reinterpret_cast<float4*>(entry + 4 + 16 * chunk);
-#pragma unroll
-                for (int c = 0; c < 4; ++c) dst[c] = make_float4(o[4 * c], o[4 * c + 1], o[4 * c + 2], o[4 * c + 3]);
-            }
-        }
     }
+    if (item.splits > 1) {
+        // One resource over the tile's entries (wave-uniform); the row is a lane offset.
+        const int tile_rows = n - row0 < TR ? n - row0 : TR;
+        const __amdgpu_buffer_rsrc_t entries =
+            handoff_resource(tile_entries, (uint32_t)(tile_rows * item.splits * kMultiRowEntry * 4));
+        const uint32_t row_at = (uint32_t)((valid ? r : 0) * item.splits * kMultiRowEntry * 4);
+        const uint32_t at = row_at + (uint32_t)(split * kMultiRowEntry * 4);
+        if (valid && chunk == 0) {
+            handoff_store(entries, at, total_max);
+            handoff_store(entries, at + 4, l);
+        }
+        if (valid && chunk_active) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                handoff_store4(entries, at + 16 + 64 * chunk + 16 * c, o[4 * c], o[4 * c + 1], o[4 * c + 2],
+                               o[4 * c + 3]);
+        }
+        // (The flag aliases the merge buffer, which every thread has read by then.)
+        if (!arrive_last_tagged(arrivals, item.splits, reinterpret_cast<int*>(lds))) return;
+        finish_merge(entries, row_at, item.splits, valid, chunk_active ? chunk : 0, total_max, l, o);
+    }
+    __syncthreads();  // the finish's tiles alias the merge buffer
+    finish_rows<D, TR>(p, head, first, row0, n, in, row_shift, total_max, l, o, lds);
 }
 
 template <int D, int PT, int TR, bool HasL, int BA, int GA, int BL, int GL>
@@ -997,7 +1409,7 @@ void multirow_chain_kernel(MultiRowParams p) {
     __shared__ int split_blocks[kMaxSplitPages];  // block ids of the split's pages
     // bf16(mu_r) of records 0 .. L - 1 (the K plane's chain), FP32.
     __shared__ __attribute__((aligned(16))) float mean_lds[Links - 1][kMaxD];
-    const int head = blockIdx.y;
+    const int head = stream_head(p);
     const bool has_mean = p.key_mean_all != nullptr;
     for (int i = threadIdx.x; i < (Links - 1) * kMaxD; i += kThreads) {
         const int r = i / kMaxD, c = i % kMaxD;
@@ -1020,367 +1432,22 @@ void multirow_chain_kernel(MultiRowParams p) {
     multirow_stream<D, PT, TR>(p, dec, lds, split_blocks);
 }
 
-// ---------------------------------------------------------------- finish
-
-// Row strides of the finish kernel's tiles for head dim D: BF16/FP16 rows
-// (halves) and the rotated history [row][channel] (FP32).  Region A holds
-// the merged rows' FP16 parts for the rotation, then the causal tiles;
-// region B the rotated history.
-template <int D>
-struct FinishGeometry {
-    static constexpr int Parts = D / 16;
-    static constexpr int FS = D + 8;
-    static constexpr int OS = D + 4;
-    static constexpr int kRotationBytes = 2 * 32 * FS * 2;                  // high and low FP16 parts
-    static constexpr int kCausalBytes = 3 * 32 * FS * 2 + 32 * 33 * 4;     // q, k, v tiles and probabilities
-    static constexpr int kRegionABytes = kRotationBytes > kCausalBytes ? kRotationBytes : kCausalBytes;
-    static constexpr int kRegionBFloats = 32 * OS;
-};
-
-__device__ __forceinline__ float row8_max(float x) {
-    x = fmaxf(x, __shfl_xor(x, 1));
-    x = fmaxf(x, __shfl_xor(x, 2));
-    return fmaxf(x, __shfl_xor(x, 4));
-}
-
-__device__ __forceinline__ float row8_sum(float x) {
-    x += __shfl_xor(x, 1);
-    x += __shfl_xor(x, 2);
-    return x + __shfl_xor(x, 4);
-}
-
-// Whether rows of a BF16 tensor at `base` with row stride `stride`
-// (elements) start on 16-byte boundaries.  The boundary guarantees 8 bytes
-// for queries and keys and 2 bytes for values and outputs.
-__device__ __forceinline__ bool aligned_rows(const void* base, int64_t stride) {
-    return (reinterpret_cast<uintptr_t>(base) & 15u) == 0 && (stride & 7) == 0;
-}
-
-// 16 consecutive BF16 values at `src` (a 32-byte aligned offset of an
-// aligned_rows tensor when `vec`) as two 16-byte words.
-__device__ __forceinline__ void load_halves16(const uint16_t* src, bool vec, uint4 (&w)[2]) {
-    if (vec) {
-        w[0] = reinterpret_cast<const uint4*>(src)[0];
-        w[1] = reinterpret_cast<const uint4*>(src)[1];
-    } else {
-        uint32_t x[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = (uint32_t)src[2 * i] | ((uint32_t)src[2 * i + 1] << 16);
-        w[0] = make_uint4(x[0], x[1], x[2], x[3]);
-        w[1] = make_uint4(x[4], x[5], x[6], x[7]);
-    }
-}
-
-// Eight BF16 values of a 16-byte word as FP32.
-__device__ __forceinline__ void widen_bf16(uint4 w, float* x) {
-    const uint32_t v[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        x[2 * i] = bf16_f32(v[i] & 0xffffu);
-        x[2 * i + 1] = bf16_f32(v[i] >> 16);
-    }
-}
-
-// One (request, head, 32-row tile) per 256-thread workgroup.  Thread t takes
-// row t / 8 of the tile and part p = t % 8 of it: the 16 channels
-// 16p..16p+15 of the merge, the query-key dots, the live values and the
-// output (parts p < D / 16), and the 4 tokens 4p..4p+3 of a live chunk's
-// scores.  The eight threads of a row are adjacent lanes of one wave.
-//   1. merge the splits' partials (m, l, O) of each row (log2 units);
-//   2. rotate the tile's 32 merged rows by R_v^T on the matrix cores (wave w
-//      computes output channels 32 w .. 32 w + 31);
-//   3. add the live tokens: in decode semantics the row's own token; in
-//      causal semantics the request's new tokens j <= row, 32 at a time with
-//      an online softmax over the rows' (m, l, O);
-//   4. write O / l in BF16.
-template <int D>
-__global__ __launch_bounds__(kThreads) void multirow_finish_kernel(MultiRowParams p) {
-    using G = FinishGeometry<D>;
-    constexpr int FS = G::FS;
-    constexpr int OS = G::OS;
-    __shared__ __attribute__((aligned(16))) uint8_t region_a[G::kRegionABytes];
-    __shared__ __attribute__((aligned(16))) float region_b[G::kRegionBFloats];
-    float* hist_rot = region_b;
-    uint16_t* q_tile = reinterpret_cast<uint16_t*>(region_a);  // causal: the rows' queries
-    uint16_t* k_tile = q_tile + 32 * FS;                      // causal: 32 live keys
-    uint16_t* v_tile = k_tile + 32 * FS;                      // causal: their values
-    float* probs = reinterpret_cast<float*>(v_tile + 32 * FS);
-    const int request = blockIdx.x;
-    const int head = blockIdx.y;
-    const int row0 = 32 * (int)blockIdx.z;
-    const int tid = threadIdx.x;
-    const int r = tid >> 3, part = tid & 7;
-    const bool part_active = part < G::Parts;
-    const bool rotate = p.value_rotation != nullptr;
-    const int wave = tid >> 6;
-    const bool rotation_wave = wave < D / 32;
-
-    // R_v as the B operand of the rotation MFMAs (16-byte loads issued
-    // before the request lookup, so that the two round trips overlap): wave
-    // w computes output channels 32 w .. 32 w + 31, lane l takes row
-    // 32 w + l % 32 of R_v at features 16 m + 8 (l / 32) .. + 7.
-    const int lane = tid & 63;
-    F16x8 rv[G::Parts];
-    if (rotate && rotation_wave) {
-        const uint16_t* src = p.value_rotation + ((int64_t)head * D + 32 * wave + (lane & 31)) * D + 8 * (lane >> 5);
-#pragma unroll
-        for (int m = 0; m < G::Parts; ++m) rv[m] = *reinterpret_cast<const F16x8*>(src + 16 * m);
-    }
-    const int first = p.query_start_loc[request];
-    int n = p.query_start_loc[request + 1] - first;
-    if (first < 0 || first >= p.rows) return;  // uniform over the workgroup, before any barrier
-    if (n > p.rows - first) n = (int)(p.rows - first);
-    if (row0 >= n) return;
-
-    const bool valid = row0 + r < n;
-    const int64_t row = (int64_t)first + row0 + (valid ? r : 0);
-    const float scale = Geometry<D>::kScoreScale;  // log2(e) / sqrt(D)
-    // The part's 16 channels of a token row (part 0's for an inactive part,
-    // whose values are never used).
-    const int64_t channels = (int64_t)head * D + 16 * (part_active ? part : 0);
-
-    // The row's query (and, in decode semantics, its own key and value).
-    const bool q_vec = aligned_rows(p.query, p.query_stride), k_vec = aligned_rows(p.key, p.key_stride),
-               v_vec = aligned_rows(p.value, p.value_stride);
-    uint4 qw[2], kw[2], vw[2];
-    load_halves16(p.query + row * p.query_stride + channels, q_vec, qw);
-    if (!part_active) qw[0] = qw[1] = make_uint4(0u, 0u, 0u, 0u);  // no share of the row's dots
-    if (!p.causal) {
-        load_halves16(p.key + row * p.key_stride + channels, k_vec, kw);
-        load_halves16(p.value + row * p.value_stride + channels, v_vec, vw);
-    }
-    const float shift = p.row_shift[row * p.heads + head];
-
-    // 1. Merge the splits online, four at a time: every load of a batch is
-    // issued before any of its arithmetic (split indices past the last are
-    // clamped and weighted zero, so no load sits behind a branch).  Rows past
-    // the request merge nothing.
-    float m = -__builtin_inff(), l = 0.f, acc[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    const float* entries = p.partials + (row * p.heads + head) * p.splits * kMultiRowEntry;
-    const int entry_part = part_active ? part : 0;
-    for (int s0 = 0; s0 < p.splits; s0 += 4) {
-        float2 ml[4];
-        float4 ox[4][4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int s = s0 + b < p.splits ? s0 + b : p.splits - 1;
-            const float* e = entries + s * kMultiRowEntry;
-            ml[b] = *reinterpret_cast<const float2*>(e);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) ox[b][c] = reinterpret_cast<const float4*>(e + 4 + 16 * entry_part)[c];
-        }
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const float ms = (valid && s0 + b < p.splits) ? ml[b].x : -__builtin_inff();
-            const float new_max = fmaxf(m, ms);
-            const float base = new_max == -__builtin_inff() ? 0.f : new_max;
-            const float keep = __builtin_amdgcn_exp2f(m - base), w = __builtin_amdgcn_exp2f(ms - base);
-            m = new_max;
-            l = fmaf(l, keep, ml[b].y * w);
-            const float x[16] = {ox[b][0].x, ox[b][0].y, ox[b][0].z, ox[b][0].w, ox[b][1].x, ox[b][1].y,
-                                 ox[b][1].z, ox[b][1].w, ox[b][2].x, ox[b][2].y, ox[b][2].z, ox[b][2].w,
-                                 ox[b][3].x, ox[b][3].y, ox[b][3].z, ox[b][3].w};
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] = fmaf(acc[i], keep, x[i] * w);
-        }
-    }
-
-    // 2. hist . R_v^T for the tile's 32 rows on the matrix cores: the merged
-    // rows divided by their sums (convex combinations of values, within the
-    // FP16 range) as FP16 high and low parts (~22 significant bits), times
-    // R_v (FP16), FP32 accumulation; the sums are multiplied back.
-    if (rotate) {
-        uint16_t* high = reinterpret_cast<uint16_t*>(region_a);  // [row][FS]
-        uint16_t* low = high + 32 * FS;
-        const float inverse = l > 0.f ? 1.0f / l : 0.f;
-        uint32_t hw[8], lw[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float x0 = acc[2 * i] * inverse, x1 = acc[2 * i + 1] * inverse;
-            const _Float16 h0 = (_Float16)x0, h1 = (_Float16)x1;
-            const _Float16 r0 = (_Float16)(x0 - (float)h0), r1 = (_Float16)(x1 - (float)h1);
-            hw[i] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-            lw[i] = (uint32_t)__builtin_bit_cast(uint16_t, r0) | ((uint32_t)__builtin_bit_cast(uint16_t, r1) << 16);
-        }
-        if (part_active) {
-            uint4* hd = reinterpret_cast<uint4*>(&high[r * FS + 16 * part]);
-            uint4* ld = reinterpret_cast<uint4*>(&low[r * FS + 16 * part]);
-            hd[0] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-            hd[1] = make_uint4(hw[4], hw[5], hw[6], hw[7]);
-            ld[0] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-            ld[1] = make_uint4(lw[4], lw[5], lw[6], lw[7]);
-        }
-        __syncthreads();
-        if (rotation_wave) {
-            // A operand: lane l takes merged row l % 32 at features 16 m + 8 (l / 32) .. + 7.
-            F32x16 rotated;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) rotated[e] = 0.f;
-            const int a_offset = (lane & 31) * FS + 8 * (lane >> 5);
-#pragma unroll
-            for (int mm = 0; mm < G::Parts; ++mm) {
-                rotated = mfma(*reinterpret_cast<const F16x8*>(&high[a_offset + 16 * mm]), rv[mm], rotated);
-                rotated = mfma(*reinterpret_cast<const F16x8*>(&low[a_offset + 16 * mm]), rv[mm], rotated);
-            }
-            // Register e of lane l: row 8 (e / 4) + 4 (l / 32) + e % 4, channel 32 w + l % 32.
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                hist_rot[(8 * (e >> 2) + 4 * (lane >> 5) + (e & 3)) * OS + 32 * wave + (lane & 31)] = rotated[e];
-        }
-        __syncthreads();
-        if (part_active) {
-#pragma unroll
-            for (int c4 = 0; c4 < 4; ++c4) {
-                const float4 x = *reinterpret_cast<const float4*>(&hist_rot[r * OS + 16 * part + 4 * c4]);
-                acc[4 * c4] = x.x * l;
-                acc[4 * c4 + 1] = x.y * l;
-                acc[4 * c4 + 2] = x.z * l;
-                acc[4 * c4 + 3] = x.w * l;
-            }
-        }
-    }
-
-    // 3. Live tokens.
-    float q[16];
-    widen_bf16(qw[0], q);
-    widen_bf16(qw[1], q + 8);
-    if (!p.causal) {
-        // The row's own token.
-        float k[16], v[16];
-        widen_bf16(kw[0], k);
-        widen_bf16(kw[1], k + 8);
-        widen_bf16(vw[0], v);
-        widen_bf16(vw[1], v + 8);
-        float dot = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dot = fmaf(q[i], k[i], dot);
-        const float score = row8_sum(dot) * scale - shift;
-        const float total_max = fmaxf(m, score);
-        const float hist_weight = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - total_max);
-        const float live = __builtin_amdgcn_exp2f(score - total_max);
-        l = fmaf(l, hist_weight, live);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = fmaf(live, v[i], acc[i] * hist_weight);
-    } else {
-        // The request's new tokens 0 .. row0 + r, in chunks of 32 shared by the tile's rows.
-        if (part_active) {
-            uint4* dst = reinterpret_cast<uint4*>(&q_tile[r * FS + 16 * part]);
-            dst[0] = qw[0];
-            dst[1] = qw[1];
-        }
-        const int live_end = n < row0 + 32 ? n : row0 + 32;
-        for (int c0 = 0; c0 < live_end; c0 += 32) {
-            __syncthreads();  // the previous chunk's reads are done
-            if (part_active) {
-                // Thread (r, part) stages the part's channels of live token c0 + r.
-                const int j = c0 + r;
-                uint4 kx[2] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)}, vx[2] = {kx[0], kx[1]};
-                if (j < n) {
-                    load_halves16(p.key + ((int64_t)first + j) * p.key_stride + channels, k_vec, kx);
-                    load_halves16(p.value + ((int64_t)first + j) * p.value_stride + channels, v_vec, vx);
-                }
-                uint4* kd = reinterpret_cast<uint4*>(&k_tile[r * FS + 16 * part]);
-                uint4* vd = reinterpret_cast<uint4*>(&v_tile[r * FS + 16 * part]);
-                kd[0] = kx[0];
-                kd[1] = kx[1];
-                vd[0] = vx[0];
-                vd[1] = vx[1];
-            }
-            __syncthreads();
-            // Scores of row r against tokens c0 + 4 part .. + 3.
-            float s[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-            for (int d = 0; d < D; d += 8) {
-                float qd[8];
-                widen_bf16(*reinterpret_cast<const uint4*>(&q_tile[r * FS + d]), qd);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float kd[8];
-                    widen_bf16(*reinterpret_cast<const uint4*>(&k_tile[(4 * part + i) * FS + d]), kd);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) s[i] = fmaf(qd[e], kd[e], s[i]);
-                }
-            }
-            float chunk_max = -__builtin_inff();
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int j = c0 + 4 * part + i;
-                s[i] = (valid && j <= row0 + r && j < n) ? s[i] * scale - shift : -__builtin_inff();
-                chunk_max = fmaxf(chunk_max, s[i]);
-            }
-            const float new_max = fmaxf(m, row8_max(chunk_max));
-            const float base = new_max == -__builtin_inff() ? 0.f : new_max;
-            const float rescale = __builtin_amdgcn_exp2f(m - base);
-            m = new_max;
-            float chunk_sum = 0.f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float w = __builtin_amdgcn_exp2f(s[i] - base);
-                probs[r * 33 + 4 * part + i] = w;
-                chunk_sum += w;
-            }
-            l = fmaf(l, rescale, row8_sum(chunk_sum));
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] *= rescale;
-            wave_sync();  // row r's probabilities come from lanes of this wave
-            if (part_active) {
-#pragma unroll 4
-                for (int jj = 0; jj < 32; ++jj) {
-                    const float w = probs[r * 33 + jj];
-                    float vd[16];
-                    widen_bf16(*reinterpret_cast<const uint4*>(&v_tile[jj * FS + 16 * part]), vd);
-                    widen_bf16(*reinterpret_cast<const uint4*>(&v_tile[jj * FS + 16 * part + 8]), vd + 8);
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[i] = fmaf(w, vd[i], acc[i]);
-                }
-            }
-        }
-    }
-
-    // 4. Output.
-    if (valid && part_active) {
-        uint32_t w[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) w[i] = bf16_rn(acc[2 * i] / l) | (bf16_rn(acc[2 * i + 1] / l) << 16);
-        uint16_t* out = p.output + row * p.output_stride + channels;
-        if (aligned_rows(p.output, p.output_stride)) {
-            reinterpret_cast<uint4*>(out)[0] = make_uint4(w[0], w[1], w[2], w[3]);
-            reinterpret_cast<uint4*>(out)[1] = make_uint4(w[4], w[5], w[6], w[7]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                out[2 * i] = (uint16_t)(w[i] & 0xffffu);
-                out[2 * i + 1] = (uint16_t)(w[i] >> 16);
-            }
-        }
-    }
-}
-
-// Rows per stream tile: 16 when the call's requests average 16 rows or
-// fewer (and the grid's z extent allows it), else 32.  The finish kernel
-// always takes 32-row tiles (the partials are per row).
-int stream_tile_rows(const MultiRowParams& p) {
-    const int64_t tiles16 = (p.rows + 15) / 16;
-    return (p.rows <= 16 * p.requests && (int64_t)p.splits * tiles16 <= 65535) ? 16 : 32;
-}
-
 template <int TR>
 dim3 stream_grid(const MultiRowParams& p) {
+    // Planned items head by head, so that the workgroups past the plan come
+    // last: one that waits for a compute unit's LDS before it can exit holds
+    // back every workgroup behind it (24 requests x 16 rows x 4096 tokens,
+    // half of the workgroups past the plan: 146 us per residual call with
+    // them in between, 121 us without).
+    if (p.items > 0) return dim3((unsigned)((int64_t)p.items * p.heads));
     return dim3((unsigned)p.requests, (unsigned)p.heads, (unsigned)(p.splits * ((p.rows + TR - 1) / TR)));
 }
 
-// The launch parameters with stream_priority set: whether the grid's active
-// workgroups, about requests x heads x splits x the average request's row
-// tiles (the others exit at once), fit the device at once.
-template <int TR>
-MultiRowParams with_priority(const MultiRowParams& params, int per_cu) {
+// The launch parameters with `resident` set: the stream workgroups that the
+// device holds at once.
+MultiRowParams with_resident(const MultiRowParams& params, int per_cu) {
     MultiRowParams p = params;
-    const int64_t average_rows = p.requests > 0 ? p.rows / p.requests : p.rows;
-    const int64_t average_tiles = average_rows > TR ? (average_rows + TR - 1) / TR : 1;
-    const int64_t active = p.requests * p.heads * p.splits * average_tiles;
-    p.stream_priority = active <= (int64_t)per_cu * p.compute_units ? 1 : 0;
+    p.resident = (int64_t)per_cu * p.compute_units;
     return p;
 }
 
@@ -1388,14 +1455,14 @@ template <int D, int PT, int TR, bool HasL, int BA, int GA, int BL, int GL>
 void launch_one(const MultiRowParams& p, hipStream_t stream) {
     const auto kernel = multirow_stream_kernel<D, PT, TR, HasL, BA, GA, BL, GL>;
     static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kThreads);
-    hipLaunchKernelGGL(kernel, stream_grid<TR>(p), dim3(kThreads), 0, stream, with_priority<TR>(p, per_cu));
+    hipLaunchKernelGGL(kernel, stream_grid<TR>(p), dim3(kThreads), 0, stream, with_resident(p, per_cu));
 }
 
 template <int D, int PT, int TR, int Links>
 void launch_chain(const MultiRowParams& p, hipStream_t stream) {
     const auto kernel = multirow_chain_kernel<D, PT, TR, Links>;
     static const int per_cu = resident_per_cu(reinterpret_cast<const void*>(kernel), kThreads);
-    hipLaunchKernelGGL(kernel, stream_grid<TR>(p), dim3(kThreads), 0, stream, with_priority<TR>(p, per_cu));
+    hipLaunchKernelGGL(kernel, stream_grid<TR>(p), dim3(kThreads), 0, stream, with_resident(p, per_cu));
 }
 
 template <int D, int PT, int TR, int BA, int GA, int BL>
@@ -1443,7 +1510,7 @@ bool launch_tr(const MultiRowParams& p, hipStream_t stream) {
 
 template <int D, int PT>
 bool launch_pt(const MultiRowParams& p, hipStream_t stream) {
-    return stream_tile_rows(p) == 16 ? launch_tr<D, PT, 16>(p, stream) : launch_tr<D, PT, 32>(p, stream);
+    return p.tile_rows == 16 ? launch_tr<D, PT, 16>(p, stream) : launch_tr<D, PT, 32>(p, stream);
 }
 
 template <int D>
@@ -1453,10 +1520,7 @@ bool launch_d(const MultiRowParams& p, hipStream_t stream) {
         launched = launch_pt<D, 16>(p, stream);
     else if (p.page_tokens == 32)
         launched = launch_pt<D, 32>(p, stream);
-    if (!launched) return false;
-    hipLaunchKernelGGL(multirow_finish_kernel<D>, dim3((unsigned)p.requests, (unsigned)p.heads, (unsigned)p.row_tiles),
-                       dim3(kThreads), 0, stream, p);
-    return true;
+    return launched;
 }
 
 }  // namespace

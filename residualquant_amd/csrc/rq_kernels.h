@@ -178,10 +178,12 @@ struct AttentionParams {
     uint64_t* arrivals;    // packed decode: workspace [rows, heads], tagged arrival counts (rq_plan.h)
     uint64_t call_tag;     // of this call (56 bits)
     float* partials;       // workspace: packed decode [heads, items, D + 2], BF16 [rows, heads, splits, D + 2]
-    int splits;            // BF16 baseline, and packed decode past kPlanRequests requests: splits of every row
-    int items;             // packed decode: workgroups per head
-    int plan_target;       // packed decode: workgroups per head that the plan spreads the work over
-    int plan_min_pages;    // and the least pages of one split
+    int splits;            // of every row: BF16 baseline, packed decode of equal lengths or past kPlanRequests
+    // Packed decode (decode_item in attention.hip):
+    int plan_min_pages;    // least pages of one split
+    int plan_target;       // workgroups per head that the plan spreads the work over
+    int plan_round_pages, plan_round_target;  // PlanSizes
+    int items;             // set by the launch: workgroups per head
     int compute_units;     // of the launching device
     int64_t resident;      // set by the launch: workgroups the device holds at once
     // Adjacent mode, loop L > 0: records 0..L of the restore chain (chain_length = L + 1, else 0)
@@ -195,14 +197,14 @@ hipError_t launch_attention(const AttentionParams& p, hipStream_t stream, hipEve
                             hipEvent_t end);
 
 // Several query rows per request over packed pages (D = 96 or 128, anchor
-// and adjacent mode): one workgroup per (request, head, row tile of 32 rows,
-// history split) streams the split's pages once for all the tile's rows on
-// MFMA tiles, then a finish launch per (row, head) merges the splits,
-// applies R_v^T and adds the live tokens.  causal = 0: the reference decode
+// and adjacent mode): one workgroup per (request, head, row tile of 16 or 32
+// rows, history split) streams the split's pages once for all the tile's rows on
+// MFMA tiles; the last split of a tile merges the splits, applies R_v^T and
+// adds the live tokens.  causal = 0: the reference decode
 // semantics (history seq_len - 1, the row's own live token); causal = 1: the
 // rows are the request's last n tokens (history seq_len - n, live tokens
 // j <= r).
-constexpr int kMultiRowEntry = 132;        // per (row, head, split): m, l, 2 unused, O[D <= 128] (log2 units)
+constexpr int kMultiRowEntry = 132;        // per (row, head, split): m, l, arrival word, O[D <= 128] (log2 units)
 constexpr int kMultiRowMaxSplits = 8;      // for parallelism (more only for very long histories)
 constexpr int kMultiRowMaxSplitPages = 1024;  // pages of one split at most
 struct MultiRowParams {
@@ -242,13 +244,19 @@ struct MultiRowParams {
     RecordRegion chain[kMaxRecords];
     const float* key_mean_all;
     int causal;
-    int splits;     // history splits per (request, head, row tile)
+    // Up to kPlanRequests requests, the history splits are planned on the
+    // device (rq_plan.h, multirow_plan): `items` stream workgroups per head,
+    // `splits` per (request, head, row tile) of equal lengths.  With more
+    // requests (items 0) every (request, head, row tile) takes `splits`.
+    int items;
+    int splits;
+    int plan_target, plan_min, plan_max, plan_max_splits;  // PlanSizes, in 32-token tiles
+    int tile_rows;        // rows of a stream tile: 16 or 32
     int compute_units;    // of the launching device
-    int stream_priority;  // set by the launch: the active workgroups fit the device at once, so their
-                          // waves take StreamPriority
-    int row_tiles;  // 32-row tiles per request in the finish grid (the stream grid takes 16 or 32 rows a tile)
-    float* partials;   // workspace [rows, heads, splits, kMultiRowEntry]
-    float* row_shift;  // workspace [rows, heads]: q'.mu_L in log2 units
+    int64_t resident;     // set by the launch: stream workgroups the device holds at once
+    int64_t entries;      // partials per head
+    float* partials;      // workspace [heads, entries, kMultiRowEntry]; a request's entries: [row, split]
+    uint64_t call_tag;    // of this call (56 bits, rq_plan.h)
 };
 hipError_t launch_multirow(const MultiRowParams& p, hipStream_t stream);
 hipError_t launch_attention_bf16(const AttentionParams& p, hipStream_t stream, hipEvent_t begin,

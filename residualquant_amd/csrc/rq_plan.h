@@ -8,32 +8,34 @@
 // the full batch; with the plan it takes 53 us, and the full batch, whose
 // equal lengths stay unsplit, 161 us as before.  Every wave derives the same plan from the lengths: a chunk size
 // that spreads the batch's total work over `target` workgroups per head, and
-// ceil(length / chunk) near-equal splits per request.  The plan takes two
-// DPP scans and no LDS or barrier (about 0.2 us once the lengths have
-// arrived); workgroups past the planned items exit.
+// ceil(length / chunk) near-equal splits per request.  The plan takes a few
+// DPP scans and no LDS or barrier (about 0.2 us for near-equal requests, 0.7
+// us else, once the lengths have arrived); workgroups past the planned items
+// exit.
 #pragma once
 
 #include "rq_device.h"
 
 namespace rq {
 
-// Requests the plan covers (64 per register set); calls with more requests
-// take the host's split count for every request.
-constexpr int kPlanChunks = 4;
-constexpr int kPlanRequests = 64 * kPlanChunks;
+// Requests the plan covers, one per lane; calls with more requests take the
+// host's split count for every request.
+constexpr int kPlanRequests = 64;
 
 // One request's share: `count` items (rows, or row tiles) of `length` units
-// each; `first` and `tokens` are carried to the item that is found.
+// each, `rows` rows in all; `first` and `tokens` are carried to the item that
+// is found.
 struct PlanEntry {
-    int count, length, first, tokens;
+    int count, length, first, tokens, rows;
 };
 
 struct PlanItem {
     int request;  // -1: no work for this item
     int index;    // which of the request's `count` items
     int split, splits;
-    int length, first, tokens;
+    int length, first, tokens, rows;
     int offset;   // item index of split 0 of this (request, index)
+    int entry;    // rows x splits of the requests before this one
     int total;    // items of the whole plan
 };
 
@@ -63,75 +65,87 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t x, int lane) {
     return x + (lane >= 16 ? t0 : 0u) + (lane >= 32 ? t1 : 0u) + (lane >= 48 ? t2 : 0u);
 }
 
-// Item `item` of the plan over `requests` (at most kPlanRequests) requests.
-// `entry(b)` returns request b's share (count 0 past the last request; its
-// loads must be safe there).  chunk = max(min_chunk, ceil(total work /
-// target)), at most max_chunk units per split (0 target: unsplit up to
-// max_chunk); at most max_splits splits.  The items number at most target +
-// the sum of the counts while max_chunk and max_splits do not bind (the host
-// sizes the grid).  The host keeps the total work below 2^31.
-// Wave-uniform; every wave of the grid computes the same plan.
-template <class Entry>
-__device__ __forceinline__ PlanItem plan_item(int requests, int item, int target, int min_chunk, int max_chunk,
-                                              int max_splits, Entry entry) {
+// The sizes of a plan.  A batch whose longest request is at most 9/8 of the
+// mean takes `even_splits` of every request, the count the host chose for
+// equal lengths as long as the page table, or fewer so that a split keeps
+// min_chunk units.  Else a request takes ceil(length / chunk) splits (at most
+// max_splits), chunk = max(min_chunk, ceil(total work / target)) units, at
+// most max_chunk (target 0: max_chunk), and at least round_chunk where smaller
+// ones would make more items than round_target; the items are ordered by size
+// in four classes, the longest first, so that what starts last is short.
+struct PlanSizes {
+    int target, even_splits, min_chunk, max_chunk, max_splits;
+    int round_chunk, round_target;
+};
+
+// Item `key` of the plan over `requests` (at most kPlanRequests) requests.
+// `own` is the share of request `lane` (count 0 past the last request).  The items number at
+// most max(even_splits x counts, target + counts) while max_chunk does not
+// bind (the host sizes the grid), and the entries (rows x splits) at most
+// max(even_splits x rows, rows + target x the most rows of one item).  The
+// host keeps the total work below 2^31.  Wave-uniform; every wave of every
+// kernel of a call derives the same plan.
+__device__ __forceinline__ PlanItem plan_find(int requests, int key, const PlanSizes& sizes, const PlanEntry& own) {
     const int lane = threadIdx.x & 63;
-    PlanEntry e[kPlanChunks];
-    uint32_t work = 0, longest = 0;
-    bool single = true;
-#pragma unroll
-    for (int j = 0; j < kPlanChunks; ++j) {
-        e[j] = PlanEntry{0, 0, 0, 0};
-        if (64 * j < requests) e[j] = entry(64 * j + lane);
-        work += (uint32_t)e[j].count * (uint32_t)e[j].length;
-        longest = max(longest, (uint32_t)e[j].length);
-        single = single && e[j].count == (64 * j + lane < requests ? 1 : 0);
-    }
-    const uint32_t total = __builtin_amdgcn_readlane(wave_scan(work, lane), 63);
-    longest = wave_max_u32(longest);
-    uint32_t chunk = (uint32_t)max_chunk;
-    // Plain batches whose longest request is at most a chunk (equal lengths
-    // that fill the device): item i is request i, and no division is taken.
-    if (requests <= 64 && longest <= (uint32_t)max_chunk && __all(single) &&
-        (target <= 0 || longest <= (uint32_t)min_chunk ||
-         (uint64_t)(longest - 1) * (uint32_t)target < total)) {
-        PlanItem r{item < requests ? item : -1, 0, 0, 1, 0, 0, 0, item, requests};
-        const int src = item < requests ? item : 0;
-        r.length = __builtin_amdgcn_readlane(e[0].length, src);
-        r.first = __builtin_amdgcn_readlane(e[0].first, src);
-        r.tokens = __builtin_amdgcn_readlane(e[0].tokens, src);
+    const uint32_t length = (uint32_t)own.length, count = (uint32_t)own.count;
+    const uint32_t min_chunk = (uint32_t)sizes.min_chunk;
+    const uint32_t total = __builtin_amdgcn_readlane(wave_scan(count * length, lane), 63);
+    const uint32_t counts = __builtin_amdgcn_readlane(wave_scan(count, lane), 63);
+    const uint32_t longest = wave_max_u32(count > 0 ? length : 0u);
+    const bool even = 8ull * longest * counts <= 9ull * total;
+    uint32_t even_splits = (uint32_t)sizes.even_splits;
+    if (even_splits > 1 && longest < even_splits * min_chunk) even_splits = max(longest / min_chunk, 1u);
+    PlanItem r{-1, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0};
+    auto take = [&](int src) {
+        r.request = src;
+        r.length = __builtin_amdgcn_readlane(own.length, src);
+        r.first = __builtin_amdgcn_readlane(own.first, src);
+        r.tokens = __builtin_amdgcn_readlane(own.tokens, src);
+        r.rows = __builtin_amdgcn_readlane(own.rows, src);
+    };
+    // Plain batches of near-equal requests that stay whole: item i is request i.
+    if (even && even_splits == 1 && __all(own.count == (lane < requests ? 1 : 0))) {
+        if (key < requests) take(key);
+        r.entry = r.first;
+        r.offset = key;
+        r.total = requests;
         return r;
     }
-    if (target > 0) {
-        const uint32_t even = (total + (uint32_t)target - 1) / (uint32_t)target;
-        chunk = even > (uint32_t)min_chunk ? even : (uint32_t)min_chunk;
-        chunk = chunk < (uint32_t)max_chunk ? chunk : (uint32_t)max_chunk;
+    uint32_t splits = even_splits;
+    int size_class = 0;
+    if (!even) {
+        uint32_t chunk = (uint32_t)sizes.max_chunk;
+        if (sizes.target > 0) {
+            const uint32_t share = (total + (uint32_t)sizes.target - 1) / (uint32_t)sizes.target;
+            const uint32_t round_share = (total + (uint32_t)sizes.round_target - 1) / (uint32_t)sizes.round_target;
+            chunk = min(max(max(share, min_chunk), min((uint32_t)sizes.round_chunk, round_share)), chunk);
+        }
+        splits = min(max((length + chunk - 1) / chunk, 1u), (uint32_t)sizes.max_splits);
+        if (splits > 1 && splits * min_chunk > length && length <= (uint32_t)sizes.max_chunk) splits -= 1;
+        // A split's share of a chunk: above 3/4, 1/2, 1/4 or less.
+        const float whole = (float)splits * (float)chunk, part = (float)length;
+        size_class = part > 0.75f * whole ? 0 : part > 0.5f * whole ? 1 : part > 0.25f * whole ? 2 : 3;
     }
-    PlanItem r{-1, 0, 0, 1, 0, 0, 0, 0, 0};
-    uint32_t base = 0;
-#pragma unroll
-    for (int j = 0; j < kPlanChunks; ++j) {
-        if (64 * j >= requests) break;
-        uint32_t splits = ((uint32_t)e[j].length + chunk - 1) / chunk;
-        splits = splits < 1u ? 1u : splits;
-        splits = splits < (uint32_t)max_splits ? splits : (uint32_t)max_splits;
-        const uint32_t items = (uint32_t)e[j].count * splits;
+    const uint32_t entry_end = wave_scan((uint32_t)own.rows * splits, lane);
+    uint32_t local = 0, base = 0;
+    for (int k = 0; k < (even ? 1 : 4); ++k) {
+        const uint32_t items = size_class == k ? count * splits : 0u;
         const uint32_t end = base + wave_scan(items, lane), begin = end - items;
-        const uint64_t mask = __ballot(begin <= (uint32_t)item && (uint32_t)item < end);
+        const uint64_t mask = __ballot(begin <= (uint32_t)key && (uint32_t)key < end);
         if (mask != 0) {
-            const int src = __builtin_ctzll(mask);
-            r.request = 64 * j + src;
-            r.splits = (int)__builtin_amdgcn_readlane(splits, src);
-            const uint32_t local = (uint32_t)item - __builtin_amdgcn_readlane(begin, src);
-            r.index = (int)(local / (uint32_t)r.splits);
-            r.split = (int)local - r.index * r.splits;
-            r.offset = item - r.split;
-            r.length = __builtin_amdgcn_readlane(e[j].length, src);
-            r.first = __builtin_amdgcn_readlane(e[j].first, src);
-            r.tokens = __builtin_amdgcn_readlane(e[j].tokens, src);
+            take(__builtin_ctzll(mask));
+            r.offset = (int)__builtin_amdgcn_readlane(begin, r.request);
+            local = (uint32_t)(key - r.offset);
         }
         base = __builtin_amdgcn_readlane(end, 63);
     }
     r.total = (int)base;
+    if (r.request < 0) return r;
+    r.splits = (int)__builtin_amdgcn_readlane(splits, r.request);
+    r.index = (int)(local / (uint32_t)r.splits);
+    r.split = (int)local - r.index * r.splits;
+    r.offset += r.index * r.splits;
+    r.entry = (int)__builtin_amdgcn_readlane(entry_end, r.request) - r.rows * r.splits;
     return r;
 }
 

@@ -1,5 +1,5 @@
-"""Decode calls whose work is planned on the device from the request lengths
-(csrc/rq_plan.h): requests of very different lengths, several rows of one
+"""Calls whose work is planned on the device from the request lengths
+(csrc/rq_plan.h), one row per request and several: requests of very different lengths, several rows of one
 request among single ones, requests without rows, more requests than one
 64-lane register set or than the plan covers, against the FP64 oracle with
 the attention bars."""
@@ -13,6 +13,7 @@ import torch
 import residualquant_amd as rq
 
 from .cases import OURO_G32, make_decode, oracle_attention
+from .test_gpu_multirow import _bf16, _oracle, _run
 
 pytestmark = pytest.mark.gpu
 
@@ -63,6 +64,31 @@ def test_planned_decode_matches_oracle(oracle, device, case):
             assert err.max() <= MAX_ABS and err.mean() <= bar, (loop, err.max(), err.mean(), bar)
     finally:
         rq.ops.set_split_target(0)
+
+
+MULTIROW_CASES = [
+    # lengths (incl. the new rows), rows per request, heads, dim, page tokens, mode
+    ([2500, 40, 300, 9, 700], [3, 2, 20, 4, 0], 16, 128, 16, "anchor"),
+    ([1900, 400, 150], [40, 3, 70], 3, 96, 32, "anchor"),
+    ([1300, 70], [4, 2], 16, 128, 16, "adjacent"),
+    ([40] * 64 + [900], [2] * 65, 1, 128, 16, "anchor"),  # more requests than the plan covers
+]
+
+
+@pytest.mark.parametrize("case", MULTIROW_CASES, ids=lambda c: f"{len(c[0])}x{c[0][0]}-d{c[3]}-pt{c[4]}-{c[5]}")
+@pytest.mark.parametrize("causal", [True, False], ids=["prefill", "decode"])
+def test_planned_multirow_matches_oracle(oracle, device, case, causal):
+    print(f"[case] planned multirow causal={causal} {str(case)[:120]}", flush=True)
+    lengths, rows, heads, dim, pt, mode = case
+    records = ADJACENT if mode == "adjacent" else OURO_G32
+    d = make_decode(lengths, heads, dim, records, seed=len(lengths) + dim, page_tokens=pt, mode=mode,
+                    anchor=0 if mode == "adjacent" else 3, rows_per_request=rows)
+    cache_np = d.group.oracle_cache(oracle)
+    cache = torch.from_numpy(cache_np).to(device)
+    for loop in (1, 3):
+        err = np.abs(_run(d, device, cache, loop, causal) - _bf16(_oracle(oracle, d, cache_np, loop, causal)))
+        print(f"[case]   loop {loop}: max {err.max():.3g} mean {err.mean():.3g}", flush=True)
+        assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS, (loop, err.max(), err.mean())
 
 
 def test_planned_decode_replays(device):
