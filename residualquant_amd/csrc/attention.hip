@@ -109,21 +109,6 @@ __device__ __forceinline__ float rows_max(float x) {
                        __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 48))));
 }
 
-// A workgroup barrier for data exchanged through LDS by ordinary LDS
-// accesses: this wave's LDS operations complete (s_waitcnt lgkmcnt(0)), then
-// s_barrier; the empty asm statements keep the compiler from moving memory
-// accesses across it.  __syncthreads (and an LDS release fence, which also
-// covers LDS writes of DMA loads) waits for every load in flight
-// (vmcnt(0)): in the decode prologues that would hold the query preparation
-// until the first page loads, issued before it, have landed.  Not for data
-// written to LDS by DMA loads or read from global memory.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt not waited
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // ------------------------------------------------------------------ prepare
 
 
@@ -710,7 +695,7 @@ __device__ __forceinline__ DecodeItem decode_item(const AttentionParams& p, int 
         const int64_t pages = min((int64_t)(history / PT + (history % PT != 0)), p.max_pages);
         const int count = b < requests ? max(hi - lo, 0) : 0;
         const PlanItem plan = plan_find(
-            requests, item, PlanSizes{p.plan_target, p.splits, p.plan_min_pages, INT_MAX, kMaxSplits, p.plan_round_pages, p.plan_round_target},
+            requests, item, PlanSizes{p.plan_target, p.splits, p.plan_min_pages, INT_MAX, kMaxSplits, p.plan_round_pages, p.plan_round_target, 18},
             PlanEntry{count, (int)pages, lo, (int)min((int64_t)history, pages * PT), count});
         d.row = __builtin_amdgcn_readfirstlane(plan.first + plan.index);
         d.splits = plan.splits;

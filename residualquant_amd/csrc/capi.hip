@@ -141,6 +141,7 @@ struct WorkspaceLayout {
 };
 
 constexpr int64_t kMultiRowMinRows = 3;          // anchor-loop calls
+constexpr int64_t kChunkMinRows = 48;            // the chunk kernels
 constexpr int64_t kMultiRowMinRowsResidual = 2;  // residual-loop calls
 
 // Several rows per request (either head dim, either mode) run the multi-row
@@ -200,6 +201,7 @@ void plan_multirow(rq::MultiRowParams& m, int splits, size_t bytes) {
     // Rows per stream tile: 16 when the call's requests average 16 rows or
     // fewer, else 32.
     m.tile_rows = m.rows <= 16 * m.requests ? 16 : 32;
+    m.plan_unit = 32;
     m.splits = splits;
     m.entries = m.rows * splits;
     if (m.requests > rq::kPlanRequests) {
@@ -239,6 +241,49 @@ uint64_t next_call_tag() {
     do tag = counter.fetch_add(1, std::memory_order_relaxed) & kMask;
     while (tag == 0);
     return tag;
+}
+
+// Whether a call's requests average enough rows for the chunk kernels
+// (chunk.hip): 1 request of 1000 tokens x 48 rows x 16 heads takes 26.8 us per
+// residual call on them and 30.9 us on 32-row tiles, 4 requests of 3000 tokens
+// x 48 rows 47 and 52 us; at 32 rows 26.5 and 24.0 us, at 24 rows x 16
+// requests of 4000 tokens 126 and 81 us.
+bool takes_chunk_kernels(int64_t rows, int64_t requests) {
+    return requests <= rq::kPlanRequests && rows >= kChunkMinRows * requests;
+}
+
+// The most partial entries that the plan of a chunk call takes per head.
+int64_t chunk_entries(int64_t rows, int heads) {
+    const int64_t target = (compute_units() + heads - 1) / heads;
+    return std::min<int64_t>(rows * rq::kChunkMaxSplits, rows + target * rq::kChunkTileRows);
+}
+
+// The plan of a chunk call: one stream workgroup fits a compute unit.
+void plan_chunk(rq::MultiRowParams& m, size_t bytes) {
+    constexpr int64_t unit = rq::kChunkUnit;
+    const int64_t units = compute_units();
+    m.tile_rows = rq::kChunkTileRows;
+    m.plan_unit = (int)unit;
+    const int64_t steps = std::max<int64_t>(1, (m.max_pages * m.page_tokens + unit - 1) / unit);
+    const int64_t row_tiles = m.rows / m.tile_rows + m.requests;  // at most, over all requests
+    m.plan_max = (int)(rq::kMultiRowMaxSplitPages * m.page_tokens / unit);
+    const int64_t forced = (steps + m.plan_max - 1) / m.plan_max;
+    m.plan_min = 2;
+    m.plan_max_splits = (int)std::max<int64_t>(rq::kChunkMaxSplits, forced);
+    const int64_t fit = (int64_t)(bytes / (sizeof(float) * rq::kMultiRowEntry) / m.heads);
+    // Equal requests: the splits that fill the compute units once.
+    const int64_t average = (m.rows + m.requests - 1) / m.requests;
+    const int64_t groups = m.requests * m.heads * ((average + m.tile_rows - 1) / m.tile_rows);
+    int64_t splits = std::max<int64_t>(units / groups, forced);
+    splits = std::min<int64_t>(splits, std::min<int64_t>(fit / m.rows, m.plan_max_splits));
+    m.splits = (int)std::max<int64_t>(splits, 1);
+    int64_t target = (3 * units / 4 + m.heads - 1) / m.heads;
+    if (m.rows * m.plan_max_splits > fit)
+        target = std::max<int64_t>(0, std::min<int64_t>(target, (fit - m.rows * forced) / m.tile_rows));
+    if (row_tiles > INT32_MAX / steps) target = 0;  // the device sums row tiles x history steps in 31 bits
+    m.plan_target = (int)target;
+    m.entries = fit;
+    m.items = (int)std::max(row_tiles * forced + target, row_tiles * m.splits);
 }
 
 // What the device-side plan of a packed decode call (decode_item in
@@ -413,7 +458,9 @@ static size_t attention_workspace_total(int64_t rows, int heads, int head_dim, i
     size_t total = workspace_layout(rows, heads, head_dim, splits).total;
     if ((head_dim == 96 || head_dim == 128) && (page_tokens == 16 || page_tokens == 32))
         total = std::max(total,
-                         multirow_bytes(rows, heads, multirow_workspace_splits(rows, heads, max_pages, page_tokens)));
+                         std::max(multirow_bytes(rows, heads,
+                                                 multirow_workspace_splits(rows, heads, max_pages, page_tokens)),
+                                  sizeof(float) * rq::kMultiRowEntry * heads * (size_t)chunk_entries(rows, heads)));
     return total;
 }
 
@@ -598,13 +645,19 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         m.compute_units = compute_units();
         m.partials = static_cast<float*>(workspace);
         m.call_tag = next_call_tag();
-        plan_multirow(m, splits, std::min(workspace_bytes, full_bytes));
+        const bool chunk = takes_chunk_kernels(rows, requests);
+        if (chunk)
+            plan_chunk(m, std::min(workspace_bytes, full_bytes));
+        else
+            plan_multirow(m, splits, std::min(workspace_bytes, full_bytes));
         if ((int64_t)splits * row_tiles > 65535 || requests > (int64_t)INT32_MAX || rows > (int64_t)INT32_MAX)
             return fail(RQ_EINVAL, "Too many rows for one multi-row attention launch");
         hipEvent_t begin = nullptr, end = nullptr;
         if (timed) timing_events(stream, &begin, &end);
         if (begin) (void)hipEventRecord(begin, stream);
-        const hipError_t launched = rq::launch_multirow(m, stream);
+        const hipError_t launched =
+            head_dim == 96 ? (chunk ? rq::launch_chunk<96>(m, stream) : rq::launch_multirow<96>(m, stream))
+                           : (chunk ? rq::launch_chunk<128>(m, stream) : rq::launch_multirow<128>(m, stream));
         if (end) (void)hipEventRecord(end, stream);
         return check_launch(launched, "multi-row attention launch");
     }

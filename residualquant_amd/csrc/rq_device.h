@@ -176,6 +176,21 @@ typedef const int32_t __attribute__((address_space(4))) ConstantInt32;
 // operations (loads and stores) are waited for.
 __device__ __forceinline__ void wait_vector_memory() { __builtin_amdgcn_s_waitcnt(0xF70); }
 
+// A workgroup barrier for data exchanged through LDS by ordinary LDS
+// accesses: this wave's LDS operations complete (s_waitcnt lgkmcnt(0)), then
+// s_barrier; the empty asm statements keep the compiler from moving memory
+// accesses across it.  __syncthreads (and an LDS release fence, which also
+// covers LDS writes of DMA loads) waits for every load in flight
+// (vmcnt(0)): in the decode prologues that would hold the query preparation
+// until the first page loads, issued before it, have landed.  Not for data
+// written to LDS by DMA loads or read from global memory.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0); vmcnt and expcnt not waited
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Wave priority by the progress of a page stream of `steps` steps: 3 for
 // the first 10/16 of the steps, then 2, 1 and from 15/16 on 0.  Two
 // workgroups whose waves share the SIMDs of a compute unit otherwise

@@ -250,15 +250,34 @@ struct MultiRowParams {
     // requests (items 0) every (request, head, row tile) takes `splits`.
     int items;
     int splits;
-    int plan_target, plan_min, plan_max, plan_max_splits;  // PlanSizes, in 32-token tiles
-    int tile_rows;        // rows of a stream tile: 16 or 32
+    int plan_target, plan_min, plan_max, plan_max_splits;  // PlanSizes, in units of plan_unit tokens
+    int plan_unit;        // 32, or 128 (chunk kernels)
+    int tile_rows;        // rows of a stream tile: 16, 32 or 256 (chunk kernels)
     int compute_units;    // of the launching device
     int64_t resident;     // set by the launch: stream workgroups the device holds at once
     int64_t entries;      // partials per head
     float* partials;      // workspace [heads, entries, kMultiRowEntry]; a request's entries: [row, split]
     uint64_t call_tag;    // of this call (56 bits, rq_plan.h)
 };
+template <int D>
 hipError_t launch_multirow(const MultiRowParams& p, hipStream_t stream);
+template <>
+hipError_t launch_multirow<96>(const MultiRowParams& p, hipStream_t stream);
+template <>
+hipError_t launch_multirow<128>(const MultiRowParams& p, hipStream_t stream);
+
+// The same call for requests of many rows (chunk.hip): 256-row tiles share
+// each dequantized page tile, the live tokens run on MFMA in a second launch.
+// Takes at most kPlanRequests requests.
+constexpr int kChunkTileRows = 256;
+constexpr int kChunkUnit = 128;      // tokens that a workgroup dequantizes per step
+constexpr int kChunkMaxSplits = 16;  // for parallelism
+template <int D>
+hipError_t launch_chunk(const MultiRowParams& p, hipStream_t stream);
+template <>
+hipError_t launch_chunk<96>(const MultiRowParams& p, hipStream_t stream);
+template <>
+hipError_t launch_chunk<128>(const MultiRowParams& p, hipStream_t stream);
 hipError_t launch_attention_bf16(const AttentionParams& p, hipStream_t stream, hipEvent_t begin,
                                  hipEvent_t end);
 

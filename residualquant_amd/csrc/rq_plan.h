@@ -73,10 +73,52 @@ __device__ __forceinline__ uint32_t wave_scan(uint32_t x, int lane) {
 // most max_chunk (target 0: max_chunk), and at least round_chunk where smaller
 // ones would make more items than round_target; the items are ordered by size
 // in four classes, the longest first, so that what starts last is short.
+// A batch whose counts already are 3/4 of the target counts as near equal up
+// to full_eighths / 8 of the mean: 13 for several rows per request (6 requests
+// of 1310..4150 tokens x 29 rows x 55 heads: 94 us with the two even splits,
+// 100 us with nine planned ones), 18 for decode (42 requests of 188..922
+// tokens, 16 heads: 4-loop step 114 us whole, 125 us planned; 64 requests of
+// 100..2000 tokens, the longest 3.2 times the mean: residual call 62 us whole,
+// 54 us planned).
 struct PlanSizes {
     int target, even_splits, min_chunk, max_chunk, max_splits;
     int round_chunk, round_target;
+    int full_eighths;
 };
+
+// What every request of a plan shares.
+struct PlanShare {
+    bool even, whole;  // near-equal requests; of one split each
+    uint32_t even_splits, chunk;
+};
+
+__device__ __forceinline__ PlanShare plan_share(const PlanSizes& sizes, const PlanEntry& own, int lane) {
+    const uint32_t length = (uint32_t)own.length, count = (uint32_t)own.count;
+    const uint32_t min_chunk = (uint32_t)sizes.min_chunk;
+    const uint32_t total = __builtin_amdgcn_readlane(wave_scan(count * length, lane), 63);
+    const uint32_t counts = __builtin_amdgcn_readlane(wave_scan(count, lane), 63);
+    const uint32_t longest = wave_max_u32(count > 0 ? length : 0u);
+    PlanShare s;
+    const bool full = 4ull * counts >= 3ull * (uint32_t)sizes.target;
+    s.even = 8ull * longest * counts <= (uint64_t)(full ? sizes.full_eighths : 9) * total;
+    s.even_splits = (uint32_t)sizes.even_splits;
+    if (s.even_splits > 1 && longest < s.even_splits * min_chunk) s.even_splits = max(longest / min_chunk, 1u);
+    s.whole = s.even && s.even_splits == 1;
+    s.chunk = (uint32_t)sizes.max_chunk;
+    if (!s.even && sizes.target > 0) {
+        const uint32_t share = (total + (uint32_t)sizes.target - 1) / (uint32_t)sizes.target;
+        const uint32_t round_share = (total + (uint32_t)sizes.round_target - 1) / (uint32_t)sizes.round_target;
+        s.chunk = min(max(max(share, min_chunk), min((uint32_t)sizes.round_chunk, round_share)), s.chunk);
+    }
+    return s;
+}
+
+__device__ __forceinline__ uint32_t plan_splits(const PlanSizes& sizes, const PlanShare& share, uint32_t length) {
+    if (share.even) return share.even_splits;
+    uint32_t splits = min(max((length + share.chunk - 1) / share.chunk, 1u), (uint32_t)sizes.max_splits);
+    if (splits > 1 && splits * (uint32_t)sizes.min_chunk > length && length <= (uint32_t)sizes.max_chunk) splits -= 1;
+    return splits;
+}
 
 // Item `key` of the plan over `requests` (at most kPlanRequests) requests.
 // `own` is the share of request `lane` (count 0 past the last request).  The items number at
@@ -88,13 +130,7 @@ struct PlanSizes {
 __device__ __forceinline__ PlanItem plan_find(int requests, int key, const PlanSizes& sizes, const PlanEntry& own) {
     const int lane = threadIdx.x & 63;
     const uint32_t length = (uint32_t)own.length, count = (uint32_t)own.count;
-    const uint32_t min_chunk = (uint32_t)sizes.min_chunk;
-    const uint32_t total = __builtin_amdgcn_readlane(wave_scan(count * length, lane), 63);
-    const uint32_t counts = __builtin_amdgcn_readlane(wave_scan(count, lane), 63);
-    const uint32_t longest = wave_max_u32(count > 0 ? length : 0u);
-    const bool even = 8ull * longest * counts <= 9ull * total;
-    uint32_t even_splits = (uint32_t)sizes.even_splits;
-    if (even_splits > 1 && longest < even_splits * min_chunk) even_splits = max(longest / min_chunk, 1u);
+    const PlanShare share = plan_share(sizes, own, lane);
     PlanItem r{-1, 0, 0, 1, 0, 0, 0, 0, 0, 0, 0};
     auto take = [&](int src) {
         r.request = src;
@@ -104,31 +140,23 @@ __device__ __forceinline__ PlanItem plan_find(int requests, int key, const PlanS
         r.rows = __builtin_amdgcn_readlane(own.rows, src);
     };
     // Plain batches of near-equal requests that stay whole: item i is request i.
-    if (even && even_splits == 1 && __all(own.count == (lane < requests ? 1 : 0))) {
+    if (share.whole && __all(own.count == (lane < requests ? 1 : 0))) {
         if (key < requests) take(key);
-        r.entry = r.first;
+        r.entry = (int)(__builtin_amdgcn_readlane(wave_scan((uint32_t)own.rows, lane), key & 63)) - r.rows;
         r.offset = key;
         r.total = requests;
         return r;
     }
-    uint32_t splits = even_splits;
+    const uint32_t splits = plan_splits(sizes, share, length);
     int size_class = 0;
-    if (!even) {
-        uint32_t chunk = (uint32_t)sizes.max_chunk;
-        if (sizes.target > 0) {
-            const uint32_t share = (total + (uint32_t)sizes.target - 1) / (uint32_t)sizes.target;
-            const uint32_t round_share = (total + (uint32_t)sizes.round_target - 1) / (uint32_t)sizes.round_target;
-            chunk = min(max(max(share, min_chunk), min((uint32_t)sizes.round_chunk, round_share)), chunk);
-        }
-        splits = min(max((length + chunk - 1) / chunk, 1u), (uint32_t)sizes.max_splits);
-        if (splits > 1 && splits * min_chunk > length && length <= (uint32_t)sizes.max_chunk) splits -= 1;
+    if (!share.even) {
         // A split's share of a chunk: above 3/4, 1/2, 1/4 or less.
-        const float whole = (float)splits * (float)chunk, part = (float)length;
+        const float whole = (float)splits * (float)share.chunk, part = (float)length;
         size_class = part > 0.75f * whole ? 0 : part > 0.5f * whole ? 1 : part > 0.25f * whole ? 2 : 3;
     }
     const uint32_t entry_end = wave_scan((uint32_t)own.rows * splits, lane);
     uint32_t local = 0, base = 0;
-    for (int k = 0; k < (even ? 1 : 4); ++k) {
+    for (int k = 0; k < (share.even ? 1 : 4); ++k) {
         const uint32_t items = size_class == k ? count * splits : 0u;
         const uint32_t end = base + wave_scan(items, lane), begin = end - items;
         const uint64_t mask = __ballot(begin <= (uint32_t)key && (uint32_t)key < end);
@@ -146,6 +174,22 @@ __device__ __forceinline__ PlanItem plan_find(int requests, int key, const PlanS
     r.split = (int)local - r.index * r.splits;
     r.offset += r.index * r.splits;
     r.entry = (int)__builtin_amdgcn_readlane(entry_end, r.request) - r.rows * r.splits;
+    return r;
+}
+
+// The splits and the first entry of request `request` in the same plan.
+struct PlanRequest {
+    int splits, entry;
+};
+
+__device__ __forceinline__ PlanRequest plan_request(int request, const PlanSizes& sizes, const PlanEntry& own) {
+    const int lane = threadIdx.x & 63;
+    const PlanShare share = plan_share(sizes, own, lane);
+    const uint32_t splits = share.whole ? 1u : plan_splits(sizes, share, (uint32_t)own.length);
+    const uint32_t entry_end = wave_scan((uint32_t)own.rows * splits, lane);
+    PlanRequest r;
+    r.splits = (int)__builtin_amdgcn_readlane(splits, request);
+    r.entry = (int)__builtin_amdgcn_readlane(entry_end, request) - __builtin_amdgcn_readlane(own.rows, request) * r.splits;
     return r;
 }
 
