@@ -103,8 +103,14 @@ __device__ __forceinline__ PlanShare plan_share(const PlanSizes& sizes, const Pl
     s.even = 8ull * longest * counts <= (uint64_t)(full ? sizes.full_eighths : 9) * total;
     s.even_splits = (uint32_t)sizes.even_splits;
     if (s.even_splits > 1 && longest < s.even_splits * min_chunk) s.even_splits = max(longest / min_chunk, 1u);
-    s.whole = s.even && s.even_splits == 1;
     s.chunk = (uint32_t)sizes.max_chunk;
+    if (s.even && s.even_splits == 1 && 8ull * longest * counts > 9ull * total && longest <= s.chunk) {
+        // Whole, but not alike: one split each, the longest first.
+        s.even = s.whole = false;
+        s.chunk = longest;
+        return s;
+    }
+    s.whole = s.even && s.even_splits == 1;
     if (!s.even && sizes.target > 0) {
         const uint32_t share = (total + (uint32_t)sizes.target - 1) / (uint32_t)sizes.target;
         const uint32_t round_share = (total + (uint32_t)sizes.round_target - 1) / (uint32_t)sizes.round_target;

@@ -136,3 +136,27 @@ def test_prefill_rejects_unsupported(device):
     q = torch.zeros((4, 2, 128), dtype=torch.bfloat16, device=device)
     with pytest.raises(RuntimeError, match="Only dropout-free"):
         rq.flash_attn_varlen_func(q, q, q, 4, cu, 4, causal=True, dropout_p=0.1)
+
+
+@pytest.mark.parametrize("lengths", [[17, 300, 0, 1, 129, 640, 55], [128, 257] + [3] * 63],
+                         ids=["ragged7", "batch65"])
+@pytest.mark.parametrize("dim,causal", [(128, True), (96, True), (128, False)])
+def test_prefill_batch_equals_its_sequences(device, lengths, dim, causal):
+    """A batch's pairs are ranked by length on the device (up to 64 sequences);
+    each sequence's rows are the bytes of a call of its own."""
+    heads, total = 3, sum(lengths)
+    generator = torch.Generator(device=device).manual_seed(total + dim)
+    q, k, v = (torch.randn((total, heads, dim), generator=generator, device=device).to(torch.bfloat16)
+               for _ in range(3))
+    starts = torch.tensor([0] + list(np.cumsum(lengths)), dtype=torch.int32, device=device)
+    out = rq.flash_attn_varlen_func(q, k, v, max(lengths), starts, max(lengths), starts, causal=causal,
+                                    out=torch.full_like(q, float("nan")))
+    at = 0
+    for n in lengths:
+        rows = slice(at, at + n)
+        at += n
+        if n == 0:
+            continue
+        one = torch.tensor([0, n], dtype=torch.int32, device=device)
+        alone = rq.flash_attn_varlen_func(q[rows], k[rows], v[rows], n, one, n, one, causal=causal)
+        assert torch.equal(out[rows].view(torch.int16), alone.view(torch.int16)), n
