@@ -14,6 +14,8 @@ device; nothing synchronizes.
 from __future__ import annotations
 
 import ctypes
+from contextlib import nullcontext
+from functools import lru_cache
 from typing import Optional, Sequence, Tuple
 
 import torch
@@ -29,32 +31,56 @@ def _require(condition: bool, message: str) -> None:
         raise RuntimeError(message)
 
 
-def _validate_bf16_token_tensor(tensor: torch.Tensor) -> None:
+# A call on one small request runs about 14 us on the GPU, and what the host
+# does per call is what a loop of such calls waits for (20 us per attention
+# call before the checks below read each tensor's shape and strides once, the
+# device context was entered only for another device than the current one, the
+# schedule's C arrays were kept by value and the stream's handle was read
+# without a Stream object; 14 us, the GPU time, with them).
+
+
+def _validate_bf16_token_tensor(tensor: torch.Tensor) -> Tuple[torch.Size, int]:
+    """The tensor's shape and token stride."""
     # common/api.h:42-49
-    _require(tensor.is_cuda and tensor.dtype == torch.bfloat16 and tensor.dim() == 3
-             and tensor.stride(1) == tensor.size(2) and tensor.stride(2) == 1,
-             "BF16 [tokens, heads, channels] with packed trailing strides required")
+    if tensor.is_cuda and tensor.dtype is torch.bfloat16:
+        shape = tensor.shape
+        if len(shape) == 3:
+            stride = tensor.stride()
+            if stride[1] == shape[2] and stride[2] == 1:
+                return shape, stride[0]
+    raise RuntimeError("BF16 [tokens, heads, channels] with packed trailing strides required")
 
 
-def _rotation_pointer(rotation: Optional[torch.Tensor], device, heads: int, head_dim: int):
+def _rotation_pointer(rotation: Optional[torch.Tensor], device: int, heads: int, head_dim: int):
     # common/api.h:51-64
     if rotation is None:
         return None
-    _require(rotation.device == device and rotation.is_contiguous() and rotation.dtype == torch.float16
-             and rotation.dim() == 3 and rotation.size(0) == heads and rotation.size(1) == head_dim
-             and rotation.size(2) == head_dim,
+    _require(rotation.get_device() == device and rotation.is_contiguous() and rotation.dtype is torch.float16
+             and rotation.shape == (heads, head_dim, head_dim),
              "Contiguous FP16 [heads, channels, channels] rotation required")
     return rotation.data_ptr()
 
 
+@lru_cache(maxsize=64)
+def _schedule_arrays(records: Tuple[Tuple[int, int], ...]):
+    # The library only reads them.
+    bits = (ctypes.c_int * max(1, len(records)))(*[r[0] for r in records])
+    groups = (ctypes.c_int * max(1, len(records)))(*[r[1] for r in records])
+    return bits, groups, ctypes.addressof(bits), ctypes.addressof(groups)
+
+
 def _schedule(records: Sequence[Sequence[int]]):
-    bits = (ctypes.c_int * max(1, len(records)))(*[int(r[0]) for r in records])
-    groups = (ctypes.c_int * max(1, len(records)))(*[int(r[1]) for r in records])
-    return bits, groups
+    """(bits, groups, their addresses) of a schedule; the arrays live as long as the caller holds them."""
+    return _schedule_arrays(tuple([(int(r[0]), int(r[1])) for r in records]))
 
 
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+def _on_device(device: int):
+    """A context on CUDA device ``device`` (nothing to do where it is current)."""
+    return nullcontext() if torch.cuda.current_device() == device else torch.cuda.device(device)
+
+
+def _stream(device: int) -> int:
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def quantize(key_value_pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]], kv_cache: torch.Tensor,
@@ -73,47 +99,51 @@ def quantize(key_value_pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]], kv_ca
     _require(kv_cache.is_cuda and kv_cache.dtype == torch.uint8 and kv_cache.is_contiguous()
              and kv_cache.dim() == 5 and kv_cache.size(0) == 2,
              "Contiguous CUDA UINT8 [2, blocks, heads, page tokens, page width] cache required")
-    heads = kv_cache.size(2)
+    device = kv_cache.get_device()
+    _, num_blocks, heads, page_tokens, page_width = kv_cache.shape
     head_dim = key_value_pairs[0][0].size(-1)
-    _require(slot_mapping.device == kv_cache.device and slot_mapping.dtype == torch.int64
+    _require(slot_mapping.get_device() == device and slot_mapping.dtype is torch.int64
              and slot_mapping.dim() == 1 and slot_mapping.is_contiguous(),
              "Contiguous INT64 slot mapping on the cache device required")
+    tokens = slot_mapping.numel()
+    pointers, strides, input_rows = ([], []), ([], []), None
     for pair in key_value_pairs:
+        layouts = []
         for tensor in pair:
-            _validate_bf16_token_tensor(tensor)
-            _require(tensor.device == kv_cache.device and tensor.size(1) == heads
-                     and tensor.size(2) == head_dim,
+            shape, stride = _validate_bf16_token_tensor(tensor)
+            rows = shape[0]
+            _require(tensor.get_device() == device and shape[1] == heads and shape[2] == head_dim,
                      "K/V must match the cache device/head count and logical channel count")
-            _require(tensor.size(0) >= slot_mapping.numel(), "Input has fewer rows than slot mapping")
+            _require(rows >= tokens, "Input has fewer rows than slot mapping")
+            layouts.append((tensor.data_ptr(), stride, rows))
+        for plane in (0, 1):
+            pointer, stride, rows = layouts[plane]
+            pointers[plane].append(pointer)
+            strides[plane].append(stride)
+            input_rows = rows if input_rows is None or rows < input_rows else input_rows
     if key_mean is not None:
-        _require(key_mean.device == kv_cache.device and key_mean.dtype == torch.float32
+        _require(key_mean.get_device() == device and key_mean.dtype is torch.float32
                  and key_mean.is_contiguous() and key_mean.dim() == 3
                  and key_mean.size(0) == len(records) and key_mean.size(1) == heads
                  and key_mean.size(2) == head_dim,
                  "Contiguous FP32 [records, heads, channels] key mean required")
-    key_rotation_ptr = _rotation_pointer(key_rotation, kv_cache.device, heads, head_dim)
-    value_rotation_ptr = _rotation_pointer(value_rotation, kv_cache.device, heads, head_dim)
+    key_rotation_ptr = _rotation_pointer(key_rotation, device, heads, head_dim)
+    value_rotation_ptr = _rotation_pointer(value_rotation, device, heads, head_dim)
     _require(coefficient_method in _COEFFICIENTS, "Unsupported coefficient")
     _require(reference_mode in _MODES, f"Unknown packed reference mode: {reference_mode}")
 
     count = len(records)
-    keys = (ctypes.c_void_p * count)(*[pair[0].data_ptr() for pair in key_value_pairs])
-    values = (ctypes.c_void_p * count)(*[pair[1].data_ptr() for pair in key_value_pairs])
-    key_strides = (ctypes.c_int64 * count)(*[pair[0].stride(0) for pair in key_value_pairs])
-    value_strides = (ctypes.c_int64 * count)(*[pair[1].stride(0) for pair in key_value_pairs])
-    input_rows = min(min(pair[0].size(0), pair[1].size(0)) for pair in key_value_pairs)
-    bits, groups = _schedule(records)
-    with torch.cuda.device(kv_cache.device):
+    pointer_array, stride_array = ctypes.c_void_p * count, ctypes.c_int64 * count
+    keys, values = pointer_array(*pointers[0]), pointer_array(*pointers[1])
+    key_strides, value_strides = stride_array(*strides[0]), stride_array(*strides[1])
+    schedule = _schedule(records)
+    with _on_device(device):
         status = _lib.lib().rq_quantize(
-            count, ctypes.cast(keys, ctypes.c_void_p), ctypes.cast(key_strides, ctypes.c_void_p),
-            ctypes.cast(values, ctypes.c_void_p), ctypes.cast(value_strides, ctypes.c_void_p),
-            input_rows, kv_cache.data_ptr(), kv_cache.size(1), heads, kv_cache.size(3),
-            kv_cache.size(4), slot_mapping.data_ptr(), slot_mapping.numel(), head_dim,
-            key_rotation_ptr, value_rotation_ptr,
-            key_mean.data_ptr() if key_mean is not None else None,
-            ctypes.cast(bits, ctypes.c_void_p), ctypes.cast(groups, ctypes.c_void_p),
-            _MODES[reference_mode], int(anchor_index), _COEFFICIENTS[coefficient_method],
-            _stream(kv_cache.device))
+            count, ctypes.addressof(keys), ctypes.addressof(key_strides), ctypes.addressof(values),
+            ctypes.addressof(value_strides), input_rows, kv_cache.data_ptr(), num_blocks, heads, page_tokens,
+            page_width, slot_mapping.data_ptr(), tokens, head_dim, key_rotation_ptr, value_rotation_ptr,
+            key_mean.data_ptr() if key_mean is not None else None, schedule[2], schedule[3],
+            _MODES[reference_mode], int(anchor_index), _COEFFICIENTS[coefficient_method], _stream(device))
     _lib.check(status)
 
 
@@ -133,25 +163,30 @@ def _workspace(workspace: Optional[torch.Tensor], needed: int, device) -> torch.
 
 
 def _validate_attention_inputs(query, key, value, output, query_start_loc, seq_lens, block_table):
-    _validate_bf16_token_tensor(query)
+    """The token strides of query, key, value and output."""
+    shape, query_stride = _validate_bf16_token_tensor(query)
+    device = query.get_device()
+    strides = [query_stride]
     for tensor in (key, value, output):
-        _validate_bf16_token_tensor(tensor)
-        _require(tensor.device == query.device and tensor.shape == query.shape,
+        other, stride = _validate_bf16_token_tensor(tensor)
+        _require(tensor.get_device() == device and other == shape,
                  "Q/K/V/output must have matching shapes and devices")
-    for tensor in (query, key):
-        _require(tensor.data_ptr() % 8 == 0 and tensor.stride(0) % 4 == 0,
-                 "Q/K addresses and token strides must be 8-byte aligned")
-    _require(query_start_loc.device == query.device and query_start_loc.dtype == torch.int32
+        strides.append(stride)
+    _require(query.data_ptr() % 8 == 0 and query_stride % 4 == 0 and key.data_ptr() % 8 == 0 and strides[1] % 4 == 0,
+             "Q/K addresses and token strides must be 8-byte aligned")
+    requests = seq_lens.numel()
+    _require(query_start_loc.get_device() == device and query_start_loc.dtype is torch.int32
              and query_start_loc.dim() == 1 and query_start_loc.is_contiguous()
-             and query_start_loc.numel() == seq_lens.numel() + 1,
+             and query_start_loc.numel() == requests + 1,
              "Contiguous INT32 query starts with one final boundary required")
-    _require(seq_lens.device == query.device and seq_lens.dtype == torch.int32
+    _require(seq_lens.get_device() == device and seq_lens.dtype is torch.int32
              and seq_lens.dim() == 1 and seq_lens.is_contiguous(),
              "Contiguous INT32 sequence lengths required")
-    _require(block_table.device == query.device and block_table.dtype == torch.int32
+    _require(block_table.get_device() == device and block_table.dtype is torch.int32
              and block_table.dim() == 2 and block_table.stride(1) == 1
-             and block_table.size(0) >= seq_lens.numel(),
+             and block_table.size(0) >= requests,
              "INT32 page table with packed rows required")
+    return strides
 
 
 def attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tensor,
@@ -167,34 +202,35 @@ def attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_ca
     in the reference) lets a caller reuse one device buffer of
     ``attention_workspace_bytes(...)`` bytes, e.g. across graph replays.
     """
-    key_rotation_ptr, value_rotation_ptr = _validate_packed_inputs(
+    strides, key_rotation_ptr, value_rotation_ptr = _validate_packed_inputs(
         query, key, value, kv_cache, output, query_start_loc, seq_lens, block_table, key_rotation, value_rotation,
         key_mean, records, reference_mode, loop_index)
-    _call_packed_attention(_lib.lib().rq_attention, query, key, value, kv_cache, output, query_start_loc,
+    _call_packed_attention(_lib.lib().rq_attention, strides, query, key, value, kv_cache, output, query_start_loc,
                            seq_lens, block_table, key_rotation_ptr, value_rotation_ptr, key_mean, records,
                            reference_mode, anchor_index, loop_index, workspace)
 
 
 def _validate_packed_inputs(query, key, value, kv_cache, output, query_start_loc, seq_lens, block_table,
                             key_rotation, value_rotation, key_mean, records, reference_mode, loop_index):
-    _validate_attention_inputs(query, key, value, output, query_start_loc, seq_lens, block_table)
-    heads, head_dim = query.size(1), query.size(2)
-    _require(kv_cache.device == query.device and kv_cache.dtype == torch.uint8
+    strides = _validate_attention_inputs(query, key, value, output, query_start_loc, seq_lens, block_table)
+    _, heads, head_dim = query.shape
+    device = query.get_device()
+    _require(kv_cache.get_device() == device and kv_cache.dtype is torch.uint8
              and kv_cache.is_contiguous() and kv_cache.dim() == 5 and kv_cache.size(0) == 2
              and kv_cache.size(2) == heads,
              "Contiguous UINT8 KV cache on the query device required")
     if key_mean is not None:
-        _require(key_mean.device == query.device and key_mean.dtype == torch.float32
+        _require(key_mean.get_device() == device and key_mean.dtype is torch.float32
                  and key_mean.is_contiguous() and key_mean.data_ptr() % 16 == 0
                  and key_mean.numel() == len(records) * heads * head_dim,
                  "16-byte aligned contiguous FP32 key mean with matching dimensions required")
-    value_rotation_ptr = _rotation_pointer(value_rotation, query.device, heads, head_dim)
-    key_rotation_ptr = _rotation_pointer(key_rotation, query.device, heads, head_dim)
+    value_rotation_ptr = _rotation_pointer(value_rotation, device, heads, head_dim)
+    key_rotation_ptr = _rotation_pointer(key_rotation, device, heads, head_dim)
     _require(key_rotation_ptr is None or key_rotation_ptr % 16 == 0,
              "16-byte aligned key rotation required for asynchronous copies")
     _require(0 <= loop_index < len(records), "Invalid loop index")
     _require(reference_mode in _MODES, f"Unknown packed reference mode: {reference_mode}")
-    return key_rotation_ptr, value_rotation_ptr
+    return strides, key_rotation_ptr, value_rotation_ptr
 
 
 def packed_prefill_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
@@ -215,34 +251,32 @@ def packed_prefill_attention(query: torch.Tensor, key: torch.Tensor, value: torc
     arguments and validation are those of ``attention`` (head_dim 96 or
     128, anchor or adjacent mode); a request may have no new rows.
     """
-    key_rotation_ptr, value_rotation_ptr = _validate_packed_inputs(
+    strides, key_rotation_ptr, value_rotation_ptr = _validate_packed_inputs(
         query, key, value, kv_cache, output, query_start_loc, seq_lens, block_table, key_rotation, value_rotation,
         key_mean, records, reference_mode, loop_index)
-    _call_packed_attention(_lib.lib().rq_packed_prefill_attention, query, key, value, kv_cache, output,
+    _call_packed_attention(_lib.lib().rq_packed_prefill_attention, strides, query, key, value, kv_cache, output,
                            query_start_loc, seq_lens, block_table, key_rotation_ptr, value_rotation_ptr, key_mean,
                            records, reference_mode, anchor_index, loop_index, workspace)
 
 
-def _call_packed_attention(function, query, key, value, kv_cache, output, query_start_loc, seq_lens, block_table,
-                           key_rotation_ptr, value_rotation_ptr, key_mean, records, reference_mode, anchor_index,
-                           loop_index, workspace):
-    heads, head_dim = query.size(1), query.size(2)
-    rows = query.size(0)
+def _call_packed_attention(function, strides, query, key, value, kv_cache, output, query_start_loc, seq_lens,
+                           block_table, key_rotation_ptr, value_rotation_ptr, key_mean, records, reference_mode,
+                           anchor_index, loop_index, workspace):
+    rows, heads, head_dim = query.shape
+    _, num_blocks, _, page_tokens, page_width = kv_cache.shape
     max_pages = block_table.size(1)
-    needed = attention_workspace_bytes(rows, heads, head_dim, max_pages, kv_cache.size(3))
-    ws = _workspace(workspace, needed, query.device)
-    bits, groups = _schedule(records)
-    with torch.cuda.device(query.device):
+    device = query.get_device()
+    ws = _workspace(workspace, attention_workspace_bytes(rows, heads, head_dim, max_pages, page_tokens), query.device)
+    schedule = _schedule(records)
+    with _on_device(device):
         status = function(
-            query.data_ptr(), query.stride(0), key.data_ptr(), key.stride(0), value.data_ptr(),
-            value.stride(0), output.data_ptr(), output.stride(0), rows, heads, head_dim,
-            kv_cache.data_ptr(), kv_cache.size(1), kv_cache.size(3), kv_cache.size(4),
-            query_start_loc.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(),
-            block_table.data_ptr(), block_table.stride(0), max_pages, key_rotation_ptr,
-            value_rotation_ptr, key_mean.data_ptr() if key_mean is not None else None,
-            len(records), ctypes.cast(bits, ctypes.c_void_p), ctypes.cast(groups, ctypes.c_void_p),
+            query.data_ptr(), strides[0], key.data_ptr(), strides[1], value.data_ptr(), strides[2],
+            output.data_ptr(), strides[3], rows, heads, head_dim, kv_cache.data_ptr(), num_blocks, page_tokens,
+            page_width, query_start_loc.data_ptr(), seq_lens.data_ptr(), seq_lens.numel(), block_table.data_ptr(),
+            block_table.stride(0), max_pages, key_rotation_ptr, value_rotation_ptr,
+            key_mean.data_ptr() if key_mean is not None else None, len(records), schedule[2], schedule[3],
             _MODES[reference_mode], int(anchor_index), int(loop_index), ws.data_ptr(),
-            ws.numel() * ws.element_size(), _stream(query.device))
+            ws.numel() * ws.element_size(), _stream(device))
     _lib.check(status)
 
 
@@ -267,15 +301,16 @@ def dequantize(kv_cache: torch.Tensor, slots: torch.Tensor, head_dim: int,
     _require(reference_mode in _MODES, f"Unknown packed reference mode: {reference_mode}")
     key_out = torch.empty((slots.numel(), heads, head_dim), dtype=torch.bfloat16, device=kv_cache.device)
     value_out = torch.empty_like(key_out)
-    bits, groups = _schedule(records)
-    with torch.cuda.device(kv_cache.device):
+    schedule = _schedule(records)
+    device = kv_cache.get_device()
+    with _on_device(device):
         status = _lib.lib().rq_dequantize(
             kv_cache.data_ptr(), kv_cache.size(1), heads, kv_cache.size(3), kv_cache.size(4),
             slots.data_ptr(), slots.numel(), head_dim,
             key_mean.data_ptr() if key_mean is not None else None, len(records),
-            ctypes.cast(bits, ctypes.c_void_p), ctypes.cast(groups, ctypes.c_void_p),
+            schedule[2], schedule[3],
             _MODES[reference_mode], int(anchor_index), int(loop_index), key_out.data_ptr(),
-            value_out.data_ptr(), _stream(kv_cache.device))
+            value_out.data_ptr(), _stream(device))
     _lib.check(status)
     return key_out, value_out
 
@@ -295,13 +330,14 @@ def paged_attention_bf16(query: torch.Tensor, key: torch.Tensor, value: torch.Te
     max_pages = block_table.size(1)
     needed = attention_workspace_bytes(rows, heads, head_dim, max_pages, cache.size(3))
     ws = _workspace(workspace, needed, query.device)
-    with torch.cuda.device(query.device):
+    device = query.get_device()
+    with _on_device(device):
         status = _lib.lib().rq_paged_attention_bf16(
             query.data_ptr(), query.stride(0), key.data_ptr(), key.stride(0), value.data_ptr(),
             value.stride(0), output.data_ptr(), output.stride(0), rows, heads, head_dim,
             cache.data_ptr(), cache.size(1), cache.size(3), query_start_loc.data_ptr(),
             seq_lens.data_ptr(), seq_lens.numel(), block_table.data_ptr(), block_table.stride(0),
-            max_pages, ws.data_ptr(), ws.numel() * ws.element_size(), _stream(query.device))
+            max_pages, ws.data_ptr(), ws.numel() * ws.element_size(), _stream(device))
     _lib.check(status)
 
 
@@ -329,32 +365,32 @@ def flash_attn_varlen_func(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ma
              "Only dropout-free, unwindowed attention without ALiBi, softcap, paged K/V or returned "
              "LSE is supported")
     cu_seqlens_k = cu_seqlens_q if cu_seqlens_k is None else cu_seqlens_k
-    for tensor in (q, k, v):
-        _validate_bf16_token_tensor(tensor)
-    _require(k.device == q.device and v.device == q.device and k.shape == v.shape
-             and k.size(2) == q.size(2), "Q/K/V must share device and head_dim; K and V must match")
+    (q_shape, q_stride), (k_shape, k_stride), (v_shape, v_stride) = map(_validate_bf16_token_tensor, (q, k, v))
+    device = q.get_device()
+    _require(k.get_device() == device and v.get_device() == device and k_shape == v_shape
+             and k_shape[2] == q_shape[2], "Q/K/V must share device and head_dim; K and V must match")
     if out is None:
         out = torch.empty_like(q)
-    _validate_bf16_token_tensor(out)
-    _require(out.device == q.device and out.shape == q.shape, "out must match q")
+    out_shape, out_stride = _validate_bf16_token_tensor(out)
+    _require(out.get_device() == device and out_shape == q_shape, "out must match q")
     for seqlens in (cu_seqlens_q, cu_seqlens_k):
-        _require(seqlens.device == q.device and seqlens.dtype == torch.int32 and seqlens.dim() == 1
+        _require(seqlens.get_device() == device and seqlens.dtype is torch.int32 and seqlens.dim() == 1
                  and seqlens.is_contiguous(), "Contiguous INT32 cu_seqlens on the Q device required")
     _require(cu_seqlens_q.numel() == cu_seqlens_k.numel() and cu_seqlens_q.numel() >= 1,
              "cu_seqlens_q and cu_seqlens_k must describe the same sequences")
-    head_dim = q.size(2)
+    _, heads_q, head_dim = q_shape
     scale = head_dim ** -0.5 if softmax_scale is None else float(softmax_scale)
     batch = cu_seqlens_q.numel() - 1
     same = cu_seqlens_q.data_ptr() == cu_seqlens_k.data_ptr()
-    needed = _lib.lib().rq_prefill_workspace_bytes(batch, q.size(1), head_dim, int(max_seqlen_q),
+    needed = _lib.lib().rq_prefill_workspace_bytes(batch, heads_q, head_dim, int(max_seqlen_q),
                                                    int(max_seqlen_k), 1 if causal else 0, 1 if same else 0)
     workspace = torch.empty(max(needed, 1), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(device):
         status = _lib.lib().rq_prefill_attention(
-            q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), out.data_ptr(),
-            out.stride(0), q.size(1), k.size(1), head_dim, cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
-            batch, int(max_seqlen_q), int(max_seqlen_k), scale, 1 if causal else 0, workspace.data_ptr(),
-            workspace.numel(), _stream(q.device))
+            q.data_ptr(), q_stride, k.data_ptr(), k_stride, v.data_ptr(), v_stride, out.data_ptr(), out_stride,
+            heads_q, k_shape[1], head_dim, cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(), batch,
+            int(max_seqlen_q), int(max_seqlen_k), scale, 1 if causal else 0, workspace.data_ptr(),
+            workspace.numel(), _stream(device))
     _lib.check(status)
     return out
 
