@@ -35,7 +35,7 @@ constexpr int kUnits = kChunkUnit / 16;  // units per step, one per wave
 static_assert(kUnits == kStreamWaves && kChunkTileRows == 32 * kStreamWaves, "one unit and 32 rows per wave");
 
 // Tiles of T tokens: K rows of KS halves, V rows of VROW halves whose 32-channel
-// chunks sit at q ^ (token % 4) at D = 128 (see Geometry in multirow.hip).
+// chunks sit at q ^ (token % 4) at D = 128 (see Geometry in rq_multirow.h).
 template <int D, int T>
 struct Tile {
     static constexpr int KS = D + 8;

@@ -497,9 +497,9 @@ __device__ __forceinline__ void finish_merge(__amdgpu_buffer_rsrc_t entries, uin
 // request's new tokens j <= row for the rows row0 .. row0 + TR - 1.  Wave w
 // takes the 32-key tiles w, w + 4, ..: raw BF16 K and V into its own LDS tile,
 // S^T = K Q^T and O^T += V^T P^T as in the stream, with the probabilities as
-// two BF16 parts (high and the rest: 16 significant bits, so the output's
-// error against float64 stays the BF16 rounding of the output, 1.9e-3, where
-// FP32 probabilities had it).  The waves' (m, l, O) and the thread's history
+// three BF16 parts (8 significant bits each, so all 24 of the FP32 value
+// multiply V, whose BF16 values and products with a part are exact in FP32; a
+// third part instead of two takes 1.6 us more of a 100 us call).  The waves' (m, l, O) and the thread's history
 // (m, l, acc; row tid / 8, channels 16 (tid % 8)..+15) then meet in LDS.
 // `shift` is the mean shift of that row.  On the vector units (scores and
 // values in FP32, 32 keys per step for the whole workgroup) the finish of 2
@@ -587,15 +587,11 @@ __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, i
         const float base = new_max == -__builtin_inff() ? 0.f : new_max;
         const float rescale = __builtin_amdgcn_exp2f(running_max - base);
         running_max = new_max;
-        Bf16x8 high[2], low[2];
         float tile_sum = 0.f;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const float w = __builtin_amdgcn_exp2f(s[e] - base);
-            const __bf16 h = (__bf16)w;
-            high[e >> 3][e & 7] = h;
-            low[e >> 3][e & 7] = (__bf16)(w - (float)h);
-            tile_sum += w;
+            s[e] = __builtin_amdgcn_exp2f(s[e] - base);
+            tile_sum += s[e];
         }
         running_sum = running_sum * rescale + tile_sum + __shfl_xor(tile_sum, 32);
         if (!__all(rescale == 1.0f)) {
@@ -606,6 +602,15 @@ __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, i
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
+            Bf16x8 high, middle, low;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float w = s[8 * j + e];
+                high[e] = (__bf16)w;
+                const float rest = w - (float)high[e];
+                middle[e] = (__bf16)rest;
+                low[e] = (__bf16)(rest - (float)middle[e]);
+            }
             const uint16_t* v_rows = v_tile + 16 * j * G::VROW;
 #pragma unroll
             for (int t = 0; t < Quarters; ++t) {
@@ -613,8 +618,9 @@ __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, i
                 const Short4 lo = read_transposed(v_rows + at);
                 const Short4 hi = read_transposed(v_rows + 8 * G::VROW + at);
                 const Bf16x8 a = __builtin_bit_cast(Bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                out[t] = mfma(a, high[j], out[t]);
-                out[t] = mfma(a, low[j], out[t]);
+                out[t] = mfma(a, high, out[t]);
+                out[t] = mfma(a, middle, out[t]);
+                out[t] = mfma(a, low, out[t]);
             }
         }
         wave_sync();  // the next tile overwrites this one
