@@ -22,7 +22,7 @@
 //
 // Measured (2 requests of 4518 and 6000 tokens x 509 rows x 16 heads, causal,
 // residual loop / anchor loop): 289 / 250 us per call on 32-row tiles with the
-// live tokens on the vector units; here 110 / 100 us (stream 85 / 77, finish 25).
+// live tokens on the vector units; here 112 / 102 us (stream 85 / 77, finish 27).
 #include "rq_multirow.h"
 
 namespace rq {

@@ -499,11 +499,12 @@ __device__ __forceinline__ void finish_merge(__amdgpu_buffer_rsrc_t entries, uin
 // S^T = K Q^T and O^T += V^T P^T as in the stream, with the probabilities as
 // three BF16 parts (8 significant bits each, so all 24 of the FP32 value
 // multiply V, whose BF16 values and products with a part are exact in FP32; a
-// third part instead of two takes 1.6 us more of a 100 us call).  The waves' (m, l, O) and the thread's history
-// (m, l, acc; row tid / 8, channels 16 (tid % 8)..+15) then meet in LDS.
-// `shift` is the mean shift of that row.  On the vector units (scores and
-// values in FP32, 32 keys per step for the whole workgroup) the finish of 2
-// requests x 509 rows x 16 heads took 124 us, here 25 us.
+// third part instead of two takes 1.6 us more of a 100 us call).  The waves'
+// (m, l, O) and the thread's history (m, l, acc; row tid / 8, channels
+// 16 (tid % 8)..+15) then meet in LDS.  `shift` is the mean shift of that row.
+// On the vector units (scores and values in FP32, 32 keys per step for the
+// whole workgroup) the finish of 2 requests x 509 rows x 16 heads took 124 us,
+// here 27 us.
 template <int D, int TR>
 __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, int first, int row0, int n, float shift,
                                             float& m, float& l, float (&acc)[16], uint8_t* lds) {
