@@ -592,8 +592,11 @@ def run_multiquery(args):
     tile_rows = 16 if rows_per <= 16 else 32
     tiles = batch * heads * ((history + 31) // 32) * ((rows_per + tile_rows - 1) // tile_rows)
     mfma_flop = tiles * 2 * 2 * 32 * tile_rows * dim
-    kernel = (f"multirow_chain_kernel<{dim},16,{tile_rows},4>" if adjacent else
-              f"multirow_stream_kernel<{dim},16,{tile_rows},true,...>") + " + multirow_finish_kernel"
+    if rows_per >= 48 and batch <= 64:
+        kernel = ("chunk_chain_kernel" if adjacent else "chunk_stream_kernel") + " + chunk_finish_kernel"
+    else:
+        kernel = (f"multirow_chain_kernel<{dim},16,{tile_rows},4>" if adjacent else
+                  f"multirow_stream_kernel<{dim},16,{tile_rows},true,...>")
     result = {
         "metric": "paged decode-attn µs/step + achieved HBM GB/s (% peak), INT2/INT4 vs bf16, 1 GPU",
         "value": step_bytes / (m["us_per_step"] * 1e-6) / 1e9,
