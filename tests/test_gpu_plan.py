@@ -120,3 +120,36 @@ def test_planned_decode_replays(device):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out.view(torch.int16), want.view(torch.int16)), lengths
+
+
+@pytest.mark.parametrize("rows", [[3, 5, 2], [60, 50, 40]], ids=["rows", "chunks"])
+def test_captured_rows_replay(device, rows):
+    """Several rows per request, captured: every replay, with other lengths in
+    place of the captured ones, equals the eager call."""
+    d = make_decode([2800, 400, 130], 2, 128, OURO_G32, seed=6, rows_per_request=rows)
+    g = d.group
+    cache = torch.zeros(g.cache_shape, dtype=torch.uint8, device=device)
+    kr, vr, km = g.device_args(device)
+    rq.quantize([(a.to(device), b.to(device)) for a, b in g.pairs], cache, g.slots.to(device), kr, vr, km, g.records,
+                g.mode, g.anchor, g.coefficient)
+    q, k, v = (t.to(device) for t in (d.query, d.key, d.value))
+    starts, lens, table = (t.to(device) for t in (d.query_start_loc, d.seq_lens, d.table))
+    out, want = torch.empty_like(q), torch.empty_like(q)
+
+    def call(to):
+        rq.packed_prefill_attention(q, k, v, cache, to, starts, lens, table, kr, vr, km, g.records, g.mode, g.anchor, 1)
+
+    call(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    captured = lens.tolist()
+    for lengths in (captured, [700, captured[1], rows[2]], [captured[0], rows[1] + 1, captured[2]]):
+        lens.copy_(torch.tensor(lengths, dtype=torch.int32))
+        call(want)
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out.view(torch.int16), want.view(torch.int16)), lengths
