@@ -493,6 +493,46 @@ __device__ __forceinline__ void finish_merge(__amdgpu_buffer_rsrc_t entries, uin
     }
 }
 
+// The causal live tokens of the thread's row (tid / 8) one by one, every product
+// in FP32 (live_tokens, where its sums are not finite).
+template <int D, int TR>
+__device__ __forceinline__ void live_tokens_fp32(const MultiRowParams& p, int head, int first, int row0, int n,
+                                                 float shift, float& m, float& l, float (&acc)[16]) {
+    const int r = threadIdx.x >> 3, part = threadIdx.x & 7;
+    const bool part_active = part < D / 16;
+    const int row = r < TR && row0 + r < n ? row0 + r : -1;  // (sees no token)
+    const int64_t channels = (int64_t)head * D + 16 * (part_active ? part : 0);
+    const bool q_vec = aligned_rows(p.query, p.query_stride), k_vec = aligned_rows(p.key, p.key_stride),
+               v_vec = aligned_rows(p.value, p.value_stride);
+    uint4 w[2];
+    float q[16];
+    load_halves16(p.query + ((int64_t)first + max(row, 0)) * p.query_stride + channels, q_vec, w);
+    widen_bf16(w[0], q);
+    widen_bf16(w[1], q + 8);
+    const int live_end = min(n, row0 + TR);
+    for (int j = 0; j < live_end; ++j) {
+        float k[16], v[16];
+        load_halves16(p.key + ((int64_t)first + j) * p.key_stride + channels, k_vec, w);
+        widen_bf16(w[0], k);
+        widen_bf16(w[1], k + 8);
+        load_halves16(p.value + ((int64_t)first + j) * p.value_stride + channels, v_vec, w);
+        widen_bf16(w[0], v);
+        widen_bf16(w[1], v + 8);
+        float dot = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dot = fmaf(q[i], k[i], dot);
+        const float score = row8_sum(part_active ? dot : 0.f) * kScoreScale<D> - shift;
+        if (j > row) continue;
+        const float new_max = fmaxf(m, score);
+        const float keep = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - new_max);
+        const float weight = __builtin_amdgcn_exp2f(score - new_max);
+        m = new_max;
+        l = fmaf(l, keep, weight);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = fmaf(weight, v[i], acc[i] * keep);
+    }
+}
+
 // Causal live tokens on MFMA, by the four waves of the tile's workgroup: the
 // request's new tokens j <= row for the rows row0 .. row0 + TR - 1.  Wave w
 // takes the 32-key tiles w, w + 4, ..: raw BF16 K and V into its own LDS tile,
@@ -505,6 +545,10 @@ __device__ __forceinline__ void finish_merge(__amdgpu_buffer_rsrc_t entries, uin
 // On the vector units (scores and values in FP32, 32 keys per step for the
 // whole workgroup) the finish of 2 requests x 509 rows x 16 heads took 124 us,
 // here 27 us.
+// A part may be zero or of the other sign, and the tokens that a row does not
+// see take part as 0 x V: a V that is not finite makes sums NaN that hold an
+// infinity or do not hold that V.  A wave with such a sum in its eight rows
+// takes their tokens again (live_tokens_fp32).
 template <int D, int TR>
 __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, int first, int row0, int n, float shift,
                                             float& m, float& l, float (&acc)[16], uint8_t* lds) {
@@ -648,18 +692,28 @@ __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, i
         total_max = fmaxf(total_max, m_w[w]);
     }
     const float keep = m == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m - total_max);
-    m = total_max;
-    l *= keep;
+    float total = l * keep, sums[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] *= keep;
+    for (int i = 0; i < 16; ++i) sums[i] = acc[i] * keep;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
         const float weight = m_w[w] == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m_w[w] - total_max);
-        l = fmaf(merge_ml[(w * 32 + r) * 2 + 1], weight, l);
+        total = fmaf(merge_ml[(w * 32 + r) * 2 + 1], weight, total);
         const float* src = &merge_o[(w * 32 + r) * MS + 16 * chunk];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = fmaf(src[i], weight, acc[i]);
+        for (int i = 0; i < 16; ++i) sums[i] = fmaf(src[i], weight, sums[i]);
     }
+    float zero = 0.f;  // stays 0 over finite sums, else NaN
+#pragma unroll
+    for (int i = 0; i < 16; ++i) zero = fmaf(sums[i], 0.f, zero);
+    if (__any(r < TR && row0 + r < n && !(zero == 0.f))) {
+        live_tokens_fp32<D, TR>(p, head, first, row0, n, shift, m, l, acc);
+        return;
+    }
+    m = total_max;
+    l = total;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = sums[i];
 }
 
 template <int D, int TR>

@@ -251,3 +251,42 @@ def test_multirow_agrees_with_per_row_kernels(oracle, device, dim, mode, records
                              g.mode, g.anchor, loop)
                 single = out.float().cpu().numpy()[0]
                 assert np.abs(multi[i] - single).max() <= MAX_ABS, (loop, i)
+
+
+@pytest.mark.parametrize("case", [([300, 37, 90], [33, 8, 64], 128, 16, "anchor"), ([220, 50], [40, 7], 96, 32, "adjacent"),
+                                  ([400, 130], [97, 70], 128, 16, "adjacent"), ([257], [257], 96, 16, "anchor"),
+                                  ([60, 40], [5, 3], 128, 32, "anchor")],
+                         ids=lambda c: f"n{sum(c[1])}-d{c[2]}-pt{c[3]}-{c[4]}")
+def test_causal_values_that_are_not_finite(oracle, device, case):
+    """New tokens whose values hold infinities and NaN: the rows that see one
+    give what its float32 sum gives, the rows that do not are as accurate as
+    ever (calls of 32-row tiles, 16-row tiles and 256-row tiles)."""
+    lengths, rows, dim, pt, mode = case
+    print(f"[case] values that are not finite: {case}", flush=True)
+    records = ADJACENT_G32 if mode == "adjacent" else OURO_G32
+    d = make_decode(lengths, 2, dim, records, seed=sum(lengths), page_tokens=pt, mode=mode,
+                    anchor=0 if mode == "adjacent" else None, rows_per_request=rows)
+    cache_np = d.group.oracle_cache(oracle)
+    cache = torch.from_numpy(cache_np).to(device)
+    first = 0
+    for n in rows:
+        middle = first + n // 2
+        d.value[first, 0, 3] = float("inf")           # every row of the request sees it
+        d.value[middle, 0, 5] = float("-inf")
+        d.value[middle, 1, dim - 1] = float("inf")
+        d.value[first + n - 1, 1, dim - 1] = float("-inf")  # both signs: NaN in the last row
+        d.value[first + n - 1, 1, 40] = float("nan")
+        first += n
+    for loop in (1, 3):
+        want = _oracle(oracle, d, cache_np, loop, True)
+        got = _run(d, device, cache, loop, True)
+        finite = np.isfinite(want)
+        assert 0 < (~finite).sum() < want.size // 4
+        special = ~finite
+        assert np.array_equal(np.isnan(got), np.isnan(want)), loop
+        assert np.array_equal(got[special & ~np.isnan(want)], want[special & ~np.isnan(want)]), loop
+        # (An ulp of values of magnitude 4 and more exceeds the bar; a request's first rows average few values.)
+        expected = _bf16(want[finite])
+        err = np.abs(got[finite] - expected)
+        print(f"[case]   loop {loop}: max {err.max():.3g} mean {err.mean():.3g}", flush=True)
+        assert (err <= np.maximum(MAX_ABS, np.abs(expected) * 2.0 ** -7)).all() and err.mean() <= MEAN_ABS
