@@ -236,7 +236,7 @@ uint64_t next_call_tag() {
         std::random_device source;
         return ((uint64_t)source() << 32) | source();
     }()};
-    constexpr uint64_t kMask = (1ull << 56) - 1;
+    constexpr uint64_t kMask = ~0ull >> rq::kArrivalBits;
     uint64_t tag;
     do tag = counter.fetch_add(1, std::memory_order_relaxed) & kMask;
     while (tag == 0);
@@ -650,6 +650,7 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
             plan_chunk(m, std::min(workspace_bytes, full_bytes));
         else
             plan_multirow(m, splits, std::min(workspace_bytes, full_bytes));
+        static_assert(rq::kMaxArrivals >= 65535, "the splits of one row tile, planned ones included");
         if ((int64_t)splits * row_tiles > 65535 || requests > (int64_t)INT32_MAX || rows > (int64_t)INT32_MAX)
             return fail(RQ_EINVAL, "Too many rows for one multi-row attention launch");
         hipEvent_t begin = nullptr, end = nullptr;

@@ -143,6 +143,11 @@ constexpr int kPrepPlanes = 64;    // 4 nibble planes x up to 16 words (each ord
 constexpr int kPrepFloats = kPrepScalars + kPrepQuery + 2 * kPrepPlanes;
 constexpr int kMaxSplits = 64;
 
+// Arrival words (rq_plan.h): the count's bits below the call's tag, and the
+// most splits of one item that it counts.
+constexpr int kArrivalBits = 16;
+constexpr int kMaxArrivals = (1 << kArrivalBits) - 1;
+
 struct AttentionParams {
     const uint16_t* query;
     int64_t query_stride;
@@ -176,7 +181,7 @@ struct AttentionParams {
     int32_t* row_request;  // BF16 baseline: workspace [rows]
     float* prep;           // BF16 baseline: workspace [rows, heads, kPrepFloats]
     uint64_t* arrivals;    // packed decode: workspace [rows, heads], tagged arrival counts (rq_plan.h)
-    uint64_t call_tag;     // of this call (56 bits)
+    uint64_t call_tag;     // of this call (48 bits)
     float* partials;       // workspace: packed decode [heads, items, D + 2], BF16 [rows, heads, splits, D + 2]
     int splits;            // of every row: BF16 baseline, packed decode of equal lengths or past kPlanRequests
     // Packed decode (decode_item in attention.hip):
@@ -257,7 +262,7 @@ struct MultiRowParams {
     int64_t resident;     // set by the launch: stream workgroups the device holds at once
     int64_t entries;      // partials per head
     float* partials;      // workspace [heads, entries, kMultiRowEntry]; a request's entries: [row, split]
-    uint64_t call_tag;    // of this call (56 bits, rq_plan.h)
+    uint64_t call_tag;    // of this call (48 bits, rq_plan.h)
 };
 template <int D>
 hipError_t launch_multirow(const MultiRowParams& p, hipStream_t stream);

@@ -15,6 +15,7 @@
 #pragma once
 
 #include "rq_device.h"
+#include "rq_kernels.h"
 
 namespace rq {
 
@@ -209,15 +210,16 @@ __device__ __forceinline__ int split_begin(int length, int split, int splits) {
 //
 // The workgroup that finishes last of a split item merges, so the splits of
 // an item count themselves in one 64-bit word of the call's workspace: the
-// upper 56 bits hold the call's tag, the lower 8 the arrivals so far.  Every
-// split first makes sure that the word carries the tag (tag_arrivals, early
+// upper 48 bits hold the call's tag, the lower 16 the arrivals so far (a long
+// page table makes several hundred splits of a request's several rows: the
+// host takes at most kMaxArrivals).  Every split first makes sure that the word carries the tag (tag_arrivals, early
 // in its prologue: a word whose tag is not this call's is replaced by an
 // empty one), so the word needs no clearing launch before the call (5 us with
 // its gap) and the arrival itself is one atomic add.  The last arrival writes
 // 0, so a replay of a captured call, which repeats the tag, starts from an
 // untagged word as well.  Tags come from a process-wide counter with a random
 // start (next_call_tag in capi.hip): stale memory equals a call's tag with
-// probability 2^-56.
+// probability 2^-48.
 
 // The word as an early load of thread 0 saw it (issued where its latency is hidden).
 __device__ __forceinline__ uint64_t peek_arrivals(const uint64_t* word) {
@@ -228,8 +230,8 @@ __device__ __forceinline__ uint64_t peek_arrivals(const uint64_t* word) {
 // A failed exchange means that the word has changed since `seen`, which only
 // another split of this call does, and only to a tagged word.
 __device__ __forceinline__ void tag_arrivals(uint64_t* word, uint64_t tag, uint64_t seen) {
-    if ((seen >> 8) != tag)
-        (void)__hip_atomic_compare_exchange_strong(word, &seen, tag << 8, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+    if ((seen >> kArrivalBits) != tag)
+        (void)__hip_atomic_compare_exchange_strong(word, &seen, tag << kArrivalBits, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -241,7 +243,7 @@ __device__ __forceinline__ bool arrive_last_tagged(uint64_t* word, int expected,
     __syncthreads();
     if (threadIdx.x == 0) {
         const uint64_t before = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool last = (int)(before & 0xff) == expected - 1;
+        const bool last = (int)(before & kMaxArrivals) == expected - 1;
         if (last) __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         *lds_flag = last;
     }

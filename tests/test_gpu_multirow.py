@@ -290,3 +290,39 @@ def test_causal_values_that_are_not_finite(oracle, device, case):
         err = np.abs(got[finite] - expected)
         print(f"[case]   loop {loop}: max {err.max():.3g} mean {err.mean():.3g}", flush=True)
         assert (err <= np.maximum(MAX_ABS, np.abs(expected) * 2.0 ** -7)).all() and err.mean() <= MEAN_ABS
+
+
+@pytest.mark.parametrize("lengths,rows,page_tokens,mode", [([34000], [3], 16, "anchor"), ([67800], [2], 32, "adjacent"),
+                                                           ([50, 33, 2] * 22, [2] * 66, 16, "anchor")],
+                         ids=["one-request", "adjacent", "past-the-plan"])
+def test_page_table_of_several_hundred_splits(oracle, device, lengths, rows, page_tokens, mode):
+    """A page table of 262 000 columns takes 257 splits (a split's block ids
+    fit its 1024-entry list), whatever part of it the requests fill: all of
+    them arrive before the output is merged, twice on one workspace."""
+    print(f"[case] wide page table: {len(lengths)} requests of {lengths[0]} tokens, {mode}", flush=True)
+    d = make_decode([600] * min(len(lengths), 3), 1, 128, ADJACENT_G32 if mode == "adjacent" else OURO_G32, seed=41,
+                    page_tokens=page_tokens, mode=mode, anchor=0 if mode == "adjacent" else None,
+                    rows_per_request=rows[:min(len(lengths), 3)])
+    g = d.group
+    cache_np = g.oracle_cache(oracle)
+    cache = torch.from_numpy(cache_np).to(device)
+    # The histories go round the filled blocks (600 tokens of each row of the table).
+    blocks = d.table[:, :600 // page_tokens]
+    d.table = blocks.repeat(len(lengths) // blocks.size(0), 262_000 // blocks.size(1) + 1)[:, :262_000].contiguous()
+    d.lengths, d.rows_per_request = lengths, rows
+    generator = torch.Generator().manual_seed(42)
+    d.query, d.key, d.value = (torch.randn((sum(rows), 1, 128), generator=generator).to(torch.bfloat16) for _ in range(3))
+    q, k, v = (t.to(device) for t in (d.query, d.key, d.value))
+    starts, lens, table = (t.to(device) for t in (d.query_start_loc, d.seq_lens, d.table))
+    kr, vr, km = g.device_args(device)
+    size = rq.ops.attention_workspace_bytes(q.size(0), 1, 128, table.size(1), page_tokens)
+    workspace = torch.full((size,), 0xFF, dtype=torch.uint8, device=device)
+    for loop in (1, 2):
+        want = _bf16(_oracle(oracle, d, cache_np, loop, False))
+        for _ in range(2):
+            out = torch.full_like(q, float("nan"))
+            rq.attention(q, k, v, cache, out, starts, lens, table, kr, vr, km, g.records, g.mode, g.anchor, loop,
+                         workspace=workspace)
+            err = np.abs(out.float().cpu().numpy() - want)
+            print(f"[case]   loop {loop}: max {err.max():.3g} mean {err.mean():.3g}", flush=True)
+            assert err.max() <= MAX_ABS and err.mean() <= MEAN_ABS, (loop, err.max(), err.mean())
