@@ -93,7 +93,11 @@ size_t rq_attention_workspace_bytes(int64_t rows, int heads, int head_dim, int64
  *   query_start_loc[b] <= i < query_start_loc[b+1] and attends to
  *   seq_lens[b]-1 history tokens read through block_table[b][t/page_tokens].
  * block_table: INT32 [>= requests, max_pages], row stride block_table_stride.
- * workspace: device memory of at least rq_attention_workspace_bytes(...).
+ * workspace: device memory of rq_attention_workspace_bytes(...).  A smaller
+ *   one that holds what the call's route requires (see rq_attention_noalloc)
+ *   is taken as well; several rows per request may then be split less.
+ * How a request's history is split, and with it the rounding of its output,
+ * follows from the lengths of all requests of the call.
  */
 int rq_attention(const void* query, int64_t query_stride, const void* key, int64_t key_stride,
                  const void* value, int64_t value_stride, void* output, int64_t output_stride,
@@ -135,15 +139,17 @@ int rq_packed_prefill_attention(const void* query, int64_t query_stride, const v
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference, whose
  * attention() allocates its temporaries per call (attention/launch.cuh:85-98).
- * Same arguments, semantics, kernels and results as rq_attention; the
- * workspace is a static device array of RQ_ATTENTION_NOALLOC_MAX_BYTES per
- * GPU, held until the process ends.  A call whose route needs more returns
- * RQ_ENOSPACE before any device work: the per-row decode kernels need
+ * Same arguments, semantics, kernels and results as rq_attention with a
+ * workspace of rq_attention_workspace_bytes(...); the workspace is a static
+ * device array of 48 MiB per GPU, held until the process ends.  A call whose
+ * route requires more than RQ_ATTENTION_NOALLOC_MAX_BYTES returns RQ_ENOSPACE
+ * before any device work: the per-row decode kernels require
  * (272 + 130 x splits) x 4 bytes per (row, head), about 5 000 (row, head)
  * pairs at one split; the multi-row kernels (2 or more rows per request)
  * (132 x splits + 1) x 4 bytes, about 2 000 pairs at eight splits.
- * (rq_attention_workspace_bytes covers both routes, so it may exceed the
- * scratch for a call that still fits.)
+ * (rq_attention_workspace_bytes covers both routes and what a call's plan may
+ * use beyond its required bytes, so it may exceed the limit for a call that
+ * still fits.)
  * Every noalloc call on one GPU shares that array.  Eager calls are ordered
  * by the library, across streams and host threads: a call on another stream
  * than the previous call first makes its stream wait for the previous

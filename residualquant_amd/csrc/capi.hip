@@ -464,6 +464,13 @@ static size_t attention_workspace_total(int64_t rows, int heads, int head_dim, i
     return total;
 }
 
+// Static scratch of rq_attention_noalloc per GPU.  A call is taken where its
+// required bytes fit RQ_ATTENTION_NOALLOC_MAX_BYTES; its plan then has the
+// whole scratch, which holds the partials of every such plan (1 request x 240
+// rows x 16 heads requires 8.1 MB and plans 32.4 MB), so that the call splits
+// its histories as the same call of rq_attention does.
+constexpr size_t kAttentionScratchBytes = (size_t)48 << 20;
+
 // RQ_ENOSPACE for a workspace smaller than the route of the call needs; a
 // call of rq_attention_noalloc names its static scratch instead.
 static int workspace_too_small(size_t needed, size_t got, bool static_scratch) {
@@ -554,6 +561,8 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
                             const int* groups, int reference_mode, int anchor_index, int loop_index,
                             void* workspace, size_t workspace_bytes, hipStream_t stream, bool timed,
                             bool causal = false, bool static_scratch = false) {
+    // What a call may require of its workspace.
+    const size_t accepted_bytes = static_scratch ? RQ_ATTENTION_NOALLOC_MAX_BYTES : workspace_bytes;
     int status = validate_schedule(head_dim, records, bits, groups, page_tokens, reference_mode,
                                    anchor_index, heads);
     if (status != RQ_OK) return status;
@@ -600,9 +609,12 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         const int64_t average_tiles = std::max<int64_t>(1, (rows / requests + 31) / 32);
         const int splits = multirow_splits(requests * heads * average_tiles, max_pages, page_tokens);
         const size_t required = multirow_bytes(rows, heads, splits);
-        const size_t full_bytes = attention_workspace_total(rows, heads, head_dim, max_pages, page_tokens);
-        if (workspace == nullptr || workspace_bytes < required)
-            return workspace_too_small(required, workspace_bytes, static_scratch);
+        if (workspace == nullptr || accepted_bytes < required)
+            return workspace_too_small(required, accepted_bytes, static_scratch);
+        // A workspace smaller than rq_attention_workspace_bytes gives makes fewer splits.
+        size_t plan_bytes = attention_workspace_total(rows, heads, head_dim, max_pages, page_tokens);
+        if (required <= RQ_ATTENTION_NOALLOC_MAX_BYTES) plan_bytes = std::min(plan_bytes, kAttentionScratchBytes);
+        plan_bytes = std::min(plan_bytes, workspace_bytes);
         rq::RecordRegion regions[rq::kMaxRecords];
         fill_regions(head_dim, records, bits, groups, page_tokens, regions);
         rq::MultiRowParams m{};
@@ -647,9 +659,9 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         m.call_tag = next_call_tag();
         const bool chunk = takes_chunk_kernels(rows, requests);
         if (chunk)
-            plan_chunk(m, std::min(workspace_bytes, full_bytes));
+            plan_chunk(m, plan_bytes);
         else
-            plan_multirow(m, splits, std::min(workspace_bytes, full_bytes));
+            plan_multirow(m, splits, plan_bytes);
         static_assert(rq::kMaxArrivals >= 65535, "the splits of one row tile, planned ones included");
         if ((int64_t)splits * row_tiles > 65535 || requests > (int64_t)INT32_MAX || rows > (int64_t)INT32_MAX)
             return fail(RQ_EINVAL, "Too many rows for one multi-row attention launch");
@@ -670,7 +682,7 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
     const int anchor_record = adjacent ? 0 : anchor_index;
     status = attention_common(query, query_stride, key, key_stride, value, value_stride, output,
                               output_stride, rows, heads, head_dim, query_start_loc, seq_lens, requests,
-                              block_table, block_table_stride, max_pages, workspace, workspace_bytes, splits, &p,
+                              block_table, block_table_stride, max_pages, workspace, accepted_bytes, splits, &p,
                               static_scratch);
     if (status != RQ_OK) return status;
     if (rows == 0) return ok();
@@ -732,7 +744,6 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
 // after the previous call's kernels.  Calls captured into a graph are not
 // (a capture cannot wait on work outside it): replays of such a graph must
 // not overlap other noalloc work on the same GPU.
-constexpr size_t kAttentionScratchBytes = RQ_ATTENTION_NOALLOC_MAX_BYTES;
 static __device__ __align__(256) uint8_t scratch[kAttentionScratchBytes];
 
 // Per device: the scratch address, and the event and stream of the last

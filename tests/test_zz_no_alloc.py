@@ -77,6 +77,31 @@ def test_noalloc_matches_workspace_entry_point(oracle, device):
             assert err.max() <= 2e-2 and err.mean() <= 1e-3, (err.max(), err.mean())
 
 
+@pytest.mark.parametrize("requests,rows,history", [(2, 100, 4700), (1, 200, 3000), (5, 40, 2000), (15, 40, 900)],
+                         ids=lambda v: str(v))
+def test_noalloc_splits_as_the_workspace_entry_point(device, requests, rows, history):
+    """Several rows per request whose plan takes more than the 8 MiB that a
+    no-alloc call may require, and up to it: the same splits, so the same
+    bytes, as with a workspace (chunk kernels, 32-row tiles)."""
+    import residualquant_amd as rq
+
+    lib = _lib.lib()
+    print(f"[case] noalloc {requests} requests x {rows} rows after {history} tokens", flush=True)
+    # Lengths far enough apart that the requests' splits are planned one by one.
+    lengths = [(history // 4 if i % 3 else history) + 1 for i in range(requests)]
+    d = make_decode(lengths, 16, 128, OURO_G32, seed=81, rows_per_request=[rows] * requests)
+    g = d.group
+    cache = torch.zeros(g.cache_shape, dtype=torch.uint8, device=device)
+    kr, vr, km = g.device_args(device)
+    rq.quantize([(a.to(device), b.to(device)) for a, b in g.pairs], cache, g.slots.to(device), kr, vr, km, g.records,
+                g.mode, g.anchor, g.coefficient)
+    for loop in (0, 3):
+        want = _call(lib, d, device, cache, loop, noalloc=False)
+        got = _call(lib, d, device, cache, loop, noalloc=True)
+        assert bool(torch.isfinite(want.float()).all())
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), f"loop {loop}"
+
+
 def test_noalloc_calls_on_two_streams_are_ordered(oracle, device):
     """Back-to-back noalloc calls on two streams with no synchronization
     between them: the library makes the second stream wait for the first
