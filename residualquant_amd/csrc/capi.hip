@@ -194,6 +194,34 @@ size_t multirow_bytes(int64_t rows, int heads, int splits) {
            align256(sizeof(float) * (size_t)rows * heads * splits * rq::kMultiRowEntry);
 }
 
+// What the plan of a call on 16- or 32-row tiles may take.
+struct MultiRowPlan {
+    int64_t tiles;       // 32-token tiles of the page table (steps of a chunk call)
+    int64_t forced;      // least splits: a split's pages fit its LDS block table
+    int64_t max_splits;  // most splits of one request, each of four tiles or more
+    int64_t target;      // workgroups per head that the work is spread over
+};
+
+MultiRowPlan multirow_plan_limits(int heads, int64_t max_pages, int page_tokens) {
+    MultiRowPlan plan;
+    plan.tiles = std::max<int64_t>(1, (max_pages * page_tokens + 31) / 32);
+    const int64_t most = (int64_t)(rq::kMultiRowMaxSplitPages - 1) * page_tokens / 32;
+    plan.forced = (plan.tiles + most - 1) / most;
+    plan.max_splits = std::max(std::min<int64_t>(rq::kMultiRowMaxSplits, std::max<int64_t>(1, plan.tiles / 4)), plan.forced);
+    // Three quarters of the two stream workgroups that a compute unit holds, so
+    // that with every request's share rounded up to whole splits all are
+    // resident at once: 16 requests of 824..8192 tokens x 4 rows x 16 heads took
+    // 62.3 us per residual call at 3/4 against 79.5 us at 1 and 76.4 us at 1/2.
+    plan.target = (3LL * compute_units() / 2 + heads - 1) / heads;
+    return plan;
+}
+
+// The most partial entries per head of such a plan.
+int64_t multirow_entries(int64_t rows, int heads, int64_t max_pages, int page_tokens) {
+    const MultiRowPlan plan = multirow_plan_limits(heads, max_pages, page_tokens);
+    return std::min<int64_t>(rows * plan.max_splits, rows * plan.forced + plan.target * 32);
+}
+
 // The plan of a multi-row call (multirow_plan in multirow.hip).  `splits`,
 // for every row alike, is what the call requires of its workspace
 // (multirow_bytes); the plan may use up to `bytes` of it.
@@ -208,23 +236,18 @@ void plan_multirow(rq::MultiRowParams& m, int splits, size_t bytes) {
         if ((int64_t)splits * ((m.rows + 15) / 16) > 65535) m.tile_rows = 32;  // the grid's z extent
         return;
     }
-    const int64_t tiles = std::max<int64_t>(1, (m.max_pages * m.page_tokens + 31) / 32);
+    const MultiRowPlan limits = multirow_plan_limits(m.heads, m.max_pages, m.page_tokens);
     const int64_t row_tiles = m.rows / m.tile_rows + m.requests;  // at most, over all requests
-    // A split's pages fit its LDS block table, so long histories take `forced` splits at least.
+    const int64_t forced = limits.forced;
     m.plan_max = (rq::kMultiRowMaxSplitPages - 1) * m.page_tokens / 32;
-    const int64_t forced = (tiles + m.plan_max - 1) / m.plan_max;
     m.plan_min = 4;  // one tile per wave
-    m.plan_max_splits = (int)std::max<int64_t>(rq::kMultiRowMaxSplits, forced);
-    // Three quarters of the two stream workgroups that a compute unit holds, so
-    // that with every request's share rounded up to whole splits all are
-    // resident at once: 16 requests of 824..8192 tokens x 4 rows x 16 heads took
-    // 62.3 us per residual call at 3/4 against 79.5 us at 1 and 76.4 us at 1/2.
+    m.plan_max_splits = (int)limits.max_splits;
     // Entries: at most rows x forced + target x tile_rows, and rows x max splits.
     const int64_t fit = (int64_t)(bytes / (sizeof(float) * rq::kMultiRowEntry) / m.heads);
-    int64_t target = (3LL * compute_units() / 2 + m.heads - 1) / m.heads;
+    int64_t target = limits.target;
     if (m.rows * m.plan_max_splits > fit)
         target = std::max<int64_t>(0, std::min<int64_t>(target, (fit - m.rows * forced) / m.tile_rows));
-    if (row_tiles > INT32_MAX / tiles) target = 0;  // the device sums row tiles x history tiles in 31 bits
+    if (row_tiles > INT32_MAX / limits.tiles) target = 0;  // the device sums row tiles x history tiles in 31 bits
     m.plan_target = (int)target;
     m.entries = fit;
     m.items = (int)std::max(row_tiles * forced + target, row_tiles * splits);
@@ -252,35 +275,48 @@ bool takes_chunk_kernels(int64_t rows, int64_t requests) {
     return requests <= rq::kPlanRequests && rows >= kChunkMinRows * requests;
 }
 
-// The most partial entries that the plan of a chunk call takes per head.
-int64_t chunk_entries(int64_t rows, int heads) {
-    const int64_t target = (compute_units() + heads - 1) / heads;
-    return std::min<int64_t>(rows * rq::kChunkMaxSplits, rows + target * rq::kChunkTileRows);
+// The same limits of a chunk call's plan, in steps of kChunkUnit tokens.
+MultiRowPlan chunk_plan_limits(int heads, int64_t max_pages, int page_tokens) {
+    MultiRowPlan plan;
+    plan.tiles = std::max<int64_t>(1, (max_pages * page_tokens + rq::kChunkUnit - 1) / rq::kChunkUnit);
+    const int64_t most = (int64_t)rq::kMultiRowMaxSplitPages * page_tokens / rq::kChunkUnit;
+    plan.forced = (plan.tiles + most - 1) / most;
+    plan.max_splits = std::max(std::min<int64_t>(rq::kChunkMaxSplits, std::max<int64_t>(1, plan.tiles / 2)), plan.forced);
+    plan.target = (3LL * compute_units() / 4 + heads - 1) / heads;
+    return plan;
+}
+
+// The most partial entries per head of such a plan.
+int64_t chunk_entries(int64_t rows, int heads, int64_t max_pages, int page_tokens) {
+    const MultiRowPlan plan = chunk_plan_limits(heads, max_pages, page_tokens);
+    // Equal requests: splits x row tiles number at most the compute units.
+    const int64_t groups = (compute_units() + heads - 1) / heads;
+    return std::min<int64_t>(rows * plan.max_splits,
+                             rows * plan.forced + std::max(plan.target, groups) * rq::kChunkTileRows);
 }
 
 // The plan of a chunk call: one stream workgroup fits a compute unit.
 void plan_chunk(rq::MultiRowParams& m, size_t bytes) {
     constexpr int64_t unit = rq::kChunkUnit;
-    const int64_t units = compute_units();
     m.tile_rows = rq::kChunkTileRows;
     m.plan_unit = (int)unit;
-    const int64_t steps = std::max<int64_t>(1, (m.max_pages * m.page_tokens + unit - 1) / unit);
+    const MultiRowPlan limits = chunk_plan_limits(m.heads, m.max_pages, m.page_tokens);
     const int64_t row_tiles = m.rows / m.tile_rows + m.requests;  // at most, over all requests
+    const int64_t forced = limits.forced;
     m.plan_max = (int)(rq::kMultiRowMaxSplitPages * m.page_tokens / unit);
-    const int64_t forced = (steps + m.plan_max - 1) / m.plan_max;
     m.plan_min = 2;
-    m.plan_max_splits = (int)std::max<int64_t>(rq::kChunkMaxSplits, forced);
+    m.plan_max_splits = (int)limits.max_splits;
     const int64_t fit = (int64_t)(bytes / (sizeof(float) * rq::kMultiRowEntry) / m.heads);
     // Equal requests: the splits that fill the compute units once.
     const int64_t average = (m.rows + m.requests - 1) / m.requests;
     const int64_t groups = m.requests * m.heads * ((average + m.tile_rows - 1) / m.tile_rows);
-    int64_t splits = std::max<int64_t>(units / groups, forced);
+    int64_t splits = std::max<int64_t>(compute_units() / groups, forced);
     splits = std::min<int64_t>(splits, std::min<int64_t>(fit / m.rows, m.plan_max_splits));
     m.splits = (int)std::max<int64_t>(splits, 1);
-    int64_t target = (3 * units / 4 + m.heads - 1) / m.heads;
+    int64_t target = limits.target;
     if (m.rows * m.plan_max_splits > fit)
         target = std::max<int64_t>(0, std::min<int64_t>(target, (fit - m.rows * forced) / m.tile_rows));
-    if (row_tiles > INT32_MAX / steps) target = 0;  // the device sums row tiles x history steps in 31 bits
+    if (row_tiles > INT32_MAX / limits.tiles) target = 0;  // the device sums row tiles x history steps in 31 bits
     m.plan_target = (int)target;
     m.entries = fit;
     m.items = (int)std::max(row_tiles * forced + target, row_tiles * m.splits);
@@ -448,19 +484,22 @@ int rq_quantize(int records, const void* const* key_ptrs, const int64_t* key_str
     return check_launch(rq::launch_quantize(p, head_dim, stream), "quantize launch");
 }
 
-// One workspace serves both paths of a packed attention call (the per-row
-// decode kernels and the multi-row kernels), so its size is the larger one.
 constexpr int kChainPerCu = 8;
 
+// One workspace serves both paths of a packed attention call (the per-row
+// decode kernels and the several-rows kernels), so its size is the larger one.
+// How the rows spread over requests is not known here: the chunk kernels take
+// a call from kChunkMinRows rows on, where one request may hold them all.
 static size_t attention_workspace_total(int64_t rows, int heads, int head_dim, int64_t max_pages,
                                         int page_tokens) {
     const int splits = std::max(split_count(rows, heads, max_pages), split_count(rows, heads, max_pages, kChainPerCu));
     size_t total = workspace_layout(rows, heads, head_dim, splits).total;
-    if ((head_dim == 96 || head_dim == 128) && (page_tokens == 16 || page_tokens == 32))
-        total = std::max(total,
-                         std::max(multirow_bytes(rows, heads,
-                                                 multirow_workspace_splits(rows, heads, max_pages, page_tokens)),
-                                  sizeof(float) * rq::kMultiRowEntry * heads * (size_t)chunk_entries(rows, heads)));
+    if ((head_dim == 96 || head_dim == 128) && (page_tokens == 16 || page_tokens == 32)) {
+        total = std::max(total, multirow_bytes(rows, heads, multirow_workspace_splits(rows, heads, max_pages, page_tokens)));
+        int64_t entries = multirow_entries(rows, heads, max_pages, page_tokens);
+        if (rows >= kChunkMinRows) entries = std::max(entries, chunk_entries(rows, heads, max_pages, page_tokens));
+        total = std::max(total, sizeof(float) * rq::kMultiRowEntry * heads * (size_t)entries);
+    }
     return total;
 }
 

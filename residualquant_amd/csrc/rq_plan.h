@@ -93,12 +93,11 @@ struct PlanShare {
     uint32_t even_splits, chunk;
 };
 
-__device__ __forceinline__ PlanShare plan_share(const PlanSizes& sizes, const PlanEntry& own, int lane) {
-    const uint32_t length = (uint32_t)own.length, count = (uint32_t)own.count;
+// `total`: count x length over the requests, `counts` their counts, `longest`
+// the longest length with a count.
+__host__ __device__ __forceinline__ PlanShare plan_share_of(const PlanSizes& sizes, uint32_t total, uint32_t counts,
+                                                            uint32_t longest) {
     const uint32_t min_chunk = (uint32_t)sizes.min_chunk;
-    const uint32_t total = __builtin_amdgcn_readlane(wave_scan(count * length, lane), 63);
-    const uint32_t counts = __builtin_amdgcn_readlane(wave_scan(count, lane), 63);
-    const uint32_t longest = wave_max_u32(count > 0 ? length : 0u);
     PlanShare s;
     const bool full = 4ull * counts >= 3ull * (uint32_t)sizes.target;
     s.even = 8ull * longest * counts <= (uint64_t)(full ? sizes.full_eighths : 9) * total;
@@ -120,7 +119,13 @@ __device__ __forceinline__ PlanShare plan_share(const PlanSizes& sizes, const Pl
     return s;
 }
 
-__device__ __forceinline__ uint32_t plan_splits(const PlanSizes& sizes, const PlanShare& share, uint32_t length) {
+__device__ __forceinline__ PlanShare plan_share(const PlanSizes& sizes, const PlanEntry& own, int lane) {
+    const uint32_t length = (uint32_t)own.length, count = (uint32_t)own.count;
+    return plan_share_of(sizes, __builtin_amdgcn_readlane(wave_scan(count * length, lane), 63),
+                         __builtin_amdgcn_readlane(wave_scan(count, lane), 63), wave_max_u32(count > 0 ? length : 0u));
+}
+
+__host__ __device__ __forceinline__ uint32_t plan_splits(const PlanSizes& sizes, const PlanShare& share, uint32_t length) {
     if (share.even) return share.even_splits;
     uint32_t splits = min(max((length + share.chunk - 1) / share.chunk, 1u), (uint32_t)sizes.max_splits);
     if (splits > 1 && splits * (uint32_t)sizes.min_chunk > length && length <= (uint32_t)sizes.max_chunk) splits -= 1;

@@ -149,15 +149,16 @@ def quantize(key_value_pairs: Sequence[Tuple[torch.Tensor, torch.Tensor]], kv_ca
 
 def attention_workspace_bytes(rows: int, heads: int, head_dim: int, max_pages: int,
                               page_tokens: int) -> int:
-    """Device workspace (bytes) that ``attention`` needs; depends on shapes only."""
+    """Device workspace (bytes) for ``attention``; depends on shapes only.  (A
+    smaller one that holds what the call's route requires is taken as well.)"""
     return int(_lib.lib().rq_attention_workspace_bytes(rows, heads, head_dim, max_pages, page_tokens))
 
 
 def _workspace(workspace: Optional[torch.Tensor], needed: int, device) -> torch.Tensor:
     if workspace is None:
         return torch.empty(needed, dtype=torch.uint8, device=device)
-    _require(workspace.is_cuda and workspace.device == device and workspace.is_contiguous()
-             and workspace.numel() * workspace.element_size() >= needed,
+    # (The library refuses one that is too small for the call's route.)
+    _require(workspace.is_cuda and workspace.device == device and workspace.is_contiguous(),
              f"Attention workspace of {needed} bytes required")
     return workspace
 

@@ -128,6 +128,18 @@ def test_workspace_size_depends_on_shapes_only(lib):
     assert lib.rq_attention_workspace_bytes(64, 16, 128, 512, 16) > a
 
 
+def test_workspace_counts_only_what_a_call_can_use(lib):
+    """Calls below the chunk kernels' 48 rows hold at most eight splits of
+    132 floats per (row, head) (and 4 bytes) over long histories, one over
+    those of a few pages; above, short histories limit the splits as well."""
+    entry = 132 * 4
+    for rows, heads, dim, pt in ((32, 16, 128, 16), (40, 16, 128, 16), (47, 16, 128, 32), (32, 55, 96, 16)):
+        assert lib.rq_attention_workspace_bytes(rows, heads, dim, 512, pt) <= rows * heads * (8 * entry + 4) + 512
+    decode = (272 + 130) * 4 + 8  # per (row, head) of the per-row kernels with one split
+    assert lib.rq_attention_workspace_bytes(128, 16, 128, 8, 16) <= 128 * 16 * max(entry + 4, decode) + 1024
+    assert lib.rq_attention_workspace_bytes(128, 16, 128, 32, 16) <= 128 * 16 * (4 * entry + 4) + 1024
+
+
 def test_workspace_grows_no_faster_than_linearly_in_rows(lib):
     """The workspace bound of a call with many rows (prefill over packed
     history) is sized for the splits its row count allows: from 64 rows up

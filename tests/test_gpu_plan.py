@@ -153,3 +153,43 @@ def test_captured_rows_replay(device, rows):
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out.view(torch.int16), want.view(torch.int16)), lengths
+
+
+@pytest.mark.parametrize("lengths,rows,mode", [([3000, 700, 90], None, "anchor"), ([2600, 1, 600], None, "adjacent"),
+                                               ([4000, 300, 600], [3, 20, 4], "anchor"),
+                                               ([3000, 400, 700], [300, 50, 110], "anchor"),
+                                               ([500] * 70, [2] * 70, "anchor")],
+                         ids=["decode", "adjacent", "rows", "chunk", "past-the-plan"])
+def test_workspace_of_the_required_size(oracle, device, lengths, rows, mode):
+    """The smallest workspace that a call takes: right results, nothing written past it."""
+    print(f"[case] required workspace {lengths[:3]} {rows and rows[:3]} {mode}", flush=True)
+    d = make_decode(lengths, 2, 128, ADJACENT if mode == "adjacent" else OURO_G32, seed=8, mode=mode,
+                    anchor=0 if mode == "adjacent" else 3, rows_per_request=rows)
+    g = d.group
+    cache_np = g.oracle_cache(oracle)
+    cache = torch.from_numpy(cache_np).to(device)
+    kr, vr, km = g.device_args(device)
+    q, k, v = (t.to(device) for t in (d.query, d.key, d.value))
+    starts, lens, table = (t.to(device) for t in (d.query_start_loc, d.seq_lens, d.table))
+    out = torch.full_like(q, float("nan"))
+
+    def call(workspace):
+        rq.attention(q, k, v, cache, out, starts, lens, table, kr, vr, km, g.records, g.mode, g.anchor, 1,
+                     workspace=workspace)
+
+    with pytest.raises(RuntimeError, match=r"Attention workspace of \d+ bytes required") as refused:
+        call(torch.empty(16, dtype=torch.uint8, device=device))
+    required = int(str(refused.value).split("workspace of ")[1].split()[0])
+    full = rq.ops.attention_workspace_bytes(q.size(0), 2, 128, table.size(1), 16)
+    assert required < full if rows and max(rows) > 100 else required <= full
+    with pytest.raises(RuntimeError, match="Attention workspace"):
+        call(torch.empty(required - 1, dtype=torch.uint8, device=device))
+    buffer = torch.full((required + 65536,), 0xA5, dtype=torch.uint8, device=device)
+    want = _bf16(_oracle(oracle, d, cache_np, 1, False))
+    for _ in range(2):
+        out.fill_(float("nan"))
+        call(buffer[:required])
+        err = np.abs(out.float().cpu().numpy() - want)
+        bar = MEAN_ABS + np.abs(want).mean() * 2.0 ** -9  # (as in test_planned_decode_matches_oracle)
+        assert err.max() <= MAX_ABS and err.mean() <= bar, (err.max(), err.mean())
+        assert bool((buffer[required:] == 0xA5).all())
