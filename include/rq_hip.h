@@ -95,7 +95,8 @@ size_t rq_attention_workspace_bytes(int64_t rows, int heads, int head_dim, int64
  * block_table: INT32 [>= requests, max_pages], row stride block_table_stride.
  * workspace: device memory of rq_attention_workspace_bytes(...).  A smaller
  *   one that holds what the call's route requires (see rq_attention_noalloc)
- *   is taken as well; several rows per request may then be split less.
+ *   is taken as well; several rows per request may then be split less.  No
+ *   alignment is required.
  * How a request's history is split, and with it the rounding of its output,
  * follows from the lengths of all requests of the call.
  */

@@ -510,6 +510,12 @@ static size_t attention_workspace_total(int64_t rows, int heads, int head_dim, i
 // its histories as the same call of rq_attention does.
 constexpr size_t kAttentionScratchBytes = (size_t)48 << 20;
 
+// The workspace of the packed kernels starts at the caller's next 16-byte
+// boundary (64-bit arrival words, 16-byte partials).  What a call requires
+// leaves room for it: the multi-row bytes hold 4 and the decode layout more
+// than 1000 bytes per (row, head) that the kernels do not use, in multiples of 256.
+static size_t to_boundary(const void* workspace) { return (0 - reinterpret_cast<uintptr_t>(workspace)) & 15; }
+
 // RQ_ENOSPACE for a workspace smaller than the route of the call needs; a
 // call of rq_attention_noalloc names its static scratch instead.
 static int workspace_too_small(size_t needed, size_t got, bool static_scratch) {
@@ -653,7 +659,7 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         // A workspace smaller than rq_attention_workspace_bytes gives makes fewer splits.
         size_t plan_bytes = attention_workspace_total(rows, heads, head_dim, max_pages, page_tokens);
         if (required <= RQ_ATTENTION_NOALLOC_MAX_BYTES) plan_bytes = std::min(plan_bytes, kAttentionScratchBytes);
-        plan_bytes = std::min(plan_bytes, workspace_bytes);
+        plan_bytes = std::min(plan_bytes, workspace_bytes - to_boundary(workspace));
         rq::RecordRegion regions[rq::kMaxRecords];
         fill_regions(head_dim, records, bits, groups, page_tokens, regions);
         rq::MultiRowParams m{};
@@ -694,7 +700,7 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         m.key_mean_anchor = (key_mean && m.has_residual) ? key_mean + (int64_t)anchor * heads * head_dim : nullptr;
         m.causal = causal ? 1 : 0;
         m.compute_units = compute_units();
-        m.partials = static_cast<float*>(workspace);
+        m.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + to_boundary(workspace));
         m.call_tag = next_call_tag();
         const bool chunk = takes_chunk_kernels(rows, requests);
         if (chunk)
@@ -741,7 +747,7 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
     p.key_mean_loop = key_mean ? key_mean + (int64_t)loop_index * heads * head_dim : nullptr;
     p.key_mean_anchor = (key_mean && p.has_residual) ? key_mean + (int64_t)anchor * heads * head_dim : nullptr;
     const DecodePlan plan = decode_plan(rows, heads, head_dim, max_pages, per_cu, page_tokens,
-                                        workspace_layout(rows, heads, head_dim, splits).total);
+                                        workspace_layout(rows, heads, head_dim, splits).total - to_boundary(workspace));
     p.plan_min_pages = plan.min_pages;
     p.plan_target = plan.target;
     p.plan_round_pages = 0;
@@ -757,8 +763,9 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
                                       (max_pages + p.plan_round_pages - 1) / p.plan_round_pages));
         p.splits = std::max(p.splits, 1);
     }
-    p.arrivals = static_cast<uint64_t*>(workspace);
-    p.partials = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + plan.partials);
+    uint8_t* const base = static_cast<uint8_t*>(workspace) + to_boundary(workspace);
+    p.arrivals = reinterpret_cast<uint64_t*>(base);
+    p.partials = reinterpret_cast<float*>(base + plan.partials);
     p.call_tag = next_call_tag();
     p.compute_units = compute_units();
     // Adjacent mode past loop 0 decodes the restore chain of records 0..loop.

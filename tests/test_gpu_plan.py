@@ -161,7 +161,8 @@ def test_captured_rows_replay(device, rows):
                                                ([500] * 70, [2] * 70, "anchor")],
                          ids=["decode", "adjacent", "rows", "chunk", "past-the-plan"])
 def test_workspace_of_the_required_size(oracle, device, lengths, rows, mode):
-    """The smallest workspace that a call takes: right results, nothing written past it."""
+    """The smallest workspace that a call takes, at any address: right results,
+    nothing written around it."""
     print(f"[case] required workspace {lengths[:3]} {rows and rows[:3]} {mode}", flush=True)
     d = make_decode(lengths, 2, 128, ADJACENT if mode == "adjacent" else OURO_G32, seed=8, mode=mode,
                     anchor=0 if mode == "adjacent" else 3, rows_per_request=rows)
@@ -186,10 +187,12 @@ def test_workspace_of_the_required_size(oracle, device, lengths, rows, mode):
         call(torch.empty(required - 1, dtype=torch.uint8, device=device))
     buffer = torch.full((required + 65536,), 0xA5, dtype=torch.uint8, device=device)
     want = _bf16(_oracle(oracle, d, cache_np, 1, False))
-    for _ in range(2):
+    for offset in (0, 0, 4, 264, 4097, 31):
+        print(f"[case]   workspace at + {offset}", flush=True)
         out.fill_(float("nan"))
-        call(buffer[:required])
+        buffer.fill_(0xA5)
+        call(buffer[offset:offset + required])
         err = np.abs(out.float().cpu().numpy() - want)
         bar = MEAN_ABS + np.abs(want).mean() * 2.0 ** -9  # (as in test_planned_decode_matches_oracle)
         assert err.max() <= MAX_ABS and err.mean() <= bar, (err.max(), err.mean())
-        assert bool((buffer[required:] == 0xA5).all())
+        assert bool((buffer[:offset] == 0xA5).all()) and bool((buffer[offset + required:] == 0xA5).all())
