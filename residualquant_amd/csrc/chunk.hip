@@ -459,21 +459,52 @@ void chunk_chain_kernel(MultiRowParams p) {
 
 // ---------------------------------------------------------------- finish
 
+// The 32-row tile of rank `key` among the call's row tiles, the deepest first:
+// the last rows, which see the most live tokens, start first, and the
+// workgroups past the tiles come last.  (Each holds its LDS until it exits: a
+// grid of every tile that each request could have, the empty ones first, took
+// 175 us per residual call of 64 requests of 500 tokens x 48 rows x 16 heads,
+// this one 147 us; 2 requests x 509 rows 98.3 and 96.6 us.)
+struct FinishTile {
+    int request, tile;  // request -1: past the last tile
+};
+
+__device__ __forceinline__ FinishTile finish_tile(const PlanEntry& own, int key) {
+    const int lane = threadIdx.x & 63;
+    const int tiles = (own.rows + 31) / 32;
+    // Tiles of index `depth` and deeper.
+    auto from = [&](int depth) __attribute__((always_inline)) {
+        return (int)__builtin_amdgcn_readlane(wave_scan((uint32_t)max(tiles - depth, 0), lane), 63);
+    };
+    if (key >= from(0)) return FinishTile{-1, 0};
+    int low = 0, high = (int)wave_max_u32((uint32_t)tiles);  // from(low) > key >= from(high)
+    while (high - low > 1) {
+        const int middle = (low + high) / 2;
+        if (from(middle) > key) low = middle;
+        else high = middle;
+    }
+    const bool has = tiles > low;
+    // (Every lane takes part in the scans.)
+    const int order = (int)wave_scan(has ? 1u : 0u, lane), wanted = key - from(high) + 1;
+    return FinishTile{__builtin_ctzll(__ballot(has && order == wanted)), low};
+}
+
 // 32 rows of one (request, head) per workgroup: finish_merge and finish_rows
 // (rq_multirow.h).
 template <int D>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 void chunk_finish_kernel(MultiRowParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[Geometry<D, 32>::kLdsBytes];
-    const int request = blockIdx.x, head = blockIdx.y;
-    // The last rows, which see the most live tokens, start first.
-    const int row0 = 32 * (int)(gridDim.z - 1 - blockIdx.z);
-    const RequestRows own = request_rows(p, request);
-    const int first = own.first, n = own.rows;
-    if (row0 >= n) return;  // uniform over the workgroup, before any barrier
+    const int head = (int)(blockIdx.x % (unsigned)p.heads);
+    const PlanEntry own = multirow_entry(p);
+    const FinishTile at = finish_tile(own, (int)(blockIdx.x / (unsigned)p.heads));
+    if (at.request < 0) return;  // uniform over the workgroup, before any barrier
+    const int request = __builtin_amdgcn_readfirstlane(at.request);
+    const int row0 = 32 * __builtin_amdgcn_readfirstlane(at.tile);
+    const int first = __builtin_amdgcn_readlane(own.first, request), n = __builtin_amdgcn_readlane(own.rows, request);
     FinishInputs<D> in;
     finish_load<D, 32>(p, head, first, row0, n, in);
-    const PlanRequest plan = plan_request(request, multirow_sizes(p), multirow_entry(p));
+    const PlanRequest plan = plan_request(request, multirow_sizes(p), own);
     const int tid = threadIdx.x, r = tid >> 3, part = tid & 7;
     const bool valid = row0 + r < n;
     const float* tile_entries =
@@ -541,9 +572,8 @@ bool launch_d(const MultiRowParams& p, hipStream_t stream) {
     const bool launched = p.page_tokens == 16 ? launch_pt<D, 16>(p, stream)
                                               : p.page_tokens == 32 && launch_pt<D, 32>(p, stream);
     if (!launched) return false;
-    hipLaunchKernelGGL(chunk_finish_kernel<D>,
-                       dim3((unsigned)p.requests, (unsigned)p.heads, (unsigned)((p.rows + 31) / 32)), dim3(kThreads), 0,
-                       stream, p);
+    const int64_t tiles = p.rows / 32 + p.requests;  // at most, over all requests
+    hipLaunchKernelGGL(chunk_finish_kernel<D>, dim3((unsigned)(tiles * p.heads)), dim3(kThreads), 0, stream, p);
     return true;
 }
 

@@ -26,6 +26,10 @@ CASES = [
     ([2100], [64], 1, ((2, 16), (4, 16), (2, 32), (4, 32)), 16, False, True, 96, "anchor"),  # eight splits
     ([600, 129], [100, 64], 2, ADJACENT_G32, 16, True, True, 128, "adjacent"),
     ([333], [289], 2, ADJACENT_G16, 32, False, False, 96, "adjacent"),
+    # row tiles of many depths, at the edges of 32 rows; the most requests
+    ([9, 40, 31, 90, 33, 200, 65, 420, 70, 96, 300], [0, 1, 31, 32, 33, 64, 65, 300, 0, 96, 129], 3, OURO_G32, 16, True,
+     True, 128, "anchor"),
+    ([60 + i for i in range(64)], [48] * 63 + [49], 1, OURO_G32, 16, True, True, 128, "anchor"),
 ]
 
 
