@@ -34,6 +34,8 @@
 // k 8 (l / 32) + e; B column l % 32, k 8 (l / 32) + e; C register r holds row
 // 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
 
+#include <algorithm>
+
 #include "rq_device.h"
 #include "rq_kernels.h"
 #include "rq_plan.h"
@@ -52,6 +54,7 @@ constexpr int kBlockQueries = kPrefillBlockQueries;  // 32 per wave
 constexpr int kBlockKeys = kPrefillBlockKeys;
 constexpr float kLazyRescale = 8.0f;  // log2 units: rescale when a row max grows by more
 constexpr int kXcds = 8;              // MI355X accelerator complex dies
+constexpr int kXcdComputeUnits = 32;  // compute units of one
 static_assert(kBlockQueries == 32 * kGroupWaves, "one 32-query MFMA column block per wave");
 
 __device__ __forceinline__ F32x16 mfma(Bf16x8 a, Bf16x8 b, F32x16 c) {
@@ -133,41 +136,90 @@ struct BlockState {
     float running_max, running_sum;  // log2 units; the sum of this half-wave's keys
 };
 
-// Pair `rank` of a batch of at most 64 sequences, the longest sequences first
-// (eight classes by key length); sequence -1 past the last pair.  The grid
-// covers max_seqlen_q in every sequence, and one workgroup (128 KB of LDS)
-// fits a compute unit, so in sequence order the pairs that do not exist hold
-// back the others and the longest sequence may come last: 12 prompts of
-// 17..1500 tokens x 16 heads (25 of 72 pairs exist) took 108 us in sequence
-// order, 40 us in this one.  Every wave of the grid ranks alike.
-struct RankedPair {
-    int sequence, item;
+// The work of workgroup `linear` in a batch of 2 to 64 sequences, one sequence
+// per lane.  The grid covers max_seqlen_q in every sequence, and one workgroup
+// (128 KB of LDS) fits a compute unit, so in sequence order the block pairs
+// that do not exist hold back the others and the longest sequence may come
+// last: 12 prompts of 17..1500 tokens x 16 heads (25 of 72 pairs exist) took
+// 108 us in that order, 40 us ranked.
+// - Sequences that are not alike are ranked by key length (eight classes, the
+//   longest first), and each XCD (linear % 8) takes every eighth (sequence,
+//   head) group in that order.  A head's K/V tiles stay in one L2 whatever the
+//   head count: with one order for all XCDs, heads innermost, 12 prompts of
+//   40..1500 tokens x 55 heads x 96 took 139 us, here 127 us.
+// - Alike sequences, all of the grid's pairs: each XCD takes a run of groups.
+//   Four groups at a time (fewer where a group's pairs fill the XCD) go pair
+//   by pair, since a group's last pair may be the short one and the dispatcher
+//   deals workgroups out in turn: 12 x 300 tokens x 55 heads (a long and a
+//   short pair each) took 83 us group by group, 69 us so; 4 x 512 tokens
+//   41.6 and 41.5 us, heads innermost 45.3 us.
+// Workgroups without work come last.
+struct PrefillItem {
+    int sequence, head, item;  // sequence -1: no work
+    int q_begin, q_len, k_begin, k_len;
 };
 
-__device__ __forceinline__ RankedPair ranked_pair(const PrefillParams& p, int rank) {
+// The first `n` (sequence, head) groups hold this many of XCD `xcd`.
+__device__ __forceinline__ int groups_of_xcd(int n, int xcd) { return (n + kXcds - 1 - xcd) / kXcds; }
+
+__device__ __forceinline__ PrefillItem ranked_item(const PrefillParams& p, int linear) {
     const int lane = threadIdx.x & 63;
     const int at = lane < p.batch ? lane : p.batch - 1;
-    const int q_len = p.cu_seqlens_q[at + 1] - p.cu_seqlens_q[at];
-    const int k_len = max(p.cu_seqlens_k[at + 1] - p.cu_seqlens_k[at], 0);
+    const int q_begin = p.cu_seqlens_q[at], q_len = p.cu_seqlens_q[at + 1] - q_begin;
+    const int k_begin = p.cu_seqlens_k[at], k_len = p.cu_seqlens_k[at + 1] - k_begin;
     // (No more pairs than the grid holds for one sequence.)
     const int blocks = min((max(q_len, 0) + kBlockQueries - 1) / kBlockQueries, p.query_blocks);
-    const uint32_t pairs = lane < p.batch ? (uint32_t)(blocks + 1) / 2 : 0u;
-    const uint32_t longest = wave_max_u32(pairs > 0 ? (uint32_t)k_len : 0u);
-    const float part = (float)k_len * 8.0f / (float)max(longest, 1u);
-    const int size_class = 7 - min((int)part, 7);
-    RankedPair r{-1, 0};
-    uint32_t base = 0;
-    for (int k = 0; k < 8; ++k) {
-        const uint32_t own = size_class == k ? pairs : 0u;
-        const uint32_t end = base + wave_scan(own, lane), begin = end - own;
-        const uint64_t mask = __ballot(begin <= (uint32_t)rank && (uint32_t)rank < end);
-        if (mask != 0) {
-            r.sequence = __builtin_ctzll(mask);
-            r.item = rank - (int)__builtin_amdgcn_readlane(begin, r.sequence);
-            break;
+    const int pairs = lane < p.batch ? (blocks + 1) / 2 : 0;
+    const uint32_t longest = wave_max_u32(pairs > 0 ? (uint32_t)max(k_len, 0) : 0u);
+    const float part = (float)max(k_len, 0) * 8.0f / (float)max(longest, 1u);
+    const int size_class = pairs > 0 ? 7 - min((int)part, 7) : 8;
+    const int xcd = linear % kXcds, slot = linear / kXcds;
+    PrefillItem r{-1, 0, 0, 0, 0, 0, 0};
+    if (__ballot(lane < p.batch && (size_class != 0 || pairs != p.items)) == 0) {
+        // Alike sequences: each XCD a run of groups, up to four at a time.
+        const int groups = p.batch * p.heads_q;
+        const int first = xcd * groups / kXcds, last = (xcd + 1) * groups / kXcds;
+        int group = first + slot;
+        if (p.items > 1) {
+            const int together = min(max(kXcdComputeUnits / p.items, 1), 4);
+            const int turn = slot / (together * p.items), local = slot - turn * together * p.items;
+            const int at = first + together * turn, width = min(together, last - at);
+            if (width <= 0 || local >= width * p.items) return r;
+            r.item = local / width;
+            group = at + local - r.item * width;
+        } else if (group >= last) {
+            return r;
         }
-        base = __builtin_amdgcn_readlane(end, 63);
+        r.sequence = group / p.heads_q;
+        r.head = group - r.sequence * p.heads_q;
+    } else {
+        // Lane i takes the i-th sequence of the ranking.
+        int position = 0, before = 0;
+#pragma unroll
+        for (int k = 0; k <= 8; ++k) {
+            const uint64_t mask = __ballot(size_class == k);
+            const int within = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+            if (size_class == k) position = before + within;
+            before += __builtin_popcountll(mask);
+        }
+        const int ranked_pairs = __builtin_amdgcn_ds_permute(4 * position, pairs);
+        const int ranked_lane = __builtin_amdgcn_ds_permute(4 * position, lane);
+        const int first_group = groups_of_xcd(lane * p.heads_q, xcd);
+        const int groups = groups_of_xcd((lane + 1) * p.heads_q, xcd) - first_group;
+        const int own = groups * ranked_pairs;
+        const int end = (int)wave_scan((uint32_t)own, lane), begin = end - own;
+        const uint64_t mask = __ballot(begin <= slot && slot < end);
+        if (mask == 0) return r;
+        const int rank = __builtin_ctzll(mask);
+        r.sequence = __builtin_amdgcn_readlane(ranked_lane, rank);
+        const int local = slot - __builtin_amdgcn_readlane(begin, rank), each = __builtin_amdgcn_readlane(groups, rank);
+        r.item = local / each;
+        r.head = kXcds * (__builtin_amdgcn_readlane(first_group, rank) + local - r.item * each) + xcd - rank * p.heads_q;
     }
+    r.q_begin = __builtin_amdgcn_readlane(q_begin, r.sequence);
+    r.q_len = __builtin_amdgcn_readlane(q_len, r.sequence);
+    r.k_begin = __builtin_amdgcn_readlane(k_begin, r.sequence);
+    r.k_len = __builtin_amdgcn_readlane(k_len, r.sequence);
     return r;
 }
 
@@ -178,15 +230,10 @@ void prefill_kernel(PrefillParams p) {
     __shared__ __attribute__((aligned(1024))) char lds[L::kBytes];
 
     int linear = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    int item, head, sequence;
-    if (p.batch > 1 && p.batch <= 64) {
-        // Heads innermost: with a multiple of 8 heads each XCD keeps its own
-        // heads' K/V tiles in its L2.
-        head = linear % gridDim.y;
-        const RankedPair pair = ranked_pair(p, linear / gridDim.y);
-        if (pair.sequence < 0) return;
-        sequence = __builtin_amdgcn_readfirstlane(pair.sequence);
-        item = __builtin_amdgcn_readfirstlane(pair.item);
+    PrefillItem work;
+    if (p.ranked != 0) {
+        work = ranked_item(p, linear);
+        if (work.sequence < 0) return;
     } else {
         // XCD-aware order: workgroups are dispatched round-robin over the 8
         // XCDs, so the linear id is remapped to give each XCD a run of
@@ -194,14 +241,17 @@ void prefill_kernel(PrefillParams p) {
         // tiles stay in that XCD's L2 (when the grid divides by 8).
         const int grid_total = gridDim.x * gridDim.y * gridDim.z;
         if (grid_total % kXcds == 0) linear = (linear % kXcds) * (grid_total / kXcds) + linear / kXcds;
-        item = linear % gridDim.x;
-        head = (linear / gridDim.x) % gridDim.y;
-        sequence = linear / (gridDim.x * gridDim.y);
+        work.item = linear % gridDim.x;
+        work.head = (linear / gridDim.x) % gridDim.y;
+        work.sequence = linear / (gridDim.x * gridDim.y);
+        work.q_begin = p.cu_seqlens_q[work.sequence];
+        work.q_len = p.cu_seqlens_q[work.sequence + 1] - work.q_begin;
+        work.k_begin = p.cu_seqlens_k[work.sequence];
+        work.k_len = p.cu_seqlens_k[work.sequence + 1] - work.k_begin;
     }
-    const int q_begin = p.cu_seqlens_q[sequence];
-    const int q_len = p.cu_seqlens_q[sequence + 1] - q_begin;
-    const int k_begin = p.cu_seqlens_k[sequence];
-    const int k_len = p.cu_seqlens_k[sequence + 1] - k_begin;
+    const int item = __builtin_amdgcn_readfirstlane(work.item), head = __builtin_amdgcn_readfirstlane(work.head);
+    const int q_begin = __builtin_amdgcn_readfirstlane(work.q_begin), q_len = __builtin_amdgcn_readfirstlane(work.q_len);
+    const int k_begin = __builtin_amdgcn_readfirstlane(work.k_begin), k_len = __builtin_amdgcn_readfirstlane(work.k_len);
     const int n_blocks = (q_len + kBlockQueries - 1) / kBlockQueries;
     if (item >= (n_blocks + 1) / 2) return;  // uniform over the workgroup, before any barrier
     const int shift = k_len - q_len;         // query i sees keys j <= i + shift (causal)
@@ -508,15 +558,19 @@ void prefill_kernel(PrefillParams p) {
 }  // namespace
 
 size_t prefill_plan(PrefillParams& p, int64_t max_seqlen_k) {
-    (void)max_seqlen_k;
     p.query_blocks = (int)((p.max_seqlen_q + kBlockQueries - 1) / kBlockQueries);
     p.items = (p.query_blocks + 1) / 2;  // block pairs per (sequence, head)
-    return 0;                            // no workspace: blocks merge within their workgroup
+    // Sequences of one block and two key tiles: nothing to rank, and the ranking's
+    // 0.6 us count (64 sequences of 60 tokens x 16 heads 29.8 against 29.2 us).
+    p.ranked = p.batch > 1 && p.batch <= 64 && std::max<int64_t>(p.max_seqlen_q, max_seqlen_k) > kBlockQueries ? 1 : 0;
+    return 0;  // no workspace: blocks merge within their workgroup
 }
 
 hipError_t launch_prefill(const PrefillParams& p, hipStream_t stream) {
     if (p.batch == 0 || p.max_seqlen_q == 0 || p.items == 0) return hipSuccess;
-    const dim3 grid((unsigned)p.items, (unsigned)p.heads_q, (unsigned)p.batch);
+    dim3 grid((unsigned)p.items, (unsigned)p.heads_q, (unsigned)p.batch);
+    // An XCD takes at most ceil(batch x heads / 8) (sequence, head) groups.
+    if (p.ranked != 0) grid = dim3((unsigned)(kXcds * p.items), (unsigned)((p.batch * p.heads_q + kXcds - 1) / kXcds));
     if (p.head_dim == 128)
         hipLaunchKernelGGL(prefill_kernel<128>, grid, dim3(kPrefillThreads), 0, stream, p);
     else if (p.head_dim == 96)

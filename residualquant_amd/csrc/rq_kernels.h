@@ -82,6 +82,7 @@ struct PrefillParams {
     // no workspace is needed.
     int query_blocks;         // ceil(max_seqlen_q / 128)
     int items;                // block pairs per (head, sequence)
+    int ranked;               // ranked_item in prefill.hip orders the work
 };
 
 constexpr int kPrefillBlockQueries = 128;

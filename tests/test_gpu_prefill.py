@@ -160,3 +160,39 @@ def test_prefill_batch_equals_its_sequences(device, lengths, dim, causal):
         one = torch.tensor([0, n], dtype=torch.int32, device=device)
         alone = rq.flash_attn_varlen_func(q[rows], k[rows], v[rows], n, one, n, one, causal=causal)
         assert torch.equal(out[rows].view(torch.int16), alone.view(torch.int16)), n
+
+
+@pytest.mark.parametrize("q_lens,k_lens,heads", [
+    ([300] * 5, None, 5),             # alike: a long and a short pair per group, groups that 8 XCDs do not divide
+    ([512, 500, 490], None, 16),      # alike within an eighth, the same pairs
+    ([2600, 2500], None, 3),          # alike: eleven pairs, two groups at a time
+    ([250] * 9, None, 1),             # alike: one pair per group
+    ([200] * 64, None, 2),            # the most sequences
+    ([900, 30, 400, 0, 257, 128], None, 13),
+    ([40, 40, 7], [900, 100, 333], 6),  # few queries over more keys
+    ([100, 3], [0, 300], 2),          # a sequence without keys
+], ids=lambda v: "" if v is None else f"{len(v)}x{v[0]}" if isinstance(v, list) else f"h{v}")
+@pytest.mark.parametrize("dim", [128, 96])
+def test_prefill_order_of_batches(device, q_lens, k_lens, heads, dim):
+    """Whatever order a batch's pairs are taken in, each sequence's rows are
+    the bytes of a call of its own."""
+    k_lens = q_lens if k_lens is None else k_lens
+    print(f"[case] prefill order {q_lens[:6]} over {k_lens[:6]} x {heads} heads x {dim}", flush=True)
+    generator = torch.Generator(device=device).manual_seed(sum(q_lens) + heads)
+    q = torch.randn((sum(q_lens), heads, dim), generator=generator, device=device).to(torch.bfloat16)
+    k, v = (torch.randn((sum(k_lens), heads, dim), generator=generator, device=device).to(torch.bfloat16)
+            for _ in range(2))
+
+    def starts(lens):
+        return torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32, device=device)
+
+    def call(q, k, v, q_lens, k_lens):
+        return rq.flash_attn_varlen_func(q, k, v, max(q_lens), starts(q_lens), max(k_lens),
+                                         cu_seqlens_k=starts(k_lens), causal=True, out=torch.full_like(q, float("nan")))
+
+    out = call(q, k, v, q_lens, k_lens)
+    for q_n, k_n, q_at, k_at in zip(q_lens, k_lens, np.cumsum([0] + q_lens), np.cumsum([0] + k_lens)):
+        if q_n == 0 or k_n == 0:
+            continue
+        alone = call(q[q_at:q_at + q_n], k[k_at:k_at + k_n], v[k_at:k_at + k_n], [q_n], [k_n])
+        assert torch.equal(out[q_at:q_at + q_n].view(torch.int16), alone.view(torch.int16)), (q_n, k_n)
