@@ -2013,12 +2013,38 @@ __global__ __launch_bounds__(kDecodeThreads) void decode_bf16_kernel(AttentionPa
 
 // ------------------------------------------------------------------ launch
 
+// Splits of every row of an adjacent-mode chain over equal lengths, at most
+// p.splits.  The chain kernels are bound by their VALU work, so a call takes as
+// long as the compute unit with the most workgroups, k: each costs its part of
+// the history and its prologue and merge (about 160 tokens' time), a unit with
+// fewer than `per_cu` workgroups at a time a third of one more, and the ends of
+// long workgroups spread (an eighth).  Loops 1 / 2 / 3 of 16 heads, with 8
+// workgroups per compute unit or one per 512 tokens -> here: 4 x 8192 tokens
+// 79 / 109 / 130 -> 60 / 80 / 99 us, 16 x 4096 117 / 172 / 205 -> 99 / 141 /
+// 176 us, 32 x 8192 326 / 507 / 638 -> 325 / 502 / 637 us.
+inline int chain_splits(const AttentionParams& p, int per_cu) {
+    const int64_t pairs = p.rows * p.heads, tokens = p.max_pages * p.page_tokens;
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int s = 1; s <= p.splits; ++s) {
+        const int64_t k = (pairs * s + p.compute_units - 1) / p.compute_units;
+        const int64_t alone = k < per_cu ? per_cu - k : k % per_cu != 0 ? 1 : 0;
+        const int64_t cost = (tokens / s + 160) * (100 * k + 35 * alone + 12);
+        if (cost < least) {
+            least = cost;
+            best = s;
+        }
+    }
+    return best;
+}
+
 // The launch parameters of a kernel of which the device holds `per_cu`
 // workgroups per compute unit at once: those and the grid.
 inline AttentionParams with_plan(const AttentionParams& params, int per_cu) {
     AttentionParams p = params;
     p.resident = (int64_t)per_cu * p.compute_units;
     if (p.requests <= kPlanRequests) {
+        if (p.chain_length > 0) p.splits = chain_splits(p, per_cu);
         // No more than one item per plan_min_pages pages of every row.
         const int64_t by_pages = std::max<int64_t>(1, (p.max_pages + p.plan_min_pages - 1) / p.plan_min_pages);
         const int64_t ragged = by_pages <= p.plan_target / p.rows ? p.rows * by_pages : p.rows + p.plan_target;

@@ -484,6 +484,9 @@ int rq_quantize(int records, const void* const* key_ptrs, const int64_t* key_str
     return check_launch(rq::launch_quantize(p, head_dim, stream), "quantize launch");
 }
 
+// Most workgroups per compute unit that an adjacent-mode call past loop 0
+// (decode_chain_kernel) is spread over; chain_splits in attention.hip takes
+// fewer where the lengths are equal.
 constexpr int kChainPerCu = 8;
 
 // One workspace serves both paths of a packed attention call (the per-row
@@ -589,12 +592,6 @@ static int attention_common(const void* query, int64_t query_stride, const void*
 // residual call measured 82.1, 85.8, 92.4 and 92.3 us at 1, 2, 3 and 4 splits
 // per (row, head)).
 static int packed_per_cu(int head_dim) { return head_dim == 96 ? 1 : 2; }
-
-// Of an adjacent-mode call past loop 0 (decode_chain_kernel): that kernel is
-// bound by its VALU work, not by HBM, and shorter page spans per workgroup
-// let one workgroup's prologue and finish overlap another's chain: at batch
-// 32 x 8k x 16 heads, loops 1 / 2 / 3 measured 364 / 512 / 660 us at two
-// workgroups per compute unit and 320 / 498 / 628 us at eight (kChainPerCu).
 
 static int attention_packed(const void* query, int64_t query_stride, const void* key, int64_t key_stride,
                             const void* value, int64_t value_stride, void* output, int64_t output_stride,
@@ -758,10 +755,11 @@ static int attention_packed(const void* query, int64_t query_stride, const void*
         const int64_t round = 2LL * compute_units();
         p.plan_round_pages = kChainRoundTokens / page_tokens;
         p.plan_round_target = (int)std::max<int64_t>(1, round * 3 / 4 / heads);
-        p.splits = (int)std::min<int64_t>(
-            splits, std::max<int64_t>((round + rows * heads - 1) / (rows * heads),
-                                      (max_pages + p.plan_round_pages - 1) / p.plan_round_pages));
-        p.splits = std::max(p.splits, 1);
+        // (Equal lengths: chain_splits in attention.hip.)
+        if (requests > rq::kPlanRequests)
+            p.splits = (int)std::max<int64_t>(
+                1, std::min<int64_t>(splits, std::max<int64_t>((round + rows * heads - 1) / (rows * heads),
+                                                               (max_pages + p.plan_round_pages - 1) / p.plan_round_pages)));
     }
     uint8_t* const base = static_cast<uint8_t*>(workspace) + to_boundary(workspace);
     p.arrivals = reinterpret_cast<uint64_t*>(base);
