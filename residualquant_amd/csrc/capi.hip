@@ -10,11 +10,11 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
-#include <random>
 #include <string>
 #include <vector>
 
@@ -253,11 +253,17 @@ void plan_multirow(rq::MultiRowParams& m, int splits, size_t bytes) {
     m.items = (int)std::max(row_tiles * forced + target, row_tiles * splits);
 }
 
-// A call's tag for its arrival words (rq_plan.h), never 0.
+// A call's tag for its arrival words (rq_plan.h), never 0.  The start is hashed
+// from the clock and a load address: std::random_device may throw, which must
+// not cross the C boundary.
 uint64_t next_call_tag() {
     static std::atomic<uint64_t> counter{[] {
-        std::random_device source;
-        return ((uint64_t)source() << 32) | source();
+        uint64_t x = (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() ^
+                     ((uint64_t)reinterpret_cast<uintptr_t>(&g_compute_units) << 20);
+        // (splitmix64)
+        x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+        x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+        return x ^ (x >> 31);
     }()};
     constexpr uint64_t kMask = ~0ull >> rq::kArrivalBits;
     uint64_t tag;

@@ -45,6 +45,14 @@ def test_library_exports_every_declared_symbol(lib):
         assert getattr(lib, name) is not None
 
 
+def test_calls_do_not_read_a_random_device(lib):
+    """std::random_device throws where it finds no source, and a C++ exception
+    must not leave a C entry point: the call tags start from the clock."""
+    out = subprocess.run(["nm", "-DC", "--undefined-only", _lib.LIB_PATH], capture_output=True, text=True,
+                         check=True).stdout
+    assert "random_device" not in out
+
+
 def _schedule(records):
     bits = (ctypes.c_int * len(records))(*[r[0] for r in records])
     groups = (ctypes.c_int * len(records))(*[r[1] for r in records])

@@ -27,7 +27,7 @@ CASES = [
     ([1700, 300, 16, 17], None, 3, 96, 16, "anchor", 64),
     ([2600, 1, 600], None, 2, 128, 16, "adjacent", 0),
     ([2100, 2050, 2090], None, 2, 96, 32, "adjacent", 0),   # near-equal chains: as many splits as fit
-    ([300] * 40, None, 13, 128, 16, "adjacent", 0),         # 520 of them: more than two per compute unit
+    ([34] * 58, None, 9, 96, 16, "adjacent", 0),            # 522 of them: more than two per compute unit
     ([1400] + [3] * 64 + [700], None, 1, 128, 16, "anchor", 9),
     ([600] + [2, 35] * 130, None, 1, 128, 16, "anchor", 600),
 ]
