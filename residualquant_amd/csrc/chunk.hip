@@ -10,11 +10,12 @@
 // are dequantized once per 256 rows, where multirow.hip's 32-row tiles do it
 // once per 32 (dequantizing is 3/4 of their vector instructions).  The tiles
 // are double-buffered with one barrier per step.  A split writes one partial
-// (m, l, O) per row.  Bound: the vector work (48% of the SIMD cycles over the
-// whole chip) and the matrix work (27%), which hardly overlap on a SIMD (the
-// two waves of a SIMD in opposite order, or 64 tokens per softmax in place of
-// 32, changed nothing; row sums of the rounded weights by dot products were
-// slower); 12% of the compute units have no workgroup (the splits are whole).
+// (m, l, O) per row.  Bound: the vector work (53% of the SIMD cycles at 2
+// requests of 8192 tokens x 509 rows x 16 heads) and the matrix work (31%),
+// which hardly overlap on a SIMD (the two waves of a SIMD in opposite order, or
+// 64 tokens per softmax in place of 32, changed nothing; row sums of the rounded
+// weights by dot products were slower); where whole splits do not fill the
+// compute units, those without a workgroup (12% at 4518 and 6000 tokens).
 //
 // chunk_finish_kernel: 32 rows of one (request, head) per workgroup of 4
 // waves merge the splits, apply R_v^T, add the live tokens and write the
@@ -22,7 +23,7 @@
 //
 // Measured (2 requests of 4518 and 6000 tokens x 509 rows x 16 heads, causal,
 // residual loop / anchor loop): 289 / 250 us per call on 32-row tiles with the
-// live tokens on the vector units; here 112 / 102 us (stream 85 / 77, finish 27).
+// live tokens on the vector units; here 104 / 97 us (stream 85 / 77).
 #include "rq_multirow.h"
 
 namespace rq {
@@ -469,9 +470,13 @@ struct FinishTile {
     int request, tile;  // request -1: past the last tile
 };
 
-__device__ __forceinline__ FinishTile finish_tile(const PlanEntry& own, int key) {
+__device__ __forceinline__ FinishTile finish_tile(int64_t requests, const PlanEntry& own, int key) {
     const int lane = threadIdx.x & 63;
     const int tiles = (own.rows + 31) / 32;
+    if (requests == 1) {
+        const int tile = __builtin_amdgcn_readfirstlane(tiles) - 1 - key;
+        return FinishTile{tile >= 0 ? 0 : -1, tile};
+    }
     // Tiles of index `depth` and deeper.
     auto from = [&](int depth) __attribute__((always_inline)) {
         return (int)__builtin_amdgcn_readlane(wave_scan((uint32_t)max(tiles - depth, 0), lane), 63);
@@ -497,7 +502,7 @@ void chunk_finish_kernel(MultiRowParams p) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[Geometry<D, 32>::kLdsBytes];
     const int head = (int)(blockIdx.x % (unsigned)p.heads);
     const PlanEntry own = multirow_entry(p);
-    const FinishTile at = finish_tile(own, (int)(blockIdx.x / (unsigned)p.heads));
+    const FinishTile at = finish_tile(p.requests, own, (int)(blockIdx.x / (unsigned)p.heads));
     if (at.request < 0) return;  // uniform over the workgroup, before any barrier
     const int request = __builtin_amdgcn_readfirstlane(at.request);
     const int row0 = 32 * __builtin_amdgcn_readfirstlane(at.tile);

@@ -498,7 +498,10 @@ __device__ __forceinline__ void finish_merge(__amdgpu_buffer_rsrc_t entries, uin
 template <int D, int TR>
 __device__ __forceinline__ void live_tokens_fp32(const MultiRowParams& p, int head, int first, int row0, int n,
                                                  float shift, float& m, float& l, float (&acc)[16]) {
-    const int r = threadIdx.x >> 3, part = threadIdx.x & 7;
+    // (Opaque: addresses shared with the path of finite sums would stay in registers over it.)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int r = tid >> 3, part = tid & 7;
     const bool part_active = part < D / 16;
     const int row = r < TR && row0 + r < n ? row0 + r : -1;  // (sees no token)
     const int64_t channels = (int64_t)head * D + 16 * (part_active ? part : 0);
@@ -671,6 +674,7 @@ __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, i
         wave_sync();  // the next tile overwrites this one
     }
     __syncthreads();  // the merge buffer aliases every wave's tiles
+    static_assert(G::kMlOffset + kWaves * 32 * 2 * 4 <= kWaves * G::kWaveBytes - 128, "the shifts stay");
     float* merge_o = reinterpret_cast<float*>(lds);
     float* merge_ml = reinterpret_cast<float*>(lds + G::kMlOffset);
 #pragma unroll
@@ -707,7 +711,8 @@ __device__ __forceinline__ void live_tokens(const MultiRowParams& p, int head, i
 #pragma unroll
     for (int i = 0; i < 16; ++i) zero = fmaf(sums[i], 0.f, zero);
     if (__any(r < TR && row0 + r < n && !(zero == 0.f))) {
-        live_tokens_fp32<D, TR>(p, head, first, row0, n, shift, m, l, acc);
+        // (The merge buffer ends before the shifts.)
+        live_tokens_fp32<D, TR>(p, head, first, row0, n, shifts[r], m, l, acc);
         return;
     }
     m = total_max;

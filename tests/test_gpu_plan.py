@@ -160,7 +160,7 @@ def test_captured_rows_replay(device, rows):
 @pytest.mark.parametrize("lengths,rows,mode", [([3000, 700, 90], None, "anchor"), ([2600, 1, 600], None, "adjacent"),
                                                ([4000, 300, 600], [3, 20, 4], "anchor"),
                                                ([3000, 400, 700], [300, 50, 110], "anchor"),
-                                               ([500] * 70, [2] * 70, "anchor")],
+                                               ([90] * 70, [2] * 70, "anchor")],
                          ids=["decode", "adjacent", "rows", "chunk", "past-the-plan"])
 def test_workspace_of_the_required_size(oracle, device, lengths, rows, mode):
     """The smallest workspace that a call takes, at any address: right results,
