@@ -251,6 +251,28 @@ void plan_multirow(rq::MultiRowParams& m, int splits, size_t bytes) {
     m.plan_target = (int)target;
     m.entries = fit;
     m.items = (int)std::max(row_tiles * forced + target, row_tiles * splits);
+    // Near-equal requests stay whole up to the length where some count of splits
+    // begins to pay.  k workgroups on the busiest compute unit take, in 16ths of
+    // one of two beside each other, 22 (k = 1), 34 (2) or 16 k and 2 more, an odd
+    // one out 11; each spends about 300 tokens' time (chains 150) in its prologue
+    // and finish, a merge 350 (170).  With two splits, 576 workgroups for 512
+    // places, 18 requests of 270 tokens x 18 rows x 16 heads took 47 us per
+    // residual call and 75 us in adjacent loop 3, whole 29 and 52 us; of 1000
+    // tokens 56 and 109 us, whole 42 and 104 us; of 4000 tokens two splits stay
+    // (residual 105 and 102 us, loop 3 310 and 338 us).
+    const bool chain = m.chain_length > 0;
+    const int64_t overhead = chain ? 5 : 9, merge = chain ? 5 : 11;  // tiles
+    const int64_t groups = m.requests * m.heads * std::max<int64_t>(1, (m.rows / m.requests + 31) / 32);
+    auto weight = [&](int64_t s) {
+        const int64_t k = (groups * s + compute_units() - 1) / compute_units();
+        return k == 1 ? 22 : k == 2 ? 34 : 16 * k + (k % 2 != 0 ? 11 : 2);
+    };
+    int64_t whole = INT32_MAX;
+    for (int s = 2; s <= std::min(splits, rq::kMultiRowMaxSplits); ++s) {
+        const int64_t gain = s * weight(1) - weight(s);  // per s tiles
+        if (gain > 0) whole = std::min(whole, s * (overhead * (weight(s) - weight(1)) + 16 * merge) / gain);
+    }
+    m.plan_whole = (int)std::max<int64_t>(whole, 0);
 }
 
 // A call's tag for its arrival words (rq_plan.h), never 0.  The start is hashed

@@ -256,7 +256,7 @@ struct MultiRowParams {
     // requests (items 0) every (request, head, row tile) takes `splits`.
     int items;
     int splits;
-    int plan_target, plan_min, plan_max, plan_max_splits;  // PlanSizes, in units of plan_unit tokens
+    int plan_target, plan_min, plan_max, plan_max_splits, plan_whole;  // PlanSizes, in units of plan_unit tokens
     int plan_unit;        // 32, or 128 (chunk kernels)
     int tile_rows;        // rows of a stream tile: 16, 32 or 256 (chunk kernels)
     int compute_units;    // of the launching device

@@ -860,7 +860,7 @@ __device__ __forceinline__ RequestRows request_rows(const MultiRowParams& p, int
 }
 
 __host__ __device__ __forceinline__ PlanSizes multirow_sizes(const MultiRowParams& p) {
-    return PlanSizes{p.plan_target, p.splits, p.plan_min, p.plan_max, p.plan_max_splits, 0, 1, p.plan_unit == kTile ? 13 : 9};
+    return PlanSizes{p.plan_target, p.splits, p.plan_min, p.plan_max, p.plan_max_splits, 0, 1, p.plan_unit == kTile ? 13 : 9, p.plan_whole};
 }
 
 // The share of request `lane` of the call's plan.

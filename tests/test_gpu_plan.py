@@ -74,6 +74,10 @@ MULTIROW_CASES = [
     ([1900, 400, 150], [40, 3, 70], 3, 96, 32, "anchor"),
     ([1300, 70], [4, 2], 16, 128, 16, "adjacent"),
     ([40] * 64 + [900], [2] * 65, 1, 128, 16, "anchor"),  # more requests than the plan covers
+    # near-equal requests: whole (10 tiles), split (22 tiles; chains from 8 tiles)
+    ([310, 300, 318], [20, 20, 20], 2, 128, 16, "anchor"),
+    ([700, 690], [20, 20], 2, 96, 32, "anchor"),
+    ([262, 262], [3, 3], 2, 128, 16, "adjacent"),
 ]
 
 
