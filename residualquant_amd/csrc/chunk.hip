@@ -89,7 +89,7 @@ __device__ __forceinline__ void chunk_stream(const MultiRowParams& p, Decoder& d
     using L = Tile<D, kChunkUnit>;
     constexpr int KS = L::KS, Quarters = D / 32, Parts = D / 16;
     const int head = (int)(blockIdx.x % (unsigned)p.heads);
-    const PlanItem item = multirow_plan(p, (int)(blockIdx.x / (unsigned)p.heads), 0, 0, 0);
+    const PlanItem item = multirow_plan<false>(p, (int)(blockIdx.x / (unsigned)p.heads), 0, 0, 0);
     const int request = __builtin_amdgcn_readfirstlane(item.request);
     if (request < 0) return;
     const int first = __builtin_amdgcn_readfirstlane(item.first), n = __builtin_amdgcn_readfirstlane(item.rows);
@@ -509,7 +509,7 @@ void chunk_finish_kernel(MultiRowParams p) {
     const int first = __builtin_amdgcn_readlane(own.first, request), n = __builtin_amdgcn_readlane(own.rows, request);
     FinishInputs<D> in;
     finish_load<D, 32>(p, head, first, row0, n, in);
-    const PlanRequest plan = plan_request(request, multirow_sizes(p), own);
+    const PlanRequest plan = plan_request(request, multirow_sizes<false>(p), own);
     const int tid = threadIdx.x, r = tid >> 3, part = tid & 7;
     const bool valid = row0 + r < n;
     const float* tile_entries =

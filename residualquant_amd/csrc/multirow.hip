@@ -78,7 +78,7 @@ __device__ __forceinline__ void multirow_stream(const MultiRowParams& p, Decoder
     constexpr int KS = G::KS;
     constexpr int QRS = G::QRS;
     const int head = stream_head(p);
-    const PlanItem item = multirow_plan(p, (int)(blockIdx.x / (unsigned)p.heads), blockIdx.x,
+    const PlanItem item = multirow_plan<true>(p, (int)(blockIdx.x / (unsigned)p.heads), blockIdx.x,
                                                (int)blockIdx.z / p.splits, (int)blockIdx.z % p.splits);
     const int request = __builtin_amdgcn_readfirstlane(item.request);
     const int first = __builtin_amdgcn_readfirstlane(item.first), n = __builtin_amdgcn_readfirstlane(item.rows);

@@ -256,7 +256,7 @@ struct MultiRowParams {
     // requests (items 0) every (request, head, row tile) takes `splits`.
     int items;
     int splits;
-    int plan_target, plan_min, plan_max, plan_max_splits, plan_whole;  // PlanSizes, in units of plan_unit tokens
+    int plan_target, plan_min, plan_max, plan_max_splits;  // PlanSizes, in units of plan_unit tokens
     int plan_unit;        // 32, or 128 (chunk kernels)
     int tile_rows;        // rows of a stream tile: 16, 32 or 256 (chunk kernels)
     int compute_units;    // of the launching device
@@ -264,6 +264,7 @@ struct MultiRowParams {
     int64_t entries;      // partials per head
     float* partials;      // workspace [heads, entries, kMultiRowEntry]; a request's entries: [row, split]
     uint64_t call_tag;    // of this call (48 bits, rq_plan.h)
+    int plan_whole;       // PlanSizes (multirow.hip)
 };
 template <int D>
 hipError_t launch_multirow(const MultiRowParams& p, hipStream_t stream);

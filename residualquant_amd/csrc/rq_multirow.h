@@ -859,8 +859,12 @@ __device__ __forceinline__ RequestRows request_rows(const MultiRowParams& p, int
     return r;
 }
 
+// (Whole false: the chunk kernels, which take no whole_length; a branch that they
+// never take cost their four-record chain 2%.)
+template <bool Whole>
 __host__ __device__ __forceinline__ PlanSizes multirow_sizes(const MultiRowParams& p) {
-    return PlanSizes{p.plan_target, p.splits, p.plan_min, p.plan_max, p.plan_max_splits, 0, 1, p.plan_unit == kTile ? 13 : 9, p.plan_whole};
+    return PlanSizes{p.plan_target, p.splits, p.plan_min, p.plan_max, p.plan_max_splits, 0, 1, p.plan_unit == kTile ? 13 : 9,
+                     Whole ? p.plan_whole : 0};
 }
 
 // The share of request `lane` of the call's plan.
@@ -875,8 +879,9 @@ __device__ __forceinline__ PlanEntry multirow_entry(const MultiRowParams& p) {
 // Item `key` of the call's plan, or, with more requests than the plan covers,
 // split `split` of the call's `splits` of row tile `tile` of `request`.
 // PlanItem: length in units of plan_unit tokens, tokens the history.
+template <bool Whole>
 __device__ __forceinline__ PlanItem multirow_plan(const MultiRowParams& p, int key, int request, int tile, int split) {
-    if (p.items > 0) return plan_find((int)p.requests, key, multirow_sizes(p), multirow_entry(p));
+    if (p.items > 0) return plan_find((int)p.requests, key, multirow_sizes<Whole>(p), multirow_entry(p));
     const RequestRows q = request_rows(p, request);
     // About requests x the average request's row tiles x splits of the items have work.
     const int64_t tiles = max(p.rows / (p.requests * p.tile_rows), (int64_t)1);

@@ -104,7 +104,7 @@ __host__ __device__ __forceinline__ PlanShare plan_share_of(const PlanSizes& siz
     s.even = 8ull * longest * counts <= (uint64_t)(full ? sizes.full_eighths : 9) * total;
     s.even_splits = (uint32_t)sizes.even_splits;
     if (s.even_splits > 1 && longest < s.even_splits * min_chunk) s.even_splits = max(longest / min_chunk, 1u);
-    if (longest <= (uint32_t)min(sizes.whole_length, sizes.max_chunk)) s.even_splits = 1;
+    if (sizes.whole_length > 0 && longest <= (uint32_t)min(sizes.whole_length, sizes.max_chunk)) s.even_splits = 1;
     s.chunk = (uint32_t)sizes.max_chunk;
     if (s.even && s.even_splits == 1 && 8ull * longest * counts > 9ull * total && longest <= s.chunk) {
         // Whole, but not alike: one split each, the longest first.

@@ -105,7 +105,7 @@ void several_rows() {
         const int64_t tokens = std::min<int64_t>(c.history[b], c.max_pages * c.page_tokens);
         length.push_back((tokens + m.plan_unit - 1) / m.plan_unit);
     }
-    const Plan plan = take(rq::multirow_sizes(m), tiles, length, c.count);
+    const Plan plan = take(chunk ? rq::multirow_sizes<false>(m) : rq::multirow_sizes<true>(m), tiles, length, c.count);
     check("rows_entries", plan.entries <= m.entries);
     check("rows_entries_in_workspace", sizeof(float) * rq::kMultiRowEntry * c.heads * (size_t)m.entries <= bytes);
     check("rows_items", plan.items <= m.items);
